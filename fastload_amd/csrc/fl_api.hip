@@ -460,6 +460,8 @@ int fl_matrix_create(fl_matrix **out, int m, int n, int nnz, const int *d_colptr
         }
         A->max_col_nnz = device_max_i32(counts.p, n, s);
         colsort_device(n, counts.p, A->perm.p, A->sortnnz.p, A->max_col_nnz, s);
+        A->iperm.alloc(std::max(n, 1));
+        invert_perm(A->perm.p, n, A->iperm.p, s);
         ElemSource src;
         src.colptr = d_colptr;
         src.perm = A->perm.p;

@@ -39,6 +39,7 @@ struct fl_matrix {
 
     // column sort (ColSort): perm[i] = original column of sorted position i; sortnnz[i] its length
     fl::DevBuf<int> perm, sortnnz;
+    fl::DevBuf<int> iperm;  // sorted position of every original column (inverse of perm)
     // per-level table (prepare/countTileNum/auxiliaryTrans): col, base depth, tall,
     // tile offset (L+1), nnz offset (L+1)
     fl::DevBuf<int> lvl_col, lvl_base, lvl_tall, lvl_tileoff, lvl_nnzoff;
@@ -163,6 +164,9 @@ struct ElemSource {
 };
 void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src, hipStream_t s, float *t_tran_ms,
                       float *t_clas_ms);
+
+// iperm[perm[i]] = i
+void invert_perm(const int *perm, int n, int *iperm, hipStream_t s);
 
 // y = A x (assign) or y += A x with one schedule. work: 2*m floats for the FAST kernel's split
 // BF16 mode. pb_bins: product array for the PB schedule (at least pb_ring entries of the value

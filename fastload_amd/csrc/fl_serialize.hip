@@ -494,11 +494,13 @@ int fl_matrix_load(fl_matrix **out, const char *path, void *stream) {
     A->nnz = nnz;
     A->W = h.W;
     A->perm.alloc(std::max(n, 1));
+    A->iperm.alloc(std::max(n, 1));
     A->sortnnz.alloc(std::max(n, 1));
     A->sortrowidx.alloc(std::max(nnz, 1));
     A->val64.alloc(std::max(nnz, 1));
     if (n) {
         FL_HIP(hipMemcpyAsync(A->perm.p, perm, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, s));
+        invert_perm(A->perm.p, n, A->iperm.p, s);
         FL_HIP(hipMemcpyAsync(A->sortnnz.p, sortnnz, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, s));
     }
     if (nnz) {
