@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "fl_matrix.h"
@@ -161,11 +162,7 @@ template <> struct RowVec<float, 4> { using type = float4; };
 template <> struct RowVec<double, 1> { using type = double; };
 template <> struct RowVec<double, 2> { using type = double2; };
 
-// K / VEC lanes own one row (64 * VEC / K rows per wave); lane j accumulates columns
-// [j*VEC, j*VEC + VEC) of the row's Y block, gathering them from X as one VEC-wide load per
-// entry. Every Y element sums its row's entries in entry order whatever VEC is. Persistent:
-// waves stride over row groups. ACC = accumulator type.
-// The waves of XCD x (workgroups with blockIdx % 8 == x; gridDim a multiple of 8) stride over the
+// k = 1: the waves of XCD x (workgroups with blockIdx % 8 == x; gridDim a multiple of 8) stride over the
 // row groups of that XCD's range [sp.r[x], sp.r[x+1]), so the rows in flight on one XCD at any
 // time are a contiguous window, and on matrices whose rows have local columns (bands, stencils,
 // block-diagonal batches) the X rows they gather stay in that XCD's L2.
@@ -184,50 +181,130 @@ __device__ __forceinline__ XcdRows xcd_rows(const RowSplit &sp) {
     return w;
 }
 
-template <typename T, typename ACC, int K, int VEC, int UNR>
-__global__ __launch_bounds__(kBlock) void k_spmm_row(RowSplit sp, const int *__restrict__ row_ptr,
+// The value of lane U0 of each group of L consecutive lanes, in all lanes of the group (which must
+// all be active). DPP moves for up to 16 lanes: quad permutes, and row broadcasts (for 8 lanes
+// one per half row, selected by the bank mask).
+template <int L, int U0>
+__device__ __forceinline__ uint32_t bcast_u32(uint32_t v) {
+    if constexpr (L == 1) return v;
+    else if constexpr (L == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, U0 | (U0 << 2) | ((2 + U0) << 4) | ((2 + U0) << 6), 0xf, 0xf, true);
+    else if constexpr (L == 4) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, U0 * 0x55, 0xf, 0xf, true);
+    else if constexpr (L == 16) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + U0, 0xf, 0xf, true);
+    else if constexpr (L == 8) {
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + U0, 0xf, 0x3, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(lo, (int)v, 0x150 + 8 + U0, 0xf, 0xc, false);
+    } else return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(((__lane_id() & ~(uint32_t)(L - 1)) + U0) * 4), (int)v);
+}
+template <int L, int U0>
+__device__ __forceinline__ float bcast(float v) { return __uint_as_float(bcast_u32<L, U0>(__float_as_uint(v))); }
+template <int L, int U0>
+__device__ __forceinline__ double bcast(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const uint32_t lo = bcast_u32<L, U0>((uint32_t)b), hi = bcast_u32<L, U0>((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// L = K / VEC lanes own one row (64 / L rows per wave, one group of rows per wave); lane j
+// accumulates columns [j*VEC, j*VEC + VEC) of the row's Y block, gathering them from X as one
+// VEC-wide load per entry. Every Y element sums its row's entries in entry order whatever VEC is.
+//
+// Bound by the vector memory path: every distinct line an instruction touches takes a turn in
+// the L1, and a gather touches one per row. So the entries are not loaded once per row and entry
+// (which cost as many turns as the X rows themselves): each lane of a row loads one of the next
+// L * Q entries, and the lanes hand them to each other with DPP moves while the next step's are in
+// flight. X rows come in groups of U, unconditionally: past the row's end the lanes read X row 0
+// (one line for all of them) and drop it, since a branch around the loads would drain them.
+// Consecutive groups run on one XCD in chunks of kRowChunk rows, dealt round-robin: rows with local
+// columns (bands, grids, block-diagonal batches) share X lines in that XCD's L2, and no XCD gets
+// all of the large blocks of a batch. One group per wave: waves that loop over several groups
+// end unevenly (grid of 64^3, k = 16 in FP64: 58 us with one group, 78 with eight).
+// Y rows of at least a line are stored with the streaming hint: they are written whole and leave the L2
+// to X (k = 32: 287 -> 274 us).
+// Measured, before -> after (one entry load per row, four entries ahead, contiguous row ranges):
+// 128 stacked Zipf(2) matrices (5.2 M rows, 37 M entries) k = 8: 398 -> 291 us; 64 of them, k = 32:
+// 395 -> 273 us; 64^3 27-point grid, k = 16 in FP64: 79 -> 58 us. With every gather
+// sent to 64 lines of X the k = 8 product takes 238 us, without gathers 121 us. Measured and not
+// kept: the columns that recur in a block of rows staged in LDS (k = 8: 290 us, k = 32: 332 us and
+// more, grid: 104 us and more: the entry loop grows by the choice of source and LDS costs waves);
+// rows ordered by length in windows of 256 (k = 8: 409 us: entries of a wave's rows no longer share
+// lines).
+constexpr int kRowChunk = 1024;
+template <typename T, typename ACC, int K, int VEC>
+__global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int *__restrict__ row_ptr,
                                                      const int *__restrict__ row_col, const T *__restrict__ row_val,
                                                      const T *__restrict__ X, T *__restrict__ Y, int accumulate) {
     using V = typename RowVec<T, VEC>::type;
-    constexpr int L = K / VEC;   // lanes per row
-    constexpr int RPW = 64 / L;  // rows per wave
-    const int lane = threadIdx.x & 63;
-    const int sub = lane / L, j = lane % L;
+    constexpr int L = K / VEC, RPW = 64 / L;  // lanes per row, rows per wave
+    constexpr int Q = L < 16 ? 16 / L : 1;    // entries per lane of a step
+    constexpr int U = L * Q < 4 ? L * Q : 4;  // X rows in flight together
+    constexpr bool kStreamY = K * sizeof(T) >= 128;
+    const int idx = blockIdx.x >> 3;
+    const long long wg = (long long)(idx / chunk * 8 + (int)(blockIdx.x & 7)) * chunk + idx % chunk;
+    const int lane = threadIdx.x & 63, sub = lane / L, j = lane % L;
+    const long long r = (wg * (kBlock / 64) + (threadIdx.x >> 6)) * RPW + sub;
+    if (r >= m) return;
     const V *__restrict__ Xv = reinterpret_cast<const V *>(X);
-    const XcdRows xw = xcd_rows(sp);
-    const long long groups = ((long long)(xw.r1 - xw.r0) + RPW - 1) / RPW;
-    for (long long gq = xw.wave; gq < groups; gq += xw.nwaves) {
-        const long long r = xw.r0 + gq * RPW + sub;
-        if (r >= xw.r1) continue;
-        const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
-        ACC acc[VEC];
+    const int e0 = row_ptr[r];
+    const int *__restrict__ pc = row_col + e0 + j;
+    const T *__restrict__ pv = row_val + e0 + j;
+    ACC acc[VEC];
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) acc[q] = 0;
-        auto add = [&](T v, const V &xv) {
-            const T *xs = reinterpret_cast<const T *>(&xv);
+    for (int q = 0; q < VEC; ++q) acc[q] = 0;
+    int c[Q], nc[Q];
+    T v[Q], nv[Q];
+    auto fetch = [&](int left, int *cc, T *vv) {  // the next entries of the row, `left` of them to come
 #pragma unroll
-            for (int q = 0; q < VEC; ++q) acc[q] += (ACC)v * (ACC)xs[q];
-        };
-        int e = e0;
-        for (; e + UNR <= e1; e += UNR) {
-            int c[UNR];
-            T v[UNR];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) {
-                c[u] = row_col[e + u];
-                v[u] = row_val[e + u];
-            }
-            V xv[UNR];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) xv[u] = Xv[(long long)c[u] * L + j];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) add(v[u], xv[u]);
+        for (int q = 0; q < Q; ++q) {
+            cc[q] = q * L + j < left ? pc[q * L] : 0;
+            vv[q] = q * L + j < left ? pv[q * L] : T(0);
         }
-        for (; e < e1; ++e) add(row_val[e], Xv[(long long)row_col[e] * L + j]);
-        T *out = Y + r * K + (long long)j * VEC;
+        pc += L * Q;
+        pv += L * Q;
+    };
+    int left = row_ptr[r + 1] - e0;
+    fetch(left, c, v);
+    for (; left > 0; left -= L * Q) {
+        fetch(left - L * Q, nc, nv);
+        static_for<0, L * Q / U>([&](auto h) {
+            constexpr int H = decltype(h)::value * U;
+            if (H < left) {
+                V x[U];
+                static_for<0, U>([&](auto u) {
+                    constexpr int k = H + decltype(u)::value;
+                    x[u] = Xv[(long long)bcast_u32<L, k % L>((uint32_t)c[k / L]) * L + j];
+                });
+                static_for<0, U>([&](auto u) {
+                    constexpr int k = H + decltype(u)::value;
+                    const T a = bcast<L, k % L>(v[k / L]);
+                    if (k < left) {
+                        const T *xs = reinterpret_cast<const T *>(&x[u]);
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) out[q] = accumulate ? (T)((ACC)out[q] + acc[q]) : (T)acc[q];
+                        for (int q = 0; q < VEC; ++q) acc[q] += (ACC)a * (ACC)xs[q];
+                    }
+                });
+            }
+        });
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            c[q] = nc[q];
+            v[q] = nv[q];
+        }
     }
+    V *out = reinterpret_cast<V *>(Y) + r * L + j;
+    V o;
+    if (accumulate) o = *out;
+    T *os = reinterpret_cast<T *>(&o);
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) os[q] = accumulate ? (T)((ACC)os[q] + acc[q]) : (T)acc[q];
+    if constexpr (kStreamY) st_stream(out, o);
+    else *out = o;
 }
 
 // k = 1: LPR = 4 lanes per row; lane j sums entries e0 + j, e0 + j + 4, ... and the four partial
@@ -293,16 +370,18 @@ static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, in
 
 template <typename T, typename ACC, int K, int VEC>
 static void launch_row_v(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    constexpr int RPW = 64 * VEC / K;
-    k_spmm_row<T, ACC, K, VEC, 4><<<row_grid(A->m, RPW), kBlock, 0, s>>>(A->row_split, A->row_ptr.p, A->row_col.p, val,
-                                                                         X, Y, accumulate);
+    constexpr int rows = 64 * VEC / K * (kBlock / 64);  // of a workgroup
+    const int wgs = div_up(A->m, rows);
+    // chunks of kRowChunk rows, shorter where that would leave an XCD fewer than eight of them
+    const int chunk = std::max(1, std::min(kRowChunk / rows, wgs / 64));
+    k_spmm_row<T, ACC, K, VEC><<<8 * chunk * div_up(wgs, 8 * chunk), kBlock, 0, s>>>(
+        A->m, chunk, A->row_ptr.p, A->row_col.p, val, X, Y, accumulate);
     FL_LAUNCH_CHECK();
 }
 
 // Widest vector that keeps at least 4 lanes per row (k >= 4), is at most 16 bytes and that X
-// and Y are aligned for. On the 512-matrix batch: k = 32 took 3.14 ms with 16-byte lanes
-// against 5.28 ms with 4-byte lanes and 3.84 ms with 32-byte lanes; k = 8 took 1.72 ms with
-// 8-byte lanes (4 per row) against 1.78 ms with 16-byte lanes (2 per row).
+// and Y are aligned for. With 1 or 2 lanes per row instead (16-byte loads from k = 4 on) 40 Zipf(2)
+// matrices at k = 4 took 86 us against 76, 128 of them at k = 8 294 against 291.
 template <typename T, typename ACC, int K>
 static void launch_row(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
     constexpr int VT = 16 / (int)sizeof(T);

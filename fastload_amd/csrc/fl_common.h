@@ -78,6 +78,16 @@ __device__ __forceinline__ T ld_stream(const T *p) {
     }
     return out;
 }
+
+// A store with the same hint, for data the kernel does not read again. T is 4 to 16 bytes.
+template <typename T>
+__device__ __forceinline__ void st_stream(T *p, const T &v) {
+    typedef unsigned int W __attribute__((ext_vector_type(sizeof(T) / 4)));
+    W w;
+    __builtin_memcpy(&w, &v, sizeof(T));
+    __builtin_nontemporal_store(w, reinterpret_cast<W *>(p));
+}
+
 inline unsigned grid_for(long long threads, int block = kBlock) { return (unsigned)((threads + block - 1) / block); }
 
 // RAII device buffer (hipMalloc'd, freed on scope exit).
