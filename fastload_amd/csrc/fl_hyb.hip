@@ -8,9 +8,9 @@
 // moved twice through the Infinity Cache), run on a sub-matrix of their own.
 //
 // Layout of the heavy part (all built on the GPU by hyb_prepare):
-//   - rows are ordered by heavy entry count, longest first, inside windows of kHybWin rows
-//     (hyb_iperm[r] = position of row r inside its window), so the 64 rows of a slice have
-//     nearly the same count;
+//   - rows are ordered by heavy entry count, longest first, inside windows of hyb_win rows, the
+//     sub-matrix's PB bands (hyb_iperm[r] = position of row r inside its window), so the 64 rows of
+//     a slice have nearly the same count;
 //   - slice s = sorted positions [64 s, 64 s + 64) is an ELL block of hyb_np[s] pair rows: slot
 //     (q, lane), at hyb_sb[s] + 64 q + lane, holds entries 2q and 2q + 1 of the lane's row as a
 //     value pair and one word of two 16-bit columns; rows shorter than the slice's longest are
@@ -18,10 +18,9 @@
 //     power-law workload the padding adds 5 % to the heavy entries. A wave reads one slot per
 //     lane per pair row: 8 (16 in FP64) + 4 contiguous bytes, with no per-entry index math;
 //   - the heavy kernel writes y by sorted position (hyb_ys), and the sub-matrix's first PB phase 2
-//     adds it to y: with bands of kHybWin rows (one band = one window) it reads hyb_ys in order
-//     and adds hyb_ys[p] to row hyb_perm[p] of its LDS sums (a gather through hyb_iperm would
-//     move a 128-byte line per 4-byte value: 14 of phase 2's 42 us on the power-law workload);
-//     with other band sizes it adds hyb_ys[(r & ~(kHybWin - 1)) + hyb_iperm[r]] to row r.
+//     adds it to y: a band is a window, so it reads hyb_ys in order and adds hyb_ys[p] to row
+//     hyb_perm[p] of its LDS sums (a gather through hyb_iperm would move a 128-byte line per
+//     4-byte value: 14 of phase 2's 42 us on the power-law workload).
 // The column sort is ascending, so the heavy columns are the last H sorted columns: heavy x is
 // sortx + (n - H), and the sub-matrix's sorted columns are the first n - H sorted columns in the
 // same order (its own column sort of already ascending counts is the identity, so it is not run),
@@ -104,17 +103,17 @@ __global__ void k_hyb_lenkey(const int *__restrict__ hptr, int m, uint32_t *__re
     }
 }
 
-__global__ void k_hyb_winkey(const int *__restrict__ rows, int m, uint32_t *__restrict__ key) {
-    HSTRIDE(p, m) key[p] = (uint32_t)(rows[p] >> kHybWinLog);
+__global__ void k_hyb_winkey(const int *__restrict__ rows, int m, int win, uint32_t *__restrict__ key) {
+    HSTRIDE(p, m) key[p] = (uint32_t)(rows[p] / win);
 }
 
-__global__ void k_hyb_pos(const int *__restrict__ rows, int m, uint16_t *__restrict__ iperm,
+__global__ void k_hyb_pos(const int *__restrict__ rows, int m, int win, uint16_t *__restrict__ iperm,
                           uint16_t *__restrict__ perm, int *__restrict__ flag) {
     HSTRIDE(p, m) {
-        const int r = rows[p];
-        iperm[r] = (uint16_t)(p & (kHybWin - 1));
-        perm[p] = (uint16_t)(r & (kHybWin - 1));
-        if ((p >> kHybWinLog) != (r >> kHybWinLog)) *flag = 1;  // a row left its window
+        const int r = rows[p], w0 = r / win * win;
+        iperm[r] = (uint16_t)(p - w0);
+        perm[p] = (uint16_t)(r - w0);
+        if (p < w0 || p - w0 >= win) *flag = 1;  // a row left its window
     }
 }
 
@@ -243,7 +242,8 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         transform_device(L.get(), L->sortnnz.p, src, s, nullptr, nullptr);
         FL_HIP(hipStreamSynchronize(s));
     }
-    pb_prepare(L.get(), bt, R, s);
+    pb_prepare(L.get(), bt, R & ~63, s);  // bands of whole slices: they are the sorting windows
+    const int win = A->hyb_win = L->pb_R;
 
     // heavy part
     const int nslice = (m + 63) / 64;
@@ -272,10 +272,10 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         k_hyb_lenkey<<<hg(m), kBlock, 0, s>>>(hptr.p, m, wkey.p, rows.p);
         FL_LAUNCH_CHECK();
         radix_sort_pairs(wkey.p, rows.p, m, 16, s);
-        k_hyb_winkey<<<hg(m), kBlock, 0, s>>>(rows.p, m, wkey.p);
+        k_hyb_winkey<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, wkey.p);
         FL_LAUNCH_CHECK();
-        radix_sort_pairs(wkey.p, rows.p, m, bits_for((uint32_t)((m - 1) >> kHybWinLog)), s);
-        k_hyb_pos<<<hg(m), kBlock, 0, s>>>(rows.p, m, A->hyb_iperm.p, A->hyb_perm.p, flag.p);
+        radix_sort_pairs(wkey.p, rows.p, m, bits_for((uint32_t)((m - 1) / win)), s);
+        k_hyb_pos<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, A->hyb_iperm.p, A->hyb_perm.p, flag.p);
         TmpBuf<int> pairs(std::max(nslice, 1), s), pscan((size_t)nslice + 1, s);
         k_hyb_pairs<<<hg(nslice), kBlock, 0, s>>>(rows.p, hptr.p, m, nslice, A->hyb_np.p, pairs.p);
         FL_LAUNCH_CHECK();
@@ -454,9 +454,9 @@ __global__ __launch_bounds__(1024) void k_hyb(int m, int H, int nslice, const lo
 
 // y = ys in row order (assign) or y += it: the HYB schedule when no light entries exist
 template <typename Y, bool ASSIGN>
-__global__ void k_hyb_unperm(int m, const uint16_t *__restrict__ iperm, const Y *__restrict__ ys, Y *__restrict__ y) {
+__global__ void k_hyb_unperm(int m, int win, const uint16_t *__restrict__ iperm, const Y *__restrict__ ys, Y *__restrict__ y) {
     HSTRIDE(r, m) {
-        const Y v = ys[(r & ~(long long)(kHybWin - 1)) + iperm[r]];
+        const Y v = ys[(int)r / win * win + iperm[r]];
         if constexpr (ASSIGN) y[r] = v;
         else y[r] += v;
     }
@@ -549,18 +549,17 @@ int spmv_hyb(fl_matrix *A, int kind, const void *x, void *y, bool assign, hipStr
         PbFold fold;
         if (heavy) {
             fold.ys = ys;
-            fold.iperm = A->hyb_iperm.p;
             fold.perm = A->hyb_perm.p;
         }
         return spmv_batched(L, FL_KERNEL_PB, kind, x, y, assign, s, bins, &fold, stream ? 1 : 0);
     }
     if (heavy) {
         if (dbl) {
-            if (assign) k_hyb_unperm<double, true><<<hg(m), kBlock, 0, s>>>(m, A->hyb_iperm.p, (const double *)ys, (double *)y);
-            else k_hyb_unperm<double, false><<<hg(m), kBlock, 0, s>>>(m, A->hyb_iperm.p, (const double *)ys, (double *)y);
+            if (assign) k_hyb_unperm<double, true><<<hg(m), kBlock, 0, s>>>(m, A->hyb_win, A->hyb_iperm.p, (const double *)ys, (double *)y);
+            else k_hyb_unperm<double, false><<<hg(m), kBlock, 0, s>>>(m, A->hyb_win, A->hyb_iperm.p, (const double *)ys, (double *)y);
         } else {
-            if (assign) k_hyb_unperm<float, true><<<hg(m), kBlock, 0, s>>>(m, A->hyb_iperm.p, (const float *)ys, (float *)y);
-            else k_hyb_unperm<float, false><<<hg(m), kBlock, 0, s>>>(m, A->hyb_iperm.p, (const float *)ys, (float *)y);
+            if (assign) k_hyb_unperm<float, true><<<hg(m), kBlock, 0, s>>>(m, A->hyb_win, A->hyb_iperm.p, (const float *)ys, (float *)y);
+            else k_hyb_unperm<float, false><<<hg(m), kBlock, 0, s>>>(m, A->hyb_win, A->hyb_iperm.p, (const float *)ys, (float *)y);
         }
         FL_LAUNCH_CHECK();
     } else if (assign) {

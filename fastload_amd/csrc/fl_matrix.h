@@ -109,12 +109,13 @@ struct fl_matrix {
     // multiplied with x held in LDS, row by row; the other columns form a sub-matrix (hyb_light,
     // its sorted column i = sorted column i here) with its own PB schedule, whose first phase 2
     // adds the heavy part's y. The rows are ordered by heavy entry count, longest first, inside
-    // windows of kHybWin rows (hyb_iperm); slice s = sorted positions [64 s, 64 s + 64) is stored
+    // windows of hyb_win rows (hyb_iperm); slice s = sorted positions [64 s, 64 s + 64) is stored
     // as hyb_np[s] pair-slots of 64 lanes: slot (q, lane) holds the lane's row's entries 2q and
     // 2q + 1 (value pair + two 16-bit columns in one word), the rows shorter than the slice's
     // longest padded with value 0 and column H (a zero in LDS).
     bool hyb_ready = false;
     int hyb_H = 0, hyb_bt = 0, hyb_R = 0, hyb_nslice = 0, hyb_grid = 0;
+    int hyb_win = 0;                  // rows of a sorting window = of a PB band (a multiple of 64)
     long long hyb_nnz = 0;            // heavy entries
     long long hyb_slots = 0;          // pair-slots of all slices (64 per pair row)
     std::unique_ptr<fl_matrix> hyb_light;
@@ -175,13 +176,11 @@ int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work,
          void *pb_bins = nullptr);
 
 // The HYB schedule's heavy part, which the first chunk's phase 2 of its PB sub-matrix adds to y.
-// ys holds the heavy sum of row r at (r & ~(kHybWin - 1)) + iperm[r] (its position inside its
-// window); perm is the inverse (position -> row inside the window). When the PB bands are the
-// windows (band rows == kHybWin), phase 2 reads ys in order and adds ys[p] to row perm[p] of the
-// band in LDS; otherwise it gathers ys through iperm as it writes each row.
+// ys holds the heavy sums by sorted position; the sorting windows are the PB bands, and perm[p] is the
+// row, inside its band, at position p. Phase 2 reads ys in order and adds ys[p] to row perm[p] of
+// the band in LDS.
 struct PbFold {
     const void *ys = nullptr;
-    const uint16_t *iperm = nullptr;
     const uint16_t *perm = nullptr;
 };
 
@@ -211,7 +210,6 @@ inline bool stream_reads(long long bytes) {
 // HYB schedule (fl_hyb.hip). Heavy x is staged in LDS: at most kHybMaxH32 FP32 or kHybMaxH64
 // FP64 columns.
 constexpr int kHybMaxH32 = 38912, kHybMaxH64 = 19456;
-constexpr int kHybWinLog = 14, kHybWin = 1 << kHybWinLog;  // rows of a sorting window
 void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s);
 void hyb_values(fl_matrix *A, int kind, hipStream_t s);
 int hyb_check(const fl_matrix *A, int kind);

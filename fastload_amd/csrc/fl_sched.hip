@@ -403,8 +403,20 @@ static std::vector<int> pb_chunk_batches(const fl_matrix *A, int C, hipStream_t 
     return cb;
 }
 
+// Rows of a band: at most R, and few enough that phase 2, one workgroup per band, has one band for
+// each of the 256 compute units; but a batch (bt * 64 entries) then writes bt * 64 / bands products
+// at a time, so there are no more bands than leave it 32. Measured (a product, 16K-row bands
+// -> these): 1.5 M rows, Poisson(12) columns, FP32: 93 -> 77 us (92 bands -> 245; 82 us at 4,096 rows,
+// 88 at 2,048); 400 K rows: 39.5 -> 19.0 (25 -> 196 bands); 3 M rows in FP64: 174 -> 172. From 4.2 M
+// rows on the bands are as tall as asked for (4.2 M power-law rows: 154 us at 16K, 171 at 8K).
+static int pb_band_rows(int m, int bt, int R) {
+    const int per = div_up(m, std::min(256, 2 * bt));
+    return std::min(R, std::max(1024, (per + 1023) / 1024 * 1024));
+}
+
 void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     ensure_batches(A, bt, 0, s);
+    R = pb_band_rows(A->m, bt, R);
     if (A->pb_ready && A->pb_R == R) return;
     A->pb_ready = false;
     A->pb_pack.release();
@@ -998,11 +1010,9 @@ struct PbVec<double> {
 // ASSIGN: y = A x (every row of the band is written, so y needs no clearing); else y += A x.
 // band_start points at one chunk's band table; the product at band-major position i is
 // bins[i - off] (off a multiple of 4), its row rowlocal[i]. FOLD adds a part of y kept in another
-// row order (PbFold), in FP64: kFoldGather adds fys[(r & ~(kHybWin - 1)) + fmap[r]] to row r as it
-// is written; kFoldScan (bands of kHybWin rows, so band b is window b) reads the band's fys in
-// order after the products and adds fys[p] to the accumulator of row fmap[p] of the band.
-constexpr int kFoldNone = 0, kFoldGather = 1, kFoldScan = 2;
-template <typename P, typename Y, int U, bool ASSIGN, int FOLD, bool S>
+// order of the band's rows (PbFold), in FP64: it is read in that order after the products, and
+// fys[p] added to the accumulator of row fmap[p] of the band.
+template <typename P, typename Y, int U, bool ASSIGN, bool FOLD, bool S>
 __global__ __launch_bounds__(kBigBlock) void k_pb2(int R, int m, const int *__restrict__ band_start,
                                                    const P *__restrict__ bins, int off,
                                                    const uint16_t *__restrict__ rowlocal, Y *__restrict__ y,
@@ -1064,36 +1074,43 @@ __global__ __launch_bounds__(kBigBlock) void k_pb2(int R, int m, const int *__re
     for (; k < nv; k += kBigBlock) T::add(acc, bv[k], rv[k]);
     __syncthreads();
     const int r0 = b * R, rows = min(R, m - r0);
-    if constexpr (FOLD == kFoldScan) {
-        // positions [r0, r0 + rows) hold the band's rows in another order: each row once, so
-        // these adds do not collide. A whole window: each thread loads its 16 consecutive
-        // positions with 16-byte loads, all in flight before the adds.
-        static_assert(kHybWin == 16 * kBigBlock, "scan fold: 16 positions per thread");
-        if (rows == kHybWin) {
-            const long long p0 = (long long)r0 + 16 * (long long)threadIdx.x;
-            constexpr int NV = 16 * (int)sizeof(Y) / 16;
-            float4 yv[NV];
-            uint4 mv[2];
+    if constexpr (FOLD) {
+        // positions [r0, r0 + rows) hold the band's rows in another order: each row once, so these adds
+        // do not collide. Four consecutive positions at a time (16-byte loads: r0 is a multiple of 64),
+        // four such groups in flight.
+        constexpr int NV = (int)sizeof(Y) / 4;  // 16-byte loads of four positions
+        const float4 *__restrict__ y4 = reinterpret_cast<const float4 *>(fys + r0);
+        const uint2 *__restrict__ m4 = reinterpret_cast<const uint2 *>(fmap + r0);
+        const int quads = rows / 4;
+        for (int q0 = threadIdx.x; q0 < quads; q0 += 4 * kBigBlock) {
+            float4 yv[4][NV];
+            uint2 mv[4];
 #pragma unroll
-            for (int j = 0; j < NV; ++j) yv[j] = reinterpret_cast<const float4 *>(fys + p0)[j];
-            mv[0] = reinterpret_cast<const uint4 *>(fmap + p0)[0];
-            mv[1] = reinterpret_cast<const uint4 *>(fmap + p0)[1];
-            const Y *yy = reinterpret_cast<const Y *>(yv);
-            const uint16_t *mm = reinterpret_cast<const uint16_t *>(mv);
+            for (int u = 0; u < 4; ++u) {
+                const int q = min(q0 + u * kBigBlock, quads - 1);
 #pragma unroll
-            for (int j = 0; j < 16; ++j) acc[mm[j]] += (double)yy[j];
-        } else {
-            for (int p = threadIdx.x; p < rows; p += kBigBlock)
-                acc[fmap[(long long)r0 + p]] += (double)fys[(long long)r0 + p];
+                for (int j = 0; j < NV; ++j) yv[u][j] = y4[q * NV + j];
+                mv[u] = m4[q];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (q0 + u * kBigBlock < quads) {
+                    const Y *yy = reinterpret_cast<const Y *>(yv[u]);
+                    acc[mv[u].x & 0xffffu] += (double)yy[0];
+                    acc[mv[u].x >> 16] += (double)yy[1];
+                    acc[mv[u].y & 0xffffu] += (double)yy[2];
+                    acc[mv[u].y >> 16] += (double)yy[3];
+                }
+            }
+        }
+        if ((int)threadIdx.x < rows - 4 * quads) {
+            const int p = r0 + 4 * quads + (int)threadIdx.x;
+            acc[fmap[p]] += (double)fys[p];
         }
         __syncthreads();
     }
     for (int r = threadIdx.x; r < rows; r += kBigBlock) {
-        double v = acc[r];
-        if constexpr (FOLD == kFoldGather) {
-            const long long g = (long long)r0 + r;
-            v += (double)fys[(g & ~(long long)(kHybWin - 1)) + fmap[g]];
-        }
+        const double v = acc[r];
         if constexpr (ASSIGN) y[r0 + r] = (Y)v;
         else y[r0 + r] += (Y)v;
     }
@@ -1157,16 +1174,12 @@ static void launch_pb(const fl_matrix *A, const V *val, const X *x, P *bins, Y *
     allow_lds(k1, std::max<size_t>(lds1, 8));
     const size_t lds2 = (size_t)A->pb_R * sizeof(double);
     const Y *fys = fold ? (const Y *)fold->ys : nullptr;
-    const bool scan = fys && fold->perm && A->pb_R == kHybWin;
-    const uint16_t *fmap = !fys ? nullptr : scan ? fold->perm : fold->iperm;
-    allow_lds(k_pb2<P, Y, 8, true, kFoldNone, S>, lds2);
-    allow_lds(k_pb2<P, Y, 8, false, kFoldNone, S>, lds2);
-    if (scan) {
-        allow_lds(k_pb2<P, Y, 8, true, kFoldScan, S>, lds2);
-        allow_lds(k_pb2<P, Y, 8, false, kFoldScan, S>, lds2);
-    } else if (fys) {
-        allow_lds(k_pb2<P, Y, 8, true, kFoldGather, S>, lds2);
-        allow_lds(k_pb2<P, Y, 8, false, kFoldGather, S>, lds2);
+    const uint16_t *fmap = fold ? fold->perm : nullptr;
+    allow_lds(k_pb2<P, Y, 8, true, false, S>, lds2);
+    allow_lds(k_pb2<P, Y, 8, false, false, S>, lds2);
+    if (fys) {
+        allow_lds(k_pb2<P, Y, 8, true, true, S>, lds2);
+        allow_lds(k_pb2<P, Y, 8, false, true, S>, lds2);
     }
     // chunk by chunk: phase 1 writes the chunk's products to the front of the product array,
     // phase 2 adds them into y (the first chunk assigns y when asked to)
@@ -1176,12 +1189,9 @@ static void launch_pb(const fl_matrix *A, const V *val, const X *x, P *bins, Y *
                                  A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p, bins);
         FL_LAUNCH_CHECK();
         // the first chunk's phase 2 writes every row once: it adds the folded part
-        const int fm = (fys && c == 0) ? (scan ? kFoldScan : kFoldGather) : kFoldNone;
-        auto k2 = (assign && c == 0)
-                      ? (fm == kFoldScan ? k_pb2<P, Y, 8, true, kFoldScan, S>
-                         : fm == kFoldGather ? k_pb2<P, Y, 8, true, kFoldGather, S> : k_pb2<P, Y, 8, true, kFoldNone, S>)
-                      : (fm == kFoldScan ? k_pb2<P, Y, 8, false, kFoldScan, S>
-                         : fm == kFoldGather ? k_pb2<P, Y, 8, false, kFoldGather, S> : k_pb2<P, Y, 8, false, kFoldNone, S>);
+        const bool add = fys && c == 0;
+        auto k2 = (assign && c == 0) ? (add ? k_pb2<P, Y, 8, true, true, S> : k_pb2<P, Y, 8, true, false, S>)
+                                     : (add ? k_pb2<P, Y, 8, false, true, S> : k_pb2<P, Y, 8, false, false, S>);
         k2<<<A->nbands, kBigBlock, lds2, s>>>(A->pb_R, A->m, A->pb_band_start.p + (size_t)c * A->nbands, bins,
                                               A->pb_chunk_off[c], A->pb_rowlocal.p, y, fys, fmap);
         FL_LAUNCH_CHECK();
