@@ -257,9 +257,10 @@ __global__ void k_check_pb(const int *__restrict__ batch_of, const uint16_t *__r
         const int bsize = batch_start[b + 1] - batch_start[b];
         if (bsize > cap || (int)lslot[g] >= bsize) atomicOr(flag, 4);
     }
-    GRID_STRIDE(b, nb) {
+    GRID_STRIDE(t, (long long)nb * 64) {  // a wave per batch
+        const long long b = t >> 6;
         const int bsize = batch_start[b + 1] - batch_start[b];
-        for (int r = run_off[b]; r < run_off[b + 1]; ++r)
+        for (int r = run_off[b] + (int)(t & 63); r < run_off[b + 1]; r += 64)
             if (run_len[r] <= 0 || run_lstart[r] < 0 || run_lstart[r] + run_len[r] > bsize || run_dest[r] < 0 ||
                 run_dest[r] + run_len[r] > ring)
                 atomicOr(flag, 8);
