@@ -159,6 +159,9 @@ void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s);
 // keys/vals are sorted in place (ping-pong through internal scratch).
 void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_t s);
 
+// Keys grouped by their top 8 bits [shift, shift + 8), and where each of the 256 groups starts.
+void radix_partition(const uint32_t *keys, uint32_t *out, int count, int shift, int *start, hipStream_t s);
+
 // Device reduction helpers.
 int device_max_i32(const int *in, int count, hipStream_t s);
 int bits_for(uint32_t v);
