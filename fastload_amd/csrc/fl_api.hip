@@ -323,7 +323,12 @@ int fl_malloc(void **dptr, size_t bytes) {
     FL_API_BEGIN
     if (!dptr) return invalid("fl_malloc: NULL");
     *dptr = nullptr;
-    FL_HIP(hipMalloc(dptr, std::max<size_t>(bytes, 1)));
+    if (hipMalloc(dptr, std::max<size_t>(bytes, 1)) != hipSuccess) {
+        (void)hipGetLastError();
+        dev_blocks_release();  // the blocks kept for later matrices
+        *dptr = nullptr;
+        FL_HIP(hipMalloc(dptr, std::max<size_t>(bytes, 1)));
+    }
     return FL_OK;
     FL_API_END
 }

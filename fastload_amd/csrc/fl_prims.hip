@@ -3,6 +3,8 @@
 // (src/formatTransform_GPU.h:402-496) and thrust::sort_by_key (src/ColSort_GPU.h:101).
 #include <atomic>
 #include <cstdarg>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "fl_common.h"
@@ -85,7 +87,6 @@ void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s) {
     exclusive_scan_i32(partial.p, partial_scan.p, nb, s);
     k_scan_tiles<<<nb, kBlock, 0, s>>>(in, out, count, partial_scan.p);
     FL_LAUNCH_CHECK();
-    // partial buffers are freed on return; hipFree synchronizes with outstanding work.
 }
 
 // ------------------------------------------------------------------------------ max-reduce
@@ -286,19 +287,184 @@ void radix_partition(const uint32_t *keys, uint32_t *out, int count, int shift, 
     FL_LAUNCH_CHECK();
 }
 
-// ------------------------------------------------------------------ temporaries' memory pool
-void tmp_pool_init() {
-    static std::atomic<unsigned long long> done{0};  // one bit per device (up to 64)
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return;
-    const unsigned long long bit = 1ull << dev;
-    if (done.load(std::memory_order_acquire) & bit) return;
-    hipMemPool_t pool;
-    if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) {
-        uint64_t keep = kTmpPoolKeep;
-        (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
+// --------------------------------------------------------------------- kept device blocks
+namespace {
+struct Kept {
+    void *p;
+    unsigned long long since;  // requests made when it was put back
+};
+struct BlockStore {
+    std::mutex mu;
+    std::multimap<std::pair<int, size_t>, Kept> blocks;  // by (device, bytes)
+    unsigned long long held = 0, requests = 0;
+};
+// never destroyed: objects may be released while the process ends
+BlockStore &block_store() {
+    static BlockStore &b = *new BlockStore();
+    return b;
+}
+
+size_t block_size(size_t bytes) {
+    const size_t grain = bytes < (1u << 20) ? 256 : 1u << 16;
+    return (bytes + grain - 1) / grain * grain;
+}
+
+// whether a block serves a request of `want` bytes (a block_size)
+bool block_fits(size_t bytes, size_t want) { return bytes >= want && bytes - bytes / 8 <= want; }
+
+// Takes the blocks that have waited longest out of the store until `room` more bytes fit, and those past
+// kBlockAge; the caller frees them without the lock.
+std::vector<void *> drop_blocks(BlockStore &b, unsigned long long room) {
+    std::vector<void *> out;
+    while (!b.blocks.empty()) {
+        auto oldest = b.blocks.begin();
+        for (auto it = b.blocks.begin(); it != b.blocks.end(); ++it)
+            if (it->second.since < oldest->second.since) oldest = it;
+        if (b.held + room <= kBlockKeep && b.requests - oldest->second.since <= kBlockAge) break;
+        out.push_back(oldest->second.p);
+        b.held -= oldest->first.second;
+        b.blocks.erase(oldest);
     }
-    done.fetch_or(bit, std::memory_order_acq_rel);
+    return out;
+}
+
+// Keeps an idle block.
+void keep_block(const DevBlock &d) {
+    if (d.bytes > kBlockKeep / 2) {
+        (void)hipFree(d.p);
+        return;
+    }
+    BlockStore &b = block_store();
+    std::vector<void *> out;
+    try {
+        std::lock_guard<std::mutex> g(b.mu);
+        out = drop_blocks(b, d.bytes);
+        b.blocks.emplace(std::make_pair(d.dev, d.bytes), Kept{d.p, b.requests});
+        b.held += d.bytes;
+    } catch (...) {  // no host memory to note it (called from destructors)
+        (void)hipFree(d.p);
+    }
+    for (void *p : out) (void)hipFree(p);
+}
+
+// This thread's released temporaries, whose kernels may still run.
+struct Pending {
+    DevBlock block;
+    hipStream_t s;
+};
+thread_local std::vector<Pending> t_pending;
+thread_local int t_depth = 0;
+
+// Waits for the temporaries' streams, then keeps the blocks (keep) or frees them.
+void settle_pending(bool keep) {
+    std::vector<Pending> done;
+    done.swap(t_pending);
+    for (size_t i = 0; i < done.size(); ++i) {
+        bool waited = false;  // for this stream
+        for (size_t k = 0; k < i && !waited; ++k) waited = done[k].s == done[i].s;
+        if (!waited && hipStreamSynchronize(done[i].s) != hipSuccess) {
+            (void)hipGetLastError();
+            keep = false;
+        }
+    }
+    for (const Pending &q : done) {
+        if (keep) keep_block(q.block);
+        else (void)hipFree(q.block.p);
+    }
+}
+}  // namespace
+
+void dev_blocks_release() {
+    BlockStore &b = block_store();
+    std::vector<void *> out;
+    {
+        std::lock_guard<std::mutex> g(b.mu);
+        for (auto &k : b.blocks) out.push_back(k.second.p);
+        b.blocks.clear();
+        b.held = 0;
+    }
+    for (void *p : out) (void)hipFree(p);
+}
+
+DevBlock dev_block_get(size_t bytes) {
+    DevBlock d;
+    FL_HIP(hipGetDevice(&d.dev));
+    d.bytes = block_size(bytes);
+    BlockStore &b = block_store();
+    {
+        std::lock_guard<std::mutex> g(b.mu);
+        ++b.requests;
+        auto it = b.blocks.lower_bound({d.dev, d.bytes});
+        if (it != b.blocks.end() && it->first.first == d.dev && block_fits(it->first.second, d.bytes)) {
+            d.p = it->second.p;
+            d.bytes = it->first.second;
+            b.held -= d.bytes;
+            b.blocks.erase(it);
+            return d;
+        }
+    }
+    if (hipMalloc(&d.p, d.bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        dev_blocks_release();
+        if (hipMalloc(&d.p, d.bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            settle_pending(false);
+            d.p = nullptr;
+            FL_HIP(hipMalloc(&d.p, d.bytes));
+        }
+    }
+    return d;
+}
+
+void dev_block_put(const DevBlock &d) {
+    int cur = d.dev;
+    (void)hipGetDevice(&cur);
+    if (cur != d.dev) (void)hipSetDevice(d.dev);
+    const bool idle = hipDeviceSynchronize() == hipSuccess;  // not while this thread captures, or after a fault
+    if (cur != d.dev) (void)hipSetDevice(cur);
+    if (!idle) {
+        (void)hipGetLastError();
+        (void)hipFree(d.p);
+        return;
+    }
+    keep_block(d);
+}
+
+DevBlock tmp_block_get(size_t bytes, hipStream_t s) {
+    const size_t want = block_size(bytes);
+    int dev = 0;
+    FL_HIP(hipGetDevice(&dev));
+    size_t best = t_pending.size();
+    for (size_t i = 0; i < t_pending.size(); ++i) {
+        const Pending &q = t_pending[i];
+        if (q.s == s && q.block.dev == dev && block_fits(q.block.bytes, want) &&
+            (best == t_pending.size() || q.block.bytes < t_pending[best].block.bytes))
+            best = i;
+    }
+    if (best < t_pending.size()) {
+        const DevBlock d = t_pending[best].block;
+        t_pending[best] = t_pending.back();
+        t_pending.pop_back();
+        return d;
+    }
+    return dev_block_get(bytes);
+}
+
+void tmp_block_put(const DevBlock &d, hipStream_t s) {
+    if (t_depth > 0) {
+        try {
+            t_pending.push_back({d, s});
+            return;
+        } catch (...) {
+        }
+    }
+    dev_block_put(d);
+}
+
+TmpScope::TmpScope() { ++t_depth; }
+
+TmpScope::~TmpScope() {
+    if (--t_depth == 0 && !t_pending.empty()) settle_pending(true);
 }
 
 // ------------------------------------------------------------------------------- errors
