@@ -67,37 +67,18 @@ __global__ void k_row_bounds(const uint32_t *__restrict__ k, int count, int m, i
     }
 }
 
-// out[k] = first row whose entries start at or after k/8 of nnz (out[0] = 0, out[8] = m)
-__global__ void k_row_split(const int *__restrict__ row_ptr, int m, int nnz, int *__restrict__ out) {
-    const int k = threadIdx.x;
-    if (k > 8) return;
-    const long long target = (long long)nnz * k / 8;
-    int lo = 0, hi = m;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (row_ptr[mid] < target) lo = mid + 1; else hi = mid;
-    }
-    out[k] = k == 8 ? m : lo;
-}
-
-static void compute_row_split(fl_matrix *A, hipStream_t s) {
-    DevBuf<int> d(9);
-    k_row_split<<<1, 64, 0, s>>>(A->row_ptr.p, A->m, A->nnz, d.p);
-    FL_LAUNCH_CHECK();
-    FL_HIP(hipMemcpyAsync(A->row_split.r, d.p, sizeof(int) * 9, hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-}
+// The row arrays end with kRowPad entries that belong to no row: the k = 1 kernel loads entries four at a time.
+constexpr int kRowPad = 4;
 
 void row_prepare(fl_matrix *A, hipStream_t s) {
     if (A->row_ready) return;
     const int nnz = A->nnz, m = A->m, T = A->tilenum;
     A->row_ptr.alloc((size_t)m + 1);
-    A->row_col.alloc(std::max(nnz, 1));
-    A->row_val32.alloc(std::max(nnz, 1));
-    A->row_val64.alloc(std::max(nnz, 1));
+    A->row_col.alloc((size_t)nnz + kRowPad);
+    A->row_val32.alloc((size_t)nnz + kRowPad);
+    A->row_val64.alloc((size_t)nnz + kRowPad);
     if (nnz == 0) {
         FL_HIP(hipMemsetAsync(A->row_ptr.p, 0, sizeof(int) * ((size_t)m + 1), s));
-        compute_row_split(A, s);
         A->row_ready = true;
         return;
     }
@@ -118,7 +99,6 @@ void row_prepare(fl_matrix *A, hipStream_t s) {
                                             A->row_val32.p, nnz);
     k_row_bounds<<<sgb((long long)m + 1), kBlock, 0, s>>>(key.p, nnz, m, A->row_ptr.p);
     FL_LAUNCH_CHECK();
-    compute_row_split(A, s);
     A->row_ready = true;
 }
 
@@ -138,9 +118,9 @@ int row_install(fl_matrix *A, const int *row_ptr, const int *row_col, const doub
         return FL_ERR_INVALID;
     }
     A->row_ptr.alloc((size_t)m + 1);
-    A->row_col.alloc(std::max(nnz, 1));
-    A->row_val64.alloc(std::max(nnz, 1));
-    A->row_val32.alloc(std::max(nnz, 1));
+    A->row_col.alloc((size_t)nnz + kRowPad);
+    A->row_val64.alloc((size_t)nnz + kRowPad);
+    A->row_val32.alloc((size_t)nnz + kRowPad);
     FL_HIP(hipMemcpyAsync(A->row_ptr.p, row_ptr, sizeof(int) * ((size_t)m + 1), hipMemcpyHostToDevice, s));
     if (nnz) {
         FL_HIP(hipMemcpyAsync(A->row_col.p, row_col, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice, s));
@@ -148,7 +128,6 @@ int row_install(fl_matrix *A, const int *row_ptr, const int *row_col, const doub
         k_row_val32<<<sgb(nnz), kBlock, 0, s>>>(A->row_val64.p, A->row_val32.p, nnz);
         FL_LAUNCH_CHECK();
     }
-    compute_row_split(A, s);
     A->row_ready = true;
     return FL_OK;
 }
@@ -161,25 +140,6 @@ template <> struct RowVec<float, 2> { using type = float2; };
 template <> struct RowVec<float, 4> { using type = float4; };
 template <> struct RowVec<double, 1> { using type = double; };
 template <> struct RowVec<double, 2> { using type = double2; };
-
-// k = 1: the waves of XCD x (workgroups with blockIdx % 8 == x; gridDim a multiple of 8) stride over the
-// row groups of that XCD's range [sp.r[x], sp.r[x+1]), so the rows in flight on one XCD at any
-// time are a contiguous window, and on matrices whose rows have local columns (bands, stencils,
-// block-diagonal batches) the X rows they gather stay in that XCD's L2.
-struct XcdRows {
-    long long wave, nwaves;
-    int r0, r1;
-};
-
-__device__ __forceinline__ XcdRows xcd_rows(const RowSplit &sp) {
-    XcdRows w;
-    const int xcd = blockIdx.x & 7;
-    w.wave = uni((int)((((blockIdx.x >> 3) * blockDim.x) + threadIdx.x) >> 6));  // wave-uniform loop
-    w.nwaves = ((long long)(gridDim.x >> 3) * blockDim.x) >> 6;
-    w.r0 = sp.r[xcd];
-    w.r1 = sp.r[xcd + 1];
-    return w;
-}
 
 // The value of lane U0 of each group of L consecutive lanes, in all lanes of the group (which must
 // all be active). DPP moves for up to 16 lanes: quad permutes, and row broadcasts (for 8 lanes
@@ -307,75 +267,107 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
     else *out = o;
 }
 
-// k = 1: LPR = 4 lanes per row; lane j sums entries e0 + j, e0 + j + 4, ... and the four partial
-// sums are added by a butterfly over the row's lanes. The order depends only on the row, so a
-// block of a stacked batch still equals its matrix run alone bit for bit. Four short gather
-// chains per row instead of one long one: the 67 M-entry power-law matrix takes 0.61 ms instead
-// of 0.88 ms with one lane per row (0.67 ms with 2 lanes, 0.59 ms with 8, which loses on short
-// rows: 9.3 vs 12.2 us on a 2.4 M-entry block-diagonal matrix of 6-entry rows).
-template <typename T, typename ACC, int LPR, int UNR>
-__global__ __launch_bounds__(kBlock) void k_spmv_rowl(RowSplit sp, const int *__restrict__ row_ptr,
-                                                      const int *__restrict__ row_col, const T *__restrict__ row_val,
-                                                      const T *__restrict__ X, T *__restrict__ Y, int accumulate) {
-    constexpr int RPW = 64 / LPR;
-    const int lane = threadIdx.x & 63;
-    const int sub = lane / LPR, j = lane % LPR;
-    const XcdRows xw = xcd_rows(sp);
-    const long long groups = ((long long)(xw.r1 - xw.r0) + RPW - 1) / RPW;
-    for (long long gq = xw.wave; gq < groups; gq += xw.nwaves) {  // uniform per wave: all lanes reach the butterfly
-        const long long r = xw.r0 + gq * RPW + sub;
-        const bool live = r < xw.r1;
-        int e0 = 0, e1 = 0;
-        if (live) {
-            e0 = row_ptr[r];
-            e1 = row_ptr[r + 1];
-        }
-        ACC acc = 0;
-        int e = e0 + j;
-        for (; e + (UNR - 1) * LPR < e1; e += UNR * LPR) {
-            int c[UNR];
-            T v[UNR], xv[UNR];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) {
-                c[u] = row_col[e + u * LPR];
-                v[u] = row_val[e + u * LPR];
-            }
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) xv[u] = X[c[u]];
-#pragma unroll
-            for (int u = 0; u < UNR; ++u) acc += (ACC)v[u] * (ACC)xv[u];
-        }
-        for (; e < e1; e += LPR) acc += (ACC)row_val[e] * (ACC)X[row_col[e]];
-#pragma unroll
-        for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-        if (live && j == 0) Y[r] = accumulate ? (T)((ACC)Y[r] + acc) : (T)acc;
-    }
+// k = 1: four lanes share a row (16 rows per wave, one group per wave); lane j adds the sums of entries
+// 4j..4j+3 of every sixteen, and a butterfly adds the four lanes' sums. The order depends only on the row, so a
+// block of a stacked batch equals its matrix run alone bit for bit.
+// Bound by the L1's turns, one per distinct line of an instruction (see k_spmm_row): a lane's four
+// entries come in one 16-byte load of columns and one or two of values (at the alignment of an
+// entry), instead of four loads that each touch the lines of all 16 rows. Loads past the row's end stay
+// inside the arrays (kRowPad); those entries gather the lane's first column again and are dropped.
+// PRE: the next sixteen entries are loaded before the gathers. That pays where rows have more than
+// sixteen entries (100^3 grid: 47 against 50 us) and costs where they do not, since the
+// gathers then wait for loads of few rows (60 stacked Zipf(2) matrices: 85 against 75 us).
+// Measured, before (four entries ahead, every fourth entry per lane) -> after: 524 K rows of diagonal
+// blocks, 24 entries each, FP32: 38 -> 26 us; 100^3 27-point grid: 70 -> 47; 80^3 in FP64: 51 -> 38; 500 K
+// uniform rows of 8: 26 -> 21; 1 M power-law rows: 117 -> 97; 60 stacked Zipf(2) matrices: 113 -> 75.
+// Two lanes per row: 32, 63, 52 us for the first three, 8 for short rows of 6 entries (10); eight: 31, 52,
+// 37 and 17 us.
+template <typename T>
+__device__ __forceinline__ void load_quad(const T *p, T *out) {
+    __builtin_memcpy(out, p, 4 * sizeof(T));
 }
 
-// Persistent grid: enough waves for the rows, at most 2048 workgroups, a multiple of 8 (one share
-// per XCD).
-static unsigned row_grid(long long m, int rows_per_wave) {
-    const long long groups = (m + rows_per_wave - 1) / rows_per_wave;
-    const unsigned g = std::min<unsigned>(grid_for(groups * 64), 256u * 8u);
-    return std::max(8u, (g + 7u) & ~7u);
+constexpr int kRowLanes = 4;
+template <typename T, typename ACC, bool PRE>
+__global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const int *__restrict__ row_ptr,
+                                                      const int *__restrict__ row_col, const T *__restrict__ row_val,
+                                                      const T *__restrict__ X, T *__restrict__ Y, int accumulate) {
+    constexpr int RPW = 64 / kRowLanes, kStep = 4 * kRowLanes;
+    const int idx = blockIdx.x >> 3;
+    const long long wg = (long long)(idx / chunk * 8 + (int)(blockIdx.x & 7)) * chunk + idx % chunk;
+    const int lane = threadIdx.x & 63, sub = lane / kRowLanes, j = lane % kRowLanes;
+    const long long r = (wg * (kBlock / 64) + (threadIdx.x >> 6)) * RPW + sub;
+    const bool live = r < m;  // all lanes reach the butterfly
+    int e0 = 0, left = 0;     // entries from this lane's next one to the row's end
+    if (live) {
+        e0 = row_ptr[r];
+        left = row_ptr[r + 1] - e0 - 4 * j;
+    }
+    const int *__restrict__ pc = row_col + e0 + 4 * j;
+    const T *__restrict__ pv = row_val + e0 + 4 * j;
+    ACC acc = 0;
+    int c[4], nc[4];
+    T v[4], nv[4];
+    if (left > 0) {
+        load_quad(pc, c);
+        load_quad(pv, v);
+    }
+    while (left > 0) {
+        pc += kStep;
+        pv += kStep;
+        if (PRE && left > kStep) {
+            load_quad(pc, nc);
+            load_quad(pv, nv);
+        }
+        T x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = X[u < left ? c[u] : c[0]];
+        ACC q = 0;  // four at a time: shorter chains of roundings
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (u < left) q += (ACC)v[u] * (ACC)x[u];
+        acc += q;
+        left -= kStep;
+        if (!PRE && left > 0) {
+            load_quad(pc, nc);
+            load_quad(pv, nv);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            c[u] = nc[u];
+            v[u] = nv[u];
+        }
+    }
+#pragma unroll
+    for (int o = kRowLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (live && j == 0) Y[r] = accumulate ? (T)((ACC)Y[r] + acc) : (T)acc;
+}
+
+// Workgroups of `rows` rows each for m rows: chunks of kRowChunk rows, shorter where that would leave an
+// XCD fewer than eight of them, and a grid of whole chunks for each XCD.
+struct RowGrid {
+    int chunk, grid;
+};
+static RowGrid row_grid(int m, int rows) {
+    const int wgs = div_up(m, rows);
+    const int chunk = std::max(1, std::min(kRowChunk / rows, wgs / 64));
+    return {chunk, 8 * chunk * div_up(wgs, 8 * chunk)};
 }
 
 template <typename T, typename ACC>
 static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    constexpr int LPR = 4;
-    k_spmv_rowl<T, ACC, LPR, 4><<<row_grid(A->m, 64 / LPR), kBlock, 0, s>>>(A->row_split, A->row_ptr.p, A->row_col.p,
-                                                                            val, X, Y, accumulate);
+    const RowGrid g = row_grid(A->m, 64 / kRowLanes * (kBlock / 64));
+    const bool pre = (long long)A->nnz > 4LL * kRowLanes * A->m;  // rows of more than one step on average
+    auto k = pre ? k_spmv_row1<T, ACC, true> : k_spmv_row1<T, ACC, false>;
+    k<<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y, accumulate);
     FL_LAUNCH_CHECK();
 }
 
 template <typename T, typename ACC, int K, int VEC>
 static void launch_row_v(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    constexpr int rows = 64 * VEC / K * (kBlock / 64);  // of a workgroup
-    const int wgs = div_up(A->m, rows);
-    // chunks of kRowChunk rows, shorter where that would leave an XCD fewer than eight of them
-    const int chunk = std::max(1, std::min(kRowChunk / rows, wgs / 64));
-    k_spmm_row<T, ACC, K, VEC><<<8 * chunk * div_up(wgs, 8 * chunk), kBlock, 0, s>>>(
-        A->m, chunk, A->row_ptr.p, A->row_col.p, val, X, Y, accumulate);
+    const RowGrid g = row_grid(A->m, 64 * VEC / K * (kBlock / 64));
+    k_spmm_row<T, ACC, K, VEC><<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y,
+                                                         accumulate);
     FL_LAUNCH_CHECK();
 }
 

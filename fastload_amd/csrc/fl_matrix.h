@@ -24,12 +24,6 @@ __device__ __forceinline__ float pack_decode(uint32_t w, const PackFmt &p) {
     return f > p.mmask ? __uint_as_float(bits) : 0.0f;
 }
 
-// Contiguous row ranges of the row-ordered kernels, one per XCD, of about equal entry counts:
-// XCD x (the workgroups with blockIdx % 8 == x) owns rows [r[x], r[x+1]).
-struct RowSplit {
-    int r[9];
-};
-
 struct fl_matrix {
     int m = 0, n = 0, nnz = 0, W = 32;
     int L = 0;        // levels (h_count)
@@ -100,7 +94,6 @@ struct fl_matrix {
     // ROW (multi-right-hand-side): the entries re-ordered by row (CSR of A, columns in the
     // original numbering, so X needs no permutation): row_ptr [m+1], row_col/row_val [nnz].
     bool row_ready = false;
-    RowSplit row_split{};
     fl::DevBuf<int> row_ptr, row_col;
     fl::DevBuf<float> row_val32;
     fl::DevBuf<double> row_val64;

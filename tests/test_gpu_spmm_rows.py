@@ -1,5 +1,5 @@
-"""GPU test of the several-right-hand-sides kernel at the edges of its steps: rows of 0 to 40 entries
-(a lane loads one of the next 16 entries), row counts around a wave's and a workgroup's share and
+"""GPU test of the row kernels at the edges of their steps: rows of 0 to 40 entries (a step is 16 entries;
+with one right-hand side a lane loads four of them at a time, up to the arrays' end), row counts around a wave's and a workgroup's share and
 around the chunks of rows dealt to the XCDs, and an X row of infinities and NaN, which may reach
 only the rows that use it (lanes past a row's end read X row 0 and drop it)."""
 import numpy as np
@@ -24,7 +24,7 @@ def rows_matrix(m, n, seed):
 
 
 @pytest.mark.parametrize("kind", [fl.VAL_F64, fl.VAL_F32], ids=["f64", "f32"])
-@pytest.mark.parametrize("k", [2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("m", [1, 15, 17, 64, 65, 1023, 1025, 9001])
 def test_spmm_row_steps(gpu, m, k, kind):
     n = 53
@@ -37,7 +37,7 @@ def test_spmm_row_steps(gpu, m, k, kind):
     np.add.at(scale, rows, np.abs(vals[:, None] * X[cols]))
     Y = run_spmm(M, X, kind, k)
     assert np.all(np.abs(Y - want) <= TOL[kind] * scale)  # empty rows: exactly 0
-    X[0, ::2], X[0, 1::2] = np.inf, np.nan
+    X[0, ::2], X[0, 1::2] = np.inf, np.nan  # k = 1: inf
     uses = np.zeros(m, bool)
     uses[rows[cols == 0]] = True
     Z = run_spmm(M, X, kind, k)
