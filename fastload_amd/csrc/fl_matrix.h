@@ -165,8 +165,9 @@ void invert_perm(const int *perm, int n, int *iperm, hipStream_t s);
 // y = A x (assign) or y += A x with one schedule. work: 2*m floats for the FAST kernel's split
 // BF16 mode. pb_bins: product array for the PB schedule (at least pb_ring entries of the value
 // kind's product type, 16-byte aligned); nullptr = the matrix's own, allocated on first use.
+// cleared: y is already zero (an assigning call of a kernel that accumulates does not clear it then).
 int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work, bool assign, hipStream_t s,
-         void *pb_bins = nullptr);
+         void *pb_bins = nullptr, bool cleared = false);
 
 // The HYB schedule's heavy part, which the first chunk's phase 2 of its PB sub-matrix adds to y.
 // ys holds the heavy sums by sorted position; the sorting windows are the PB bands, and perm[p] is the

@@ -370,12 +370,13 @@ static int spmv_check(const fl_matrix *A, int kernel, int kind, const void *work
 // clearing; the other kernels accumulate, so y is cleared with a fill kernel first (WIN and
 // WINR then store the rows a single batch owns and add the shared ones atomically).
 int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work, bool assign, hipStream_t s,
-         void *pb_bins) {
+         void *pb_bins, bool cleared) {
     const int rc = spmv_check(A, kernel, kind, work);
     if (rc) return rc;
     const size_t ybytes = (size_t)A->m * ((kind == FL_VAL_F64 || kind == FL_VAL_BF16X2) ? 8 : 4);
     // PB and HYB write every row once when assigning; the other kernels accumulate
-    if (assign && (A->tilenum == 0 || (kernel != FL_KERNEL_PB && kernel != FL_KERNEL_HYB))) zero_fill(y, ybytes, s);
+    if (assign && !cleared && (A->tilenum == 0 || (kernel != FL_KERNEL_PB && kernel != FL_KERNEL_HYB)))
+        zero_fill(y, ybytes, s);
     if (A->tilenum == 0) return FL_OK;
     if (kernel == FL_KERNEL_HYB) return spmv_hyb(A, kind, x, y, assign, s, pb_bins);
     if (kernel == FL_KERNEL_WIN || kernel == FL_KERNEL_WINR || kernel == FL_KERNEL_PB)
