@@ -178,6 +178,7 @@ int fl_formatTransform(double *timeFormatTran, double *timeFormatclas, slide_mat
     A.n = colA;
     A.nnz = nnz;
     A.W = 32;
+    A.max_col_nnz = colA ? sortnnz_tmp[colA - 1] : 0;
     DevBuf<int> sn, trow, P((size_t)colA + 1);
     DevBuf<double> tval;
     upload(sn, sortnnz_tmp, colA, s);

@@ -22,48 +22,27 @@ static unsigned sgb(long long count) { return std::max(1u, std::min<unsigned>(gr
 #define GSTRIDE(i, count) \
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < (count); i += (long long)gridDim.x * blockDim.x)
 
-// original column of every entry (tile order): tile t, lane l -> perm[tile_colidx[t] + l]
-__global__ void k_col_of(int T, int W, const int *__restrict__ tile_ptr, const int *__restrict__ tile_len,
-                         const int *__restrict__ tile_colidx, const int *__restrict__ perm, int *__restrict__ col_of) {
-    GSTRIDE(g, (long long)T * W) {
-        const long long t = g / W;
-        const int l = (int)(g - t * W);
-        if (l < tile_len[t]) col_of[tile_ptr[t] + l] = perm[tile_colidx[t] + l];
-    }
+// length of every original column
+__global__ void k_col_lengths(const int *__restrict__ perm, const int *__restrict__ sortnnz, int n, int *__restrict__ len) {
+    GSTRIDE(i, n) len[perm[i]] = sortnnz[i];
 }
 
-__global__ void k_rows_key(const int *__restrict__ col, uint32_t *__restrict__ key, int *__restrict__ order, int count) {
+__global__ void k_rows_fill(const int *__restrict__ order, const ColEntry *__restrict__ ents, int *__restrict__ rcol,
+                            double *__restrict__ rv64, float *__restrict__ rv32, int count) {
     GSTRIDE(i, count) {
-        key[i] = (uint32_t)col[i];
-        order[i] = (int)i;
+        const ColEntry e = ents[order[i]];
+        rcol[i] = e.col;
+        rv64[i] = e.val;
+        rv32[i] = (float)e.val;
     }
 }
 
-__global__ void k_rows_key2(const int *__restrict__ row, const int *__restrict__ order, uint32_t *__restrict__ key,
-                            int count) {
-    GSTRIDE(i, count) key[i] = (uint32_t)row[order[i]];
-}
-
-__global__ void k_rows_fill(const int *__restrict__ order, const int *__restrict__ col_of,
-                            const double *__restrict__ val, int *__restrict__ rcol, double *__restrict__ rv64,
-                            float *__restrict__ rv32, int count) {
-    GSTRIDE(i, count) {
-        const int g = order[i];
-        rcol[i] = col_of[g];
-        const double v = val[g];
-        rv64[i] = v;
-        rv32[i] = (float)v;
-    }
-}
-
+// start[r] = first position of a key >= r, r in [0, m]; keys ascending
 __global__ void k_row_bounds(const uint32_t *__restrict__ k, int count, int m, int *__restrict__ start) {
-    GSTRIDE(r, (long long)m + 1) {
-        int lo = 0, hi = count;
-        while (lo < hi) {
-            const int mid = (int)(((long long)lo + hi) >> 1);
-            if (k[mid] < (uint32_t)r) lo = mid + 1; else hi = mid;
-        }
-        start[r] = lo;
+    GSTRIDE(i, (long long)count + 1) {
+        const long long lo = i == 0 ? 0 : (long long)k[i - 1] + 1;
+        const long long hi = i == count ? m : (long long)k[i];
+        for (long long r = lo; r <= hi; ++r) start[r] = (int)i;
     }
 }
 
@@ -72,7 +51,7 @@ constexpr int kRowPad = 4;
 
 void row_prepare(fl_matrix *A, hipStream_t s) {
     if (A->row_ready) return;
-    const int nnz = A->nnz, m = A->m, T = A->tilenum;
+    const int nnz = A->nnz, m = A->m, n = A->n;
     A->row_ptr.alloc((size_t)m + 1);
     A->row_col.alloc((size_t)nnz + kRowPad);
     A->row_val32.alloc((size_t)nnz + kRowPad);
@@ -82,22 +61,19 @@ void row_prepare(fl_matrix *A, hipStream_t s) {
         A->row_ready = true;
         return;
     }
-    DevBuf<int> col_of(nnz), order(nnz);
-    DevBuf<uint32_t> key(nnz);
-    k_col_of<<<sgb((long long)T * A->W), kBlock, 0, s>>>(T, A->W, A->tile_ptr.p, A->tile_len.p, A->tile_colidx.p,
-                                                         A->perm.p, col_of.p);
-    // (row, original column) order: stable by column, then stable by row. The order inside a row
-    // then depends only on A, not on the column sort, so a block of a batch sums exactly as the
-    // same matrix alone.
-    k_rows_key<<<sgb(nnz), kBlock, 0, s>>>(col_of.p, key.p, order.p, nnz);
+    // (row, original column) order: the entries in original column order (columns_from_tiles), then stable by
+    // row. The order inside a row then depends only on A, not on the column sort, so a block of a batch
+    // sums exactly as the same matrix alone.
+    TmpBuf<int> len(n, s), colptr((size_t)n + 1, s), order(nnz, s);
+    TmpBuf<uint32_t> key(nnz, s);
+    TmpBuf<ColEntry> ents(nnz, s);
+    k_col_lengths<<<sgb(n), kBlock, 0, s>>>(A->perm.p, A->sortnnz.p, n, len.p);
     FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->n - 1, 0)), s);
-    k_rows_key2<<<sgb(nnz), kBlock, 0, s>>>(A->sortrowidx.p, order.p, key.p, nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(m - 1, 0)), s);
-    k_rows_fill<<<sgb(nnz), kBlock, 0, s>>>(order.p, col_of.p, A->val64.p, A->row_col.p, A->row_val64.p,
-                                            A->row_val32.p, nnz);
-    k_row_bounds<<<sgb((long long)m + 1), kBlock, 0, s>>>(key.p, nnz, m, A->row_ptr.p);
+    exclusive_scan_i32(len.p, colptr.p, n, s);
+    columns_from_tiles(A, 0, colptr.p, 0, A->perm.p, key.p, ents.p, s);
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(m - 1, 0)), s);
+    k_rows_fill<<<sgb(nnz), kBlock, 0, s>>>(order.p, ents.p, A->row_col.p, A->row_val64.p, A->row_val32.p, nnz);
+    k_row_bounds<<<sgb((long long)nnz + 1), kBlock, 0, s>>>(key.p, nnz, m, A->row_ptr.p);
     FL_LAUNCH_CHECK();
     A->row_ready = true;
 }

@@ -51,40 +51,8 @@ static int hread(const int *d, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------------ preparation
-// (sorted column, entry) pairs of every entry in tile order
-__global__ void k_hyb_scol(int T, int W, const int *__restrict__ tile_ptr, const int *__restrict__ tile_len,
-                           const int *__restrict__ tile_colidx, uint32_t *__restrict__ key, int *__restrict__ order) {
-    HSTRIDE(g, (long long)T * W) {
-        const long long t = g / W;
-        const int l = (int)(g - t * W);
-        if (l < tile_len[t]) {
-            const int e = tile_ptr[t] + l;
-            key[e] = (uint32_t)(tile_colidx[t] + l);
-            order[e] = e;
-        }
-    }
-}
-
 __global__ void k_hyb_iota(int *__restrict__ v, int count) {
     HSTRIDE(i, count) v[i] = (int)i;
-}
-
-// the light entries (first `count` of the column-sorted order) as a column-sorted CSC
-__global__ void k_hyb_light(const int *__restrict__ order, const int *__restrict__ row, const double *__restrict__ val,
-                            int count, int *__restrict__ trow, double *__restrict__ tval) {
-    HSTRIDE(i, count) {
-        const int e = order[i];
-        trow[i] = row[e];
-        tval[i] = val[e];
-    }
-}
-
-__global__ void k_hyb_rowkey(const int *__restrict__ order_h, const int *__restrict__ row, int count,
-                             uint32_t *__restrict__ key, int *__restrict__ idx) {
-    HSTRIDE(i, count) {
-        key[i] = (uint32_t)row[order_h[i]];
-        idx[i] = (int)i;
-    }
 }
 
 // ptr[r] = first i with key[i] >= r, r in [0, nb]; key ascending
@@ -129,33 +97,42 @@ __global__ void k_hyb_pairs(const int *__restrict__ rows, const int *__restrict_
 }
 
 // One lane per sorted position writes its row's slots: the heavy entries in column order, then
-// the padding (value 0, column H) up to the slice's pair rows.
-__global__ void k_hyb_fill(int m, int H, const int *__restrict__ rows, const int *__restrict__ np,
+// the padding (value 0, column H) up to the slice's pair rows (all padding past the last row). Bound by the
+// gathers of the entries, one line each; two pair rows at a time keep four in flight per lane.
+__global__ void k_hyb_fill(int m, int nslice, int H, const int *__restrict__ rows, const int *__restrict__ np,
                            const long long *__restrict__ sb, const int *__restrict__ hptr, const int *__restrict__ ridx,
-                           const int *__restrict__ order_h, const uint32_t *__restrict__ scol_h, int first_heavy,
-                           const double *__restrict__ val, uint32_t *__restrict__ col2, double *__restrict__ val2) {
-    HSTRIDE(p, m) {
+                           const ColEntry *__restrict__ ents, uint32_t *__restrict__ col2, double2 *__restrict__ val2) {
+    // one position per thread; consecutive workgroups of an XCD take consecutive slices, so the lines of the
+    // entries that a sorting window's rows share are fetched once (7.4 M heavy entries: 195 us with the slices dealt round-robin, 148 so; the three
+    // dependent reads per entry before that took 545)
+    const long long p = ((long long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) * kBlock + threadIdx.x;
+    if (p < (long long)nslice * 64) {
         const long long s = p >> 6;
-        const int lane = (int)(p & 63), r = rows[p], base = hptr[r], L = hptr[r + 1] - base;
+        const int lane = (int)(p & 63);
+        int base = 0, L = 0;
+        if (p < m) {
+            const int r = rows[p];
+            base = hptr[r];
+            L = hptr[r + 1] - base;
+        }
         const int P = np[s];
-        for (int q = 0; q < P; ++q) {
-            const long long slot = sb[s] + 64LL * q + lane;
-            uint32_t c[2];
-            double v[2];
-            for (int h = 0; h < 2; ++h) {
-                const int j = 2 * q + h;
-                if (j < L) {
-                    const int i = ridx[base + j];
-                    c[h] = scol_h[i] - (uint32_t)first_heavy;
-                    v[h] = val[order_h[i]];
-                } else {
-                    c[h] = (uint32_t)H;
-                    v[h] = 0.0;
-                }
+        for (int q = 0; q < P; q += 2) {
+            int at[4];
+            ColEntry e[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) at[h] = 2 * q + h < L ? ridx[base + 2 * q + h] : -1;
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                e[h] = ColEntry{0.0, H, 0};
+                if (at[h] >= 0) e[h] = ents[at[h]];
             }
-            col2[slot] = c[0] | (c[1] << 16);
-            val2[2 * slot] = v[0];
-            val2[2 * slot + 1] = v[1];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (q + h >= P) break;
+                const long long slot = sb[s] + 64LL * (q + h) + lane;
+                col2[slot] = (uint32_t)e[2 * h].col | ((uint32_t)e[2 * h + 1].col << 16);
+                val2[slot] = make_double2(e[2 * h].val, e[2 * h + 1].val);
+            }
         }
     }
 }
@@ -199,17 +176,8 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     A->hyb_val32.release();
     A->hyb_ys32.release();
     A->hyb_ys64.release();
-    const int m = A->m, n = A->n, nnz = A->nnz, T = A->tilenum, nl = n - H;
-    // entries by sorted column (stable: inside a column in tile order, i.e. by depth)
-    TmpBuf<uint32_t> key(std::max(nnz, 1), s);
-    TmpBuf<int> order(std::max(nnz, 1), s);
-    if (nnz > 0) {
-        k_hyb_scol<<<hg((long long)T * A->W), kBlock, 0, s>>>(T, A->W, A->tile_ptr.p, A->tile_len.p, A->tile_colidx.p,
-                                                             key.p, order.p);
-        FL_LAUNCH_CHECK();
-        radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(n - 1, 0)), s);
-    }
-    TmpBuf<int> cps((size_t)n + 1, s);
+    const int m = A->m, n = A->n, nnz = A->nnz, nl = n - H;
+    TmpBuf<int> cps((size_t)n + 1, s);  // entries of the sorted columns before each
     exclusive_scan_i32(A->sortnnz.p, cps.p, n, s);
     const int nnz_l = nl > 0 ? hread(cps.p + nl, s) : 0;
     const int nnz_h = nnz - nnz_l;
@@ -229,18 +197,9 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         L->max_col_nnz = hread(A->sortnnz.p + nl - 1, s);
     }
     {
-        TmpBuf<int> trow(std::max(nnz_l, 1), s);
-        TmpBuf<double> tval(std::max(nnz_l, 1), s);
-        if (nnz_l > 0) {
-            k_hyb_light<<<hg(nnz_l), kBlock, 0, s>>>(order.p, A->sortrowidx.p, A->val64.p, nnz_l, trow.p, tval.p);
-            FL_LAUNCH_CHECK();
-        }
         ElemSource src;
-        src.P = cps.p;
-        src.rowidx = trow.p;
-        src.val = tval.p;
-        transform_device(L.get(), L->sortnnz.p, src, s, nullptr, nullptr);
-        FL_HIP(hipStreamSynchronize(s));
+        src.parent = A;
+        transform_device(L.get(), L->sortnnz.p, src, s, nullptr, nullptr, false);
     }
     pb_prepare(L.get(), bt, R & ~63, s);  // bands of whole slices: they are the sorting windows
     const int win = A->hyb_win = L->pb_R;
@@ -257,13 +216,13 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     TmpBuf<int> hptr((size_t)m + 1, s), rows(std::max(m, 1), s), flag(1, s);
     TmpBuf<uint32_t> rkey(std::max(nnz_h, 1), s);
     TmpBuf<int> ridx(std::max(nnz_h, 1), s);
+    TmpBuf<ColEntry> ents(std::max(nnz_h, 1), s);
     FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
     FL_HIP(hipMemsetAsync(A->hyb_sb.p, 0, sizeof(long long) * ((size_t)nslice + 1), s));
     if (m > 0) {
         if (nnz_h > 0) {  // heavy entries by row (stable: inside a row by column)
-            k_hyb_rowkey<<<hg(nnz_h), kBlock, 0, s>>>(order.p + nnz_l, A->sortrowidx.p, nnz_h, rkey.p, ridx.p);
-            FL_LAUNCH_CHECK();
-            radix_sort_pairs(rkey.p, ridx.p, nnz_h, bits_for((uint32_t)(m - 1)), s);
+            columns_from_tiles(A, nl, cps.p, nnz_l, nullptr, rkey.p, ents.p, s);
+            radix_sort_positions(rkey.p, ridx.p, nnz_h, bits_for((uint32_t)(m - 1)), s);
         }
         k_hyb_bounds<<<hg((long long)nnz_h + 1), kBlock, 0, s>>>(rkey.p, nnz_h, m, hptr.p);
         FL_LAUNCH_CHECK();
@@ -295,12 +254,14 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     A->hyb_slots = slots;
     A->hyb_col2.alloc((size_t)padded);
     A->hyb_val64.alloc((size_t)padded * 2);
-    k_hyb_fill_u32<<<hg(padded), kBlock, 0, s>>>(A->hyb_col2.p, (uint32_t)H | ((uint32_t)H << 16), padded);
+    k_hyb_fill_u32<<<hg(padded - slots), kBlock, 0, s>>>(A->hyb_col2.p + slots, (uint32_t)H | ((uint32_t)H << 16),
+                                                         padded - slots);
     FL_LAUNCH_CHECK();
-    FL_HIP(hipMemsetAsync(A->hyb_val64.p, 0, sizeof(double) * (size_t)padded * 2, s));
-    if (m > 0 && nnz_h > 0) {
-        k_hyb_fill<<<hg(m), kBlock, 0, s>>>(m, H, rows.p, A->hyb_np.p, A->hyb_sb.p, hptr.p, ridx.p, order.p + nnz_l,
-                                            key.p + nnz_l, nl, A->val64.p, A->hyb_col2.p, A->hyb_val64.p);
+    FL_HIP(hipMemsetAsync(A->hyb_val64.p + 2 * slots, 0, sizeof(double) * 2 * (size_t)(padded - slots), s));
+    if (slots > 0) {
+        k_hyb_fill<<<(grid_for((long long)nslice * 64) + 7u) & ~7u, kBlock, 0, s>>>(m, nslice, H, rows.p, A->hyb_np.p, A->hyb_sb.p, hptr.p,
+                                                                 ridx.p, ents.p, A->hyb_col2.p,
+                                                                 (double2 *)A->hyb_val64.p);
         FL_LAUNCH_CHECK();
     }
     FL_HIP(hipStreamSynchronize(s));

@@ -148,16 +148,31 @@ void colsort_device(int n, const int *d_counts, int *d_perm, int *d_sortnnz, int
 //   tiled mode (tiled = true): A->sortrowidx / A->val64 already hold the elements in tile order
 //     (a layout read back from a file); only the level table, tile metadata and classification
 //     are computed
+//   parent mode: the elements are those of the parent's first n sorted columns (its levels are the first
+//     levels here), copied from its tiles
 struct ElemSource {
     bool tiled = false;
+    const fl_matrix *parent = nullptr;
     const int *P = nullptr;
     const int *colptr = nullptr;
     const int *perm = nullptr;
     const int *rowidx = nullptr;
     const double *val = nullptr;
 };
+// classify: also the segments and tile formats (the drop-in kernel's, exported with the layout)
 void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src, hipStream_t s, float *t_tran_ms,
-                      float *t_clas_ms);
+                      float *t_clas_ms, bool classify = true);
+
+// One entry of a column-ordered list: 16 bytes, so that a later gather by row takes one line per entry.
+struct ColEntry {
+    double val;
+    int col;
+    int pad;
+};
+// The entries of sorted columns [first, n) in column order, each column's by depth: entry d of sorted column i goes
+// to dst[i] + d - base: its row to rows, its value and column (col_of[i], or i - first when col_of is null) to ents.
+void columns_from_tiles(const fl_matrix *A, int first, const int *dst, int base, const int *col_of, uint32_t *rows,
+                        ColEntry *ents, hipStream_t s);
 
 // iperm[perm[i]] = i
 void invert_perm(const int *perm, int n, int *iperm, hipStream_t s);

@@ -250,21 +250,284 @@ __global__ void k_tiles(int T, int L, int n, int nnz, int W, const int *__restri
     }
 }
 
-// Tile data layout (dataTrans, formatTransform_GPU.h:152-171): one thread per (tile, lane).
-__global__ void k_tile_data(int T, int W, const int *__restrict__ tile_ptr, const int *__restrict__ tile_len,
-                            const int *__restrict__ tile_colidx, const int *__restrict__ tile_depth, ElemSource src,
-                            int *__restrict__ sortrowidx, double *__restrict__ sortval) {
+// ------------------------------------------------------------------- columns <-> tiles
+// The levels as kernels read them: element (sorted column i, depth d) is at
+//   nnzoff_k + j * tall_k * W + (d - base_k) * len + lane,  j, lane = divmod(i - col_k, W),
+// in level k (base_k <= d < base_k + tall_k), len = W except in the level's last chunk.
+struct Levels {
+    const int *__restrict__ col;
+    const int *__restrict__ base;
+    const int *__restrict__ tall;
+    const int *__restrict__ nnzoff;
+    int L, n, W;
+};
+
+struct Level {
+    int col, base, tall, off, chunks, last;  // last = length of the tiles of the last chunk
+
+    __device__ __forceinline__ void load(const Levels &lv, int k) {
+        set(lv, uni(lv.col[k]), uni(lv.base[k]), uni(lv.tall[k]), uni(lv.nnzoff[k]));
+    }
+    __device__ __forceinline__ void set(const Levels &lv, int c, int b, int t, int o) {
+        col = c;
+        base = b;
+        tall = t;
+        off = o;
+        const int width = lv.n - col;
+        chunks = (width + lv.W - 1) / lv.W;
+        last = width - (chunks - 1) * lv.W;
+    }
+    __device__ __forceinline__ int at(const Levels &lv, int i, int d) const {
+        const int w = i - col, lg = lv.W == 64 ? 6 : 5;
+        const int j = w >> lg;
+        return off + ((j * tall) << lg) + (d - base) * (j == chunks - 1 ? last : lv.W) + (w & (lv.W - 1));
+    }
+};
+
+// Walks between column order and tile order: a wave takes 64 consecutive sorted columns, a lane each, and
+// kWalkDepth consecutive depths; on the tile side its lanes touch one or two runs of consecutive positions
+// for each depth. One thread per element in tile order instead fetched a whole line of the column for
+// each entry, level after level. A long column is spread over many waves: item q of group g is its depths
+// from q * kWalkDepth on.
+// Tiles from columns, 10 M power-law entries: one thread per element 193 us, this with a lane per column on both
+// sides 139, with 16-byte pieces through LDS 121, with the levels in lanes 112 (67 M entries: 690; 4 M
+// entries of uniform columns of 8: 149 -> 56). Columns from tiles, 7.4 M entries: 242, 98 and 89 us.
+constexpr int kWalkDepth = 32;
+
+__global__ void k_walk_items(const int *__restrict__ sortnnz, int n, int groups, int *__restrict__ items) {
+    for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < groups; g += (long long)gridDim.x * blockDim.x)
+        items[g] = (sortnnz[min((int)g * 64 + 63, n - 1)] + kWalkDepth - 1) / kWalkDepth;
+}
+
+struct Walk {
+    const int *__restrict__ start;     // [groups + 1] items before each group
+    const int *__restrict__ level_of;  // [depths]
+    int groups, first_group, depths;
+};
+
+// level_of[d] = the level of depth d
+__global__ void k_depth_levels(const int *__restrict__ base, int L, int depths, int *__restrict__ level_of) {
+    for (long long d = (long long)blockIdx.x * blockDim.x + threadIdx.x; d < depths; d += (long long)gridDim.x * blockDim.x)
+        level_of[d] = find_level(base, L, (int)d);
+}
+
+// The levels of a wave's depths, those of d0 + u in lane u: read with readlane, so the walk does not wait for
+// memory where the level changes with every depth or two (long columns).
+struct LaneLevels {
+    int col, base, tall, off;
+    __device__ __forceinline__ void load(const Levels &lv, const int *__restrict__ level_of, int depths, int d0) {
+        const int k = level_of[min(d0 + (int)(threadIdx.x & (kWalkDepth - 1)), depths - 1)];
+        col = lv.col[k];
+        base = lv.base[k];
+        tall = lv.tall[k];
+        off = lv.nnzoff[k];
+    }
+    __device__ __forceinline__ Level get(const Levels &lv, int u) const {
+        Level l;
+        l.set(lv, __builtin_amdgcn_readlane(col, u), __builtin_amdgcn_readlane(base, u),
+              __builtin_amdgcn_readlane(tall, u), __builtin_amdgcn_readlane(off, u));
+        return l;
+    }
+};
+
+// The wave's item -> its group and first depth; false past the last item.
+__device__ __forceinline__ bool walk_item(const Walk &w, int &g, int &d0) {
+    const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const long long item = wave + uni(w.start[w.first_group]);
+    if (item >= uni(w.start[w.groups])) return false;
+    int lo = w.first_group, hi = w.groups - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (uni(w.start[mid]) <= item) lo = mid; else hi = mid - 1;
+    }
+    g = uni(lo);
+    d0 = ((int)item - uni(w.start[g])) * kWalkDepth;
+    return true;
+}
+
+// A wave's stage: kStageDepth entries of each of its 64 columns. The column side is accessed by pieces of 16
+// bytes, consecutive lanes on consecutive pieces of a column (a lane per column and entry makes as many
+// requests, each for a line of its own); the tile side by a lane per column.
+constexpr int kStageDepth = 8;
+struct WalkStage {
+    alignas(16) double val[64][kStageDepth];
+    alignas(16) int row[64][kStageDepth];
+    long long at[64];  // column side: position of the column's first entry
+    int len[64], col[64];
+};
+
+// Tile data layout (dataTrans, formatTransform_GPU.h:152-171) from columns: column i's entries start at
+// start[i] (start of perm[i] in colptr when start is null) of src rows and values, count entries in all.
+__global__ __launch_bounds__(kBlock) void k_fill_tiles(Walk w, Levels lv, const int *__restrict__ sortnnz,
+                                                       const int *__restrict__ start, const int *__restrict__ colptr,
+                                                       const int *__restrict__ perm, const int *__restrict__ src_row,
+                                                       const double *__restrict__ src_val, int count,
+                                                       int *__restrict__ sortrowidx, double *__restrict__ sortval) {
+    __shared__ WalkStage stage[kBlock / 64];
+    int g, d0;
+    if (!walk_item(w, g, d0)) return;
+    WalkStage &st = stage[threadIdx.x >> 6];
+    const int lane = (int)(threadIdx.x & 63), i = g * 64 + lane;
+    const int len = i < lv.n ? sortnnz[i] : 0;
+    st.len[lane] = len;
+    st.at[lane] = len > d0 ? (start ? start[i] : colptr[perm[i]]) : 0;
+    LaneLevels ll;
+    ll.load(lv, w.level_of, w.depths, d0);
+    for (int d = d0; d < d0 + kWalkDepth; d += kStageDepth) {
+        if (!ballot64(d < len)) break;
+        // pieces of 4 rows or 2 values; whole loads also past the column's end, up to the arrays' end
+#pragma unroll
+        for (int q = 0; q < kStageDepth / 4; ++q) {
+            const int t = q * 64 + lane, c = t / (kStageDepth / 4), o = t % (kStageDepth / 4) * 4;
+            const long long at = st.at[c] + d + o;
+            const int left = st.len[c] - d - o;
+            alignas(16) int row[4] = {0, 0, 0, 0};
+            if (left > 0) {
+                if (at + 4 <= count) {
+                    __builtin_memcpy(row, src_row + at, sizeof row);
+                } else {
+                    for (int u = 0; u < 4 && u < left; ++u) row[u] = src_row[at + u];
+                }
+            }
+            *reinterpret_cast<int4 *>(&st.row[c][o]) = *reinterpret_cast<int4 *>(row);
+        }
+#pragma unroll
+        for (int q = 0; q < kStageDepth / 2; ++q) {
+            const int t = q * 64 + lane, c = t / (kStageDepth / 2), o = t % (kStageDepth / 2) * 2;
+            const long long at = st.at[c] + d + o;
+            const int left = st.len[c] - d - o;
+            alignas(16) double val[2] = {0.0, 0.0};
+            if (left > 0) {
+                if (at + 2 <= count) __builtin_memcpy(val, src_val + at, sizeof val);
+                else val[0] = src_val[at];
+            }
+            *reinterpret_cast<double2 *>(&st.val[c][o]) = *reinterpret_cast<double2 *>(val);
+        }
+        __builtin_amdgcn_wave_barrier();  // the wave's own LDS accesses are in order
+#pragma unroll
+        for (int u = 0; u < kStageDepth; ++u) {
+            if (!ballot64(d + u < len)) break;
+            const Level l = ll.get(lv, d - d0 + u);
+            if (d + u < len) {
+                const int p = l.at(lv, i, d + u);
+                sortrowidx[p] = st.row[lane][u];
+                sortval[p] = st.val[lane][u];
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_columns_from_tiles(Walk w, Levels lv, const int *__restrict__ sortnnz,
+                                                               int first, const int *__restrict__ dst, int base,
+                                                               const int *__restrict__ col_of,
+                                                               const int *__restrict__ sortrowidx,
+                                                               const double *__restrict__ sortval,
+                                                               uint32_t *__restrict__ rows, ColEntry *__restrict__ ents) {
+    __shared__ WalkStage stage[kBlock / 64];
+    int g, d0;
+    if (!walk_item(w, g, d0)) return;
+    WalkStage &st = stage[threadIdx.x >> 6];
+    const int lane = (int)(threadIdx.x & 63), i = g * 64 + lane;
+    const int len = i >= first && i < lv.n ? sortnnz[i] : 0;
+    st.len[lane] = len;
+    if (len > d0) {
+        const int col = col_of ? col_of[i] : i - first;
+        st.col[lane] = col;
+        st.at[lane] = (long long)dst[col_of ? col : i] - base;
+    }
+    LaneLevels ll;
+    ll.load(lv, w.level_of, w.depths, d0);
+    for (int d = d0; d < d0 + kWalkDepth; d += kStageDepth) {
+        if (!ballot64(d < len)) break;
+        int p[kStageDepth];
+#pragma unroll
+        for (int u = 0; u < kStageDepth; ++u) {
+            const Level l = ll.get(lv, d - d0 + u);
+            p[u] = d + u < len ? l.at(lv, i, d + u) : -1;
+        }
+        int row[kStageDepth];
+        double val[kStageDepth];
+#pragma unroll
+        for (int u = 0; u < kStageDepth; ++u) {
+            row[u] = p[u] >= 0 ? sortrowidx[p[u]] : 0;
+            val[u] = p[u] >= 0 ? sortval[p[u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kStageDepth; ++u) {
+            st.row[lane][u] = row[u];
+            st.val[lane][u] = val[u];
+        }
+        __builtin_amdgcn_wave_barrier();  // the wave's own LDS accesses are in order
+#pragma unroll
+        for (int q = 0; q < kStageDepth; ++q) {  // kStageDepth lanes write a column's entries
+            const int t = q * 64 + lane, c = t / kStageDepth, o = t % kStageDepth;
+            if (d + o < st.len[c]) {
+                const long long at = st.at[c] + d + o;
+                rows[at] = (uint32_t)st.row[c][o];
+                ents[at] = ColEntry{st.val[c][o], st.col[c], 0};
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Tile data of a sub-matrix of the parent's first n sorted columns (parent mode): one thread per (tile, lane).
+__global__ void k_copy_tiles(int T, int W, const int *__restrict__ tile_ptr, const int *__restrict__ tile_len,
+                             const int *__restrict__ tile_colidx, const int *__restrict__ tile_depth,
+                             const int *__restrict__ tileoff, Levels pl, const int *__restrict__ prow,
+                             const double *__restrict__ pval, int L, int *__restrict__ sortrowidx,
+                             double *__restrict__ sortval) {
     const long long total = (long long)T * W;
     for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (long long)gridDim.x * blockDim.x) {
-        const long long t = g / W;
-        const int l = (int)(g - t * W);
+        const int t = uni((int)(g / W));  // W = 64: a wave per tile
+        const int l = (int)(g - (long long)t * W);
+        Level lev;
+        lev.load(pl, find_level(tileoff, L, t));
         if (l >= tile_len[t]) continue;
-        const int sc = tile_colidx[t] + l, d = tile_depth[t];
-        const long long at = src.P ? (long long)src.P[sc] + d : (long long)src.colptr[src.perm[sc]] + d;
+        const int at = lev.at(pl, tile_colidx[t] + l, tile_depth[t]);
         const int dst = tile_ptr[t] + l;
-        sortrowidx[dst] = src.rowidx[at];
-        sortval[dst] = src.val[at];
+        sortrowidx[dst] = prow[at];
+        sortval[dst] = pval[at];
     }
+}
+
+static Levels levels_of(const fl_matrix *A) {
+    return {A->lvl_col.p, A->lvl_base.p, A->lvl_tall.p, A->lvl_nnzoff.p, A->L, A->n, A->W};
+}
+
+// start[g] = items of the groups before g. At most walk_bound items in all: a group has as many as its longest
+// column needs, which is no longer than any column of the next group; the last two groups are bounded by
+// the longest column (the last one may have fewer than 64 columns).
+struct WalkPlan {
+    TmpBuf<int> start, level_of;
+    Walk w;
+    WalkPlan(const fl_matrix *A, const int *sortnnz, int first, hipStream_t s) : start(s), level_of(s) {
+        const int groups = div_up(A->n, 64), depths = std::max(A->max_col_nnz, 1);
+        TmpBuf<int> items(groups, s);
+        start.alloc((size_t)groups + 1);
+        level_of.alloc(depths);
+        k_walk_items<<<stride_grid(groups), kBlock, 0, s>>>(sortnnz, A->n, groups, items.p);
+        k_depth_levels<<<stride_grid(depths), kBlock, 0, s>>>(A->lvl_base.p, A->L, depths, level_of.p);
+        FL_LAUNCH_CHECK();
+        exclusive_scan_i32(items.p, start.p, groups, s);
+        w = {start.p, level_of.p, groups, first / 64, depths};
+    }
+};
+
+static long long walk_bound(int columns, long long entries, int longest) {
+    return div_up(columns, 64) + 1 + (entries / 64 + 2LL * longest) / kWalkDepth + 1;
+}
+
+static unsigned walk_grid(long long items) { return (unsigned)((items + kBlock / 64 - 1) / (kBlock / 64)); }
+
+void columns_from_tiles(const fl_matrix *A, int first, const int *dst, int base, const int *col_of, uint32_t *rows,
+                        ColEntry *ents, hipStream_t s) {
+    if (A->nnz == 0 || first >= A->n) return;
+    const WalkPlan plan(A, A->sortnnz.p, first, s);
+    k_columns_from_tiles<<<walk_grid(walk_bound(A->n - first + 64, A->nnz, A->max_col_nnz)), kBlock, 0, s>>>(
+        plan.w, levels_of(A), A->sortnnz.p, first, dst, base, col_of, A->sortrowidx.p, A->val64.p, rows, ents);
+    FL_LAUNCH_CHECK();
 }
 
 // Segments + tile format (Pre4CountRow .. Pre4tileclass, formatTransform_GPU.h:188-285):
@@ -341,7 +604,7 @@ static int read_int(const int *d, hipStream_t s) {
 }
 
 void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src, hipStream_t s, float *t_tran_ms,
-                      float *t_clas_ms) {
+                      float *t_clas_ms, bool classify) {
     const int n = A->n, nnz = A->nnz, W = A->W;
     hipEvent_t e0, e1, e2;
     FL_HIP(hipEventCreate(&e0));
@@ -383,22 +646,28 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
     A->tile_ptr.alloc((size_t)T + 1);
     A->tile_len.alloc(std::max(T, 1));
     A->tile_colidx.alloc(std::max(T, 1));
-    A->tile_format.alloc(std::max(T, 1));
+    if (classify) A->tile_format.alloc(std::max(T, 1));
     TmpBuf<int> tile_depth(std::max(T, 1), s);
     if (!src.tiled) {
         A->sortrowidx.alloc(std::max(nnz, 1));
         A->val64.alloc(std::max(nnz, 1));
     }
-    A->sortrowindex.alloc(std::max(nnz, 1));
+    if (classify) A->sortrowindex.alloc(std::max(nnz, 1));
     if (T > 0) {
         k_tiles<<<stride_grid(T), kBlock, 0, s>>>(T, L, n, nnz, W, A->lvl_col.p, A->lvl_base.p, A->lvl_tall.p,
                                                   A->lvl_tileoff.p, A->lvl_nnzoff.p, A->tile_ptr.p, A->tile_len.p,
                                                   A->tile_colidx.p, tile_depth.p);
         FL_LAUNCH_CHECK();
-        if (!src.tiled) {
-            k_tile_data<<<stride_grid((long long)T * W), kBlock, 0, s>>>(T, W, A->tile_ptr.p, A->tile_len.p,
-                                                                         A->tile_colidx.p, tile_depth.p, src,
-                                                                         A->sortrowidx.p, A->val64.p);
+        if (src.parent) {
+            k_copy_tiles<<<stride_grid((long long)T * W), kBlock, 0, s>>>(
+                T, W, A->tile_ptr.p, A->tile_len.p, A->tile_colidx.p, tile_depth.p, A->lvl_tileoff.p,
+                levels_of(src.parent), src.parent->sortrowidx.p, src.parent->val64.p, L, A->sortrowidx.p, A->val64.p);
+            FL_LAUNCH_CHECK();
+        } else if (!src.tiled) {
+            const WalkPlan plan(A, d_sortnnz, 0, s);
+            k_fill_tiles<<<walk_grid(walk_bound(n, nnz, A->max_col_nnz)), kBlock, 0, s>>>(
+                plan.w, levels_of(A), d_sortnnz, src.P, src.colptr, src.perm, src.rowidx, src.val, nnz, A->sortrowidx.p,
+                A->val64.p);
             FL_LAUNCH_CHECK();
         }
     } else {
@@ -407,33 +676,35 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
     FL_HIP(hipEventRecord(e1, s));
 
     // classification
-    TmpBuf<int> seg_count(std::max(T, 1), s);
-    A->countrow.alloc((size_t)T + 1);
-    if (T > 0) {
-        const long long waves = ((long long)T + (64 / W) - 1) / (64 / W);
-        const unsigned g = grid_for(waves * 64);
-        if (W == 32)
-            k_classify<32><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowidx.p, A->sortrowindex.p,
-                                                seg_count.p, A->tile_format.p);
-        else
-            k_classify<64><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowidx.p, A->sortrowindex.p,
-                                                seg_count.p, A->tile_format.p);
-        FL_LAUNCH_CHECK();
-    }
-    exclusive_scan_i32(seg_count.p, A->countrow.p, T, s);
-    A->segsum = read_int(A->countrow.p + T, s);
-    A->segmentoffset.alloc((size_t)A->segsum + 1);
-    FL_HIP(hipMemsetAsync(A->segmentoffset.p + A->segsum, 0, sizeof(int), s));
-    if (T > 0) {
-        const long long waves = ((long long)T + (64 / W) - 1) / (64 / W);
-        const unsigned g = grid_for(waves * 64);
-        if (W == 32)
-            k_segoff<32><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowindex.p, A->countrow.p,
-                                              A->segmentoffset.p);
-        else
-            k_segoff<64><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowindex.p, A->countrow.p,
-                                              A->segmentoffset.p);
-        FL_LAUNCH_CHECK();
+    if (classify) {
+        TmpBuf<int> seg_count(std::max(T, 1), s);
+        A->countrow.alloc((size_t)T + 1);
+        if (T > 0) {
+            const long long waves = ((long long)T + (64 / W) - 1) / (64 / W);
+            const unsigned g = grid_for(waves * 64);
+            if (W == 32)
+                k_classify<32><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowidx.p, A->sortrowindex.p,
+                                                    seg_count.p, A->tile_format.p);
+            else
+                k_classify<64><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowidx.p, A->sortrowindex.p,
+                                                    seg_count.p, A->tile_format.p);
+            FL_LAUNCH_CHECK();
+        }
+        exclusive_scan_i32(seg_count.p, A->countrow.p, T, s);
+        A->segsum = read_int(A->countrow.p + T, s);
+        A->segmentoffset.alloc((size_t)A->segsum + 1);
+        FL_HIP(hipMemsetAsync(A->segmentoffset.p + A->segsum, 0, sizeof(int), s));
+        if (T > 0) {
+            const long long waves = ((long long)T + (64 / W) - 1) / (64 / W);
+            const unsigned g = grid_for(waves * 64);
+            if (W == 32)
+                k_segoff<32><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowindex.p, A->countrow.p,
+                                                  A->segmentoffset.p);
+            else
+                k_segoff<64><<<g, kBlock, 0, s>>>(T, A->tile_ptr.p, A->tile_len.p, A->sortrowindex.p, A->countrow.p,
+                                                  A->segmentoffset.p);
+            FL_LAUNCH_CHECK();
+        }
     }
     FL_HIP(hipEventRecord(e2, s));
 

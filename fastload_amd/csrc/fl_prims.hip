@@ -1,6 +1,7 @@
 // Device primitives for the preprocessing pipeline: exclusive scan, stable LSD radix sort of
 // (key, index) pairs, max reduction. These replace the reference's CUB DeviceScan calls
 // (src/formatTransform_GPU.h:402-496) and thrust::sort_by_key (src/ColSort_GPU.h:101).
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <map>
@@ -155,7 +156,8 @@ __global__ __launch_bounds__(kBlock) void k_radix_hist(const uint32_t *__restric
 // global_base[d] + (i - local_base[d]): consecutive threads write consecutive positions of one
 // digit's run, instead of every key going straight to one of 256 scattered buckets. The tile's
 // digit counts are the differences of the scanned histogram (offsets).
-// PAIRS: the values move with the keys; else keys alone (vals_in and vals_out unused).
+// PAIRS: the values move with the keys (vals_in null: the values are the input positions); else keys alone
+// (vals_in and vals_out unused).
 template <bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t *__restrict__ keys_in,
                                                           const int *__restrict__ vals_in,
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t *__rest
         const bool valid = i < count;
         const uint32_t key = valid ? keys_in[i] : 0u;
         int val = 0;
-        if constexpr (PAIRS) val = valid ? vals_in[i] : 0;
+        if constexpr (PAIRS) val = !vals_in ? (int)i : valid ? vals_in[i] : 0;
         const int d = (int)((key >> shift) & (kRadix - 1));
         uint64_t peers = ballot64(valid);
 #pragma unroll
@@ -233,8 +235,19 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const uint32_t *__rest
     }
 }
 
-void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_t s) {
-    if (count <= 1 || bits <= 0) return;
+__global__ void k_positions(int *__restrict__ v, int count) {
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
+        v[i] = (int)i;
+}
+
+static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool positions, hipStream_t s) {
+    if (count <= 1 || bits <= 0) {
+        if (positions && count > 0) {
+            k_positions<<<std::min(grid_for(count), 65536u), kBlock, 0, s>>>(vals, count);
+            FL_LAUNCH_CHECK();
+        }
+        return;
+    }
     const int nb = div_up(count, kSortTile);
     const long long hcount = (long long)nb * kRadix;
     if (hcount > 0x7fffffffLL) {
@@ -252,7 +265,7 @@ void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_
         k_radix_hist<<<nb, kBlock, 0, s>>>(kin, count, shift, nb, hist.p);
         FL_LAUNCH_CHECK();
         exclusive_scan_i32(hist.p, offs.p, (int)hcount, s);
-        k_radix_scatter<true><<<nb, kBlock, 0, s>>>(kin, vin, kout, vout, count, shift, nb, offs.p);
+        k_radix_scatter<true><<<nb, kBlock, 0, s>>>(kin, positions && p == 0 ? nullptr : vin, kout, vout, count, shift, nb, offs.p);
         FL_LAUNCH_CHECK();
         std::swap(kin, kout);
         std::swap(vin, vout);
@@ -263,6 +276,14 @@ void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_
     }
     // no wait here: the temporaries are freed in stream order, and the caller's later work on s
     // (or its own readback) comes after the sort
+}
+
+void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_t s) {
+    sort_pairs(keys, vals, count, bits, false, s);
+}
+
+void radix_sort_positions(uint32_t *keys, int *order, int count, int bits, hipStream_t s) {
+    sort_pairs(keys, order, count, bits, true, s);
 }
 
 __global__ void k_bin_starts(const int *__restrict__ offs, int nblocks, int count, int *__restrict__ start) {
