@@ -8,7 +8,11 @@
 // per-block partial sums in FP64 that the next kernel's blocks each reduce again, so no host round
 // trip and no atomics are needed. The product's two helper launches (sp = p[perm] and the fill of q) are
 // part of the p kernel: of 53 us of an iteration on the 80^3 27-point grid in FP64 they took 10, and
-// the three vector kernels with them take 17. `check_every` iterations are captured once into a
+// the three vector kernels with them take 17. With WIN and WINR the product sums p . q as well (DotWith), so an
+// iteration is three launches: a solve on 22^3 860 -> 769 us, 40^3 1615 -> 1507, 60^3 3653 -> 3577, 80^3
+// 7615 -> 7573 (there the product takes 2 us more, and the next kernel 1 us for reading p and q anew, of the
+// 4.7 of the separate dot product). With ROW it stays a kernel of its own: parts added by atomics would make its
+// solves, the same bit for bit from run to run, differ. `check_every` iterations are captured once into a
 // hipGraph and replayed; the kernels write the residual history to pinned host memory, and between
 // replays the host reads it and stops at the first one below the tolerance. Vectors stay in the original order; values and
 // vectors are FP64 (FL_VAL_F64) or FP32 (FL_VAL_F32, dot products still summed in FP64).
@@ -27,7 +31,7 @@ namespace {
 // Blocks of the vector kernels = partial sums per dot product. Few: every block sums all partials first. A solve on
 // 80^3 and on 40^3: 512 x 1024 threads 7.76 and 2.01 ms, 512 x 512 7.54 and 1.71, 256 x 1024 7.56 and 1.74,
 // 256 x 512 7.62 and 1.61, 128 x 1024 8.07 and 1.72.
-constexpr int kParts = 256;
+constexpr int kParts = kDotParts;
 constexpr int kThreads = 512;
 
 // Sum of v over the block, returned to every thread.
@@ -42,9 +46,10 @@ __device__ double block_sum(double v, double *lds) {
     return t;
 }
 
-__device__ double sum_parts(const double *__restrict__ part, double *lds) {
+// stride: kDotStride where a product may have added the parts, 1 where blocks stored them
+__device__ double sum_parts(const double *__restrict__ part, int stride, double *lds) {
     double v = 0.0;
-    for (int i = threadIdx.x; i < kParts; i += blockDim.x) v += part[i];
+    for (int i = threadIdx.x; i < kParts; i += blockDim.x) v += part[i * stride];
     return block_sum(v, lds);
 }
 
@@ -70,17 +75,21 @@ __global__ __launch_bounds__(kThreads) void k_dot(long long n, const T *__restri
     const Range g = block_range(n);
     for (long long i = g.i; i < g.end; i += kThreads) v += (double)a[i] * (double)b[i];
     v = block_sum(v, lds);
-    if (threadIdx.x == 0) part[blockIdx.x] = v;
+    if (threadIdx.x == 0) part[blockIdx.x * kDotStride] = v;
 }
 
 // The next product's operands, written with p: sp = p in the column order of the tiles (sp null: the product
-// reads p), and q = 0 where the product adds to it (clear).
+// reads p), q = 0 where the product adds to it (clear), and the parts of p . q where it sums those (parts not null).
 template <typename T>
 struct NextProduct {
     const int *iperm;
     T *sp;
     T *q;
     int clear;
+    double *parts;
+    __device__ __forceinline__ void begin() const {
+        if (parts && threadIdx.x == 0) parts[blockIdx.x * kDotStride] = 0.0;
+    }
     __device__ __forceinline__ void put(long long i, T p) const {
         if (sp) sp[iperm[i]] = p;
         if (clear) q[i] = T(0);
@@ -95,6 +104,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_init(long long n, const T *__re
     __shared__ double lds[kThreads / 64];
     double v = 0.0;
     const Range g = block_range(n);
+    next.begin();
     for (long long i = g.i; i < g.end; i += kThreads) {
         const T ri = b[i] - next.q[i];
         r[i] = ri;
@@ -107,9 +117,10 @@ __global__ __launch_bounds__(kThreads) void k_cg_init(long long n, const T *__re
 }
 
 // dst = sum of the partials (one block)
-__global__ __launch_bounds__(kThreads) void k_finish(const double *__restrict__ part, double *__restrict__ dst) {
+__global__ __launch_bounds__(kThreads) void k_finish(const double *__restrict__ part, int stride,
+                                                     double *__restrict__ dst) {
     __shared__ double lds[kThreads / 64];
-    const double t = sum_parts(part, lds);
+    const double t = sum_parts(part, stride, lds);
     if (threadIdx.x == 0) *dst = t;
 }
 
@@ -129,7 +140,7 @@ __global__ __launch_bounds__(kThreads) void k_cg_xr(long long n, const double *_
         p0 = p[g.i];
         q0 = q[g.i];
     }
-    const double pq = sum_parts(part_pq, lds);
+    const double pq = sum_parts(part_pq, kDotStride, lds);
     const double alpha = pq > 0.0 ? *rr / pq : 0.0;
     const T a = (T)alpha;
     double v = 0.0;
@@ -159,12 +170,13 @@ __global__ __launch_bounds__(kThreads) void k_cg_p(long long n, const double *__
                                                    double *__restrict__ hist) {
     __shared__ double lds[kThreads / 64];
     const Range g = block_range(n);
+    next.begin();
     T r0 = T(0), p0 = T(0);
     if (g.i < g.end) {
         r0 = r[g.i];
         p0 = p[g.i];
     }
-    const double rn = sum_parts(part_rr, lds);
+    const double rn = sum_parts(part_rr, 1, lds);
     const double ro = *rr_old;
     const T beta = (T)(ro > 0.0 ? rn / ro : 0.0);
     for (long long i = g.i; i < g.end;) {
@@ -220,20 +232,27 @@ static bool adds_to_q(const CgState *c) {
     return c->kernel != FL_KERNEL_ROW && c->kernel != FL_KERNEL_PB && c->kernel != FL_KERNEL_HYB;
 }
 
+// Whether the product sums p . q too.
+static bool sums_pq(const CgState *c) { return c->kernel == FL_KERNEL_WIN || c->kernel == FL_KERNEL_WINR; }
+
 template <typename T>
 static NextProduct<T> next_product(CgState *c) {
     const bool row = c->kernel == FL_KERNEL_ROW;
-    return {c->A->iperm.p, row ? nullptr : vec<T>(c, 3), vec<T>(c, 2), adds_to_q(c) ? 1 : 0};
+    return {c->A->iperm.p, row ? nullptr : vec<T>(c, 3), vec<T>(c, 2), adds_to_q(c) ? 1 : 0,
+            sums_pq(c) ? c->part1.p : nullptr};
 }
 
 // q = A v. The row kernel reads v in the original column order; the other schedules read the copy sp in
-// the tiles' order. ready: sp holds v and q is clear (NextProduct); else both are done here.
+// the tiles' order. ready: sp holds v, q and the parts of v . q are clear (NextProduct), and the latter are
+// wanted; else sp and q are prepared here.
 template <typename T>
 static int product(CgState *c, const T *v, T *q, bool ready) {
     if (c->kernel == FL_KERNEL_ROW) return spmm_row(c->A, c->kind, 1, v, q, 0, c->s);
     T *sp = vec<T>(c, 3);
     if (!ready) permute_x(c->A, v, sp, sizeof(T) == 8, c->s);
-    return spmv(c->A, c->kernel, c->kind, sp, q, nullptr, true, c->s, nullptr, ready && adds_to_q(c));
+    const DotWith dot{v, c->part1.p};
+    return spmv(c->A, c->kernel, c->kind, sp, q, nullptr, true, c->s, nullptr, ready && adds_to_q(c),
+                ready && sums_pq(c) ? &dot : nullptr);
 }
 
 // One iteration: q = A p; x, r update; p update with the next product's operands. `slot` = 0/1 picks the rr
@@ -244,7 +263,7 @@ static int cg_iteration(CgState *c, T *x, int slot, int h) {
     T *r = vec<T>(c, 0), *p = vec<T>(c, 1), *q = vec<T>(c, 2);
     const int rc = product<T>(c, p, q, true);
     if (rc) return rc;
-    k_dot<T><<<kParts, kThreads, 0, c->s>>>(n, p, q, c->part1.p);
+    if (!sums_pq(c)) k_dot<T><<<kParts, kThreads, 0, c->s>>>(n, p, q, c->part1.p);
     k_cg_xr<T><<<kParts, kThreads, 0, c->s>>>(n, c->part1.p, c->sc.p + slot, x, r, p, q, c->part2.p);
     k_cg_p<T><<<kParts, kThreads, 0, c->s>>>(n, c->part2.p, c->sc.p + slot, c->sc.p + (1 - slot), p, r,
                                              next_product<T>(c), c->hist + h);
@@ -259,11 +278,11 @@ static int cg_solve(CgState *c, const T *b, T *x, int max_iter, double rtol, int
     T *r = vec<T>(c, 0), *p = vec<T>(c, 1), *q = vec<T>(c, 2);
     // ||b||, then r = b - A x, p = r, rr = r.r (eager)
     k_dot<T><<<kParts, kThreads, 0, s>>>(n, b, b, c->part1.p);
-    k_finish<<<1, kThreads, 0, s>>>(c->part1.p, c->sc.p + 2);
+    k_finish<<<1, kThreads, 0, s>>>(c->part1.p, kDotStride, c->sc.p + 2);
     const int rc = product<T>(c, x, q, false);
     if (rc) return rc;
-    k_cg_init<T><<<kParts, kThreads, 0, s>>>(n, b, r, p, next_product<T>(c), c->part1.p);
-    k_finish<<<1, kThreads, 0, s>>>(c->part1.p, c->sc.p);
+    k_cg_init<T><<<kParts, kThreads, 0, s>>>(n, b, r, p, next_product<T>(c), c->part2.p);
+    k_finish<<<1, kThreads, 0, s>>>(c->part2.p, 1, c->sc.p);
     FL_LAUNCH_CHECK();
     double h0[3];
     FL_HIP(hipMemcpyAsync(h0, c->sc.p, sizeof(double) * 3, hipMemcpyDeviceToHost, s));
@@ -346,7 +365,7 @@ int fl_cg_create(fl_cg **out, fl_matrix *A, int kernel, int val_kind) {
         const size_t n = (size_t)std::max(A->n, 1);
         if (val_kind == FL_VAL_F64) c->vec64.alloc(4 * n);
         else c->vec32.alloc(4 * n);
-        c->part1.alloc(kParts);
+        c->part1.alloc(kParts * kDotStride);
         c->part2.alloc(kParts);
         c->sc.alloc(3);
         // one eager product checks the schedule and makes any first-use allocation now, not

@@ -181,8 +181,20 @@ void invert_perm(const int *perm, int n, int *iperm, hipStream_t s);
 // BF16 mode. pb_bins: product array for the PB schedule (at least pb_ring entries of the value
 // kind's product type, 16-byte aligned); nullptr = the matrix's own, allocated on first use.
 // cleared: y is already zero (an assigning call of a kernel that accumulates does not clear it then).
+// dot: see DotWith (WIN and WINR, assigning, FL_VAL_F64 or FL_VAL_F32; the other kernels ignore it).
+struct DotWith;
 int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work, bool assign, hipStream_t s,
-         void *pb_bins = nullptr, bool cleared = false);
+         void *pb_bins = nullptr, bool cleared = false, const DotWith *dot = nullptr);
+
+// A product that also sums v . y (v in row order, of y's type) into parts[i * kDotStride], i < kDotParts, which
+// the caller has cleared; the dot product is the sum of the parts. Four parts to a 128-byte line: of one line's
+// atomics one is served at a time (3,375 batches, 80^3 grid: sixteen parts to a line 1 us slower per product,
+// one to a line the next kernel 0.2 us slower).
+constexpr int kDotParts = 256, kDotStride = 4;
+struct DotWith {
+    const void *v = nullptr;
+    double *parts = nullptr;
+};
 
 // The HYB schedule's heavy part, which the first chunk's phase 2 of its PB sub-matrix adds to y.
 // ys holds the heavy sums by sorted position; the sorting windows are the PB bands, and perm[p] is the
@@ -197,7 +209,7 @@ struct PbFold {
 // value, slot and product streams with / without the streaming hint, -1 decides by size
 // (stream_reads of batched_stream_bytes).
 int spmv_batched(fl_matrix *A, int kernel, int kind, const void *x, void *y, bool assign, hipStream_t s,
-                 void *pb_bins, const PbFold *fold = nullptr, int stream = -1);
+                 void *pb_bins, const PbFold *fold = nullptr, int stream = -1, const DotWith *dot = nullptr);
 // Bytes a WIN/WINR/PB SpMV reads once: values (+ 16-bit slots unless packed), and for PB the
 // products and their 16-bit rows read back by phase 2.
 long long batched_stream_bytes(const fl_matrix *A, int kernel, int kind);

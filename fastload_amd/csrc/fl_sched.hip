@@ -880,11 +880,14 @@ __device__ __forceinline__ void stage_group(P *stage, const TileGroup<V, X, MODE
 // the first group before the barrier that ends the slot clearing.
 // ASSIGN: y was cleared before the launch and this is its only accumulation, so a row owned by
 // this batch is stored without reading y first (shared rows still take an atomic).
-template <typename V, typename X, typename Y, int MODE, int U, int BT, int NT, bool ASSIGN>
+// DOT: the batch's part of v . (A x) besides (DotWith): every slot's sum times its row's v, in FP64,
+// whoever owns the row; one atomic per batch.
+template <typename V, typename X, typename Y, int MODE, int U, int BT, int NT, bool ASSIGN, bool DOT>
 __global__ __launch_bounds__(NT) void k_win(OrdTiles ot, int bt, const uint16_t *__restrict__ slot,
                                             const V *__restrict__ val, PackFmt pf, int spare,
                                             const X *__restrict__ x, const int *__restrict__ win_rows,
-                                            const int *__restrict__ win_off, Y *__restrict__ y) {
+                                            const int *__restrict__ win_off, Y *__restrict__ y,
+                                            const Y *__restrict__ v, double *__restrict__ dots) {
     extern __shared__ double acc[];
     const int b = blockIdx.x;
     const WaveTiles w = wave_tiles<NT>(ot, bt, b);
@@ -909,7 +912,13 @@ __global__ __launch_bounds__(NT) void k_win(OrdTiles ot, int bt, const uint16_t 
         add_group<V, X, MODE, U>(acc, cur);
         if (more) cur = nxt;
     }
+    Y fv[KP];
+    if constexpr (DOT) {
+#pragma unroll
+        for (int k = 0; k < KP; ++k) fv[k] = v[frow[k] & 0x7fffffff];
+    }
     __syncthreads();
+    double dot = 0.0;
     auto flush = [&](int i, int r) {
         if (r >= 0) {  // only this batch touches row r
             if constexpr (ASSIGN) y[r] = (Y)acc[i];
@@ -921,9 +930,26 @@ __global__ __launch_bounds__(NT) void k_win(OrdTiles ot, int bt, const uint16_t 
 #pragma unroll
     for (int k = 0; k < KP; ++k) {
         const int i = threadIdx.x + k * NT;
-        if (i < ns) flush(i, frow[k]);
+        if (i < ns) {
+            if constexpr (DOT) dot += acc[i] * (double)fv[k];
+            flush(i, frow[k]);
+        }
     }
-    for (int i = threadIdx.x + KP * NT; i < ns; i += NT) flush(i, win_rows[s0 + i]);
+    for (int i = threadIdx.x + KP * NT; i < ns; i += NT) {
+        const int r = win_rows[s0 + i];
+        if constexpr (DOT) dot += acc[i] * (double)v[r & 0x7fffffff];
+        flush(i, r);
+    }
+    if constexpr (DOT) {
+        for (int o = 32; o > 0; o >>= 1) dot += __shfl_down(dot, o, 64);
+        __shared__ double waves[NT / 64];
+        if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = dot;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < NT / 64; ++w) dot += waves[w];
+            unsafeAtomicAdd(&dots[(b & (kDotParts - 1)) * kDotStride], dot);
+        }
+    }
 }
 
 
@@ -1132,16 +1158,16 @@ static void allow_lds(K kern, size_t bytes) {
     FL_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-template <typename V, typename X, typename Y, int MODE, int NT, bool ASSIGN>
+template <typename V, typename X, typename Y, int MODE, int NT, bool ASSIGN, bool DOT>
 static auto win_kernel(int bt) {
     constexpr int U = sizeof(X) == 4 ? 8 : 4;  // tiles per group: 8 keeps the 4-byte-x kinds within 64 VGPRs
-    return (bt == 256) ? k_win<V, X, Y, MODE, U, 256, NT, ASSIGN>
-           : (bt == 128) ? k_win<V, X, Y, MODE, U, 128, NT, ASSIGN> : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN>;
+    return (bt == 256) ? k_win<V, X, Y, MODE, U, 256, NT, ASSIGN, DOT>
+           : (bt == 128) ? k_win<V, X, Y, MODE, U, 128, NT, ASSIGN, DOT> : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN, DOT>;
 }
 
 template <typename V, typename X, typename Y, int MODE>
 static void launch_win(const fl_matrix *A, const V *val, const X *x, Y *y, bool assign,
-                       hipStream_t s) {
+                       hipStream_t s, const DotWith *dot = nullptr) {
     const PackFmt pf = A->win_pf;
     const uint16_t *slot = mode_kind(MODE) == kPacked ? nullptr : A->win_slot.p;
     // LDS for the most distinct rows any batch has (at most bt*64). Workgroups of 4 waves per 64
@@ -1150,13 +1176,19 @@ static void launch_win(const fl_matrix *A, const V *val, const X *x, Y *y, bool 
     // + 64 spare slots, one per lane, for the lanes past a tile's end
     const size_t lds = ((size_t)std::max(A->win_maxslots, 1) + 64) * sizeof(double);
     const int nt = std::min(A->bt * 4, 512);
-    auto kern = (nt == 256) ? (assign ? win_kernel<V, X, Y, MODE, 256, true>(A->bt)
-                                      : win_kernel<V, X, Y, MODE, 256, false>(A->bt))
-                            : (assign ? win_kernel<V, X, Y, MODE, 512, true>(A->bt)
-                                      : win_kernel<V, X, Y, MODE, 512, false>(A->bt));
+    auto kern = (nt == 256) ? (assign ? win_kernel<V, X, Y, MODE, 256, true, false>(A->bt)
+                                      : win_kernel<V, X, Y, MODE, 256, false, false>(A->bt))
+                            : (assign ? win_kernel<V, X, Y, MODE, 512, true, false>(A->bt)
+                                      : win_kernel<V, X, Y, MODE, 512, false, false>(A->bt));
+    if constexpr (mode_kind(MODE) == kPlain && std::is_same<X, V>::value) {  // FL_VAL_F64, FL_VAL_F32
+        if (dot)
+            kern = (nt == 256) ? win_kernel<V, X, Y, MODE, 256, true, true>(A->bt)
+                               : win_kernel<V, X, Y, MODE, 512, true, true>(A->bt);
+    }
     allow_lds(kern, lds);
     kern<<<A->nbatches, nt, lds, s>>>(ord_tiles(A), A->bt, slot, val, pf, std::max(A->win_maxslots, 1), x,
-                                      A->win_rows.p, A->win_off.p, y);
+                                      A->win_rows.p, A->win_off.p, y, dot ? (const Y *)dot->v : nullptr,
+                                      dot ? dot->parts : nullptr);
     FL_LAUNCH_CHECK();
 }
 
@@ -1213,7 +1245,7 @@ long long batched_stream_bytes(const fl_matrix *A, int kernel, int kind) {
 }
 
 int spmv_batched(fl_matrix *A, int kernel, int kind, const void *x, void *y, bool assign, hipStream_t s,
-                 void *pb_bins, const PbFold *fold, int stream) {
+                 void *pb_bins, const PbFold *fold, int stream, const DotWith *dot) {
     const bool win = (kernel == FL_KERNEL_WIN || kernel == FL_KERNEL_WINR);
     double *bins64 = (double *)pb_bins;
     float *bins32 = (float *)pb_bins;
@@ -1226,14 +1258,14 @@ int spmv_batched(fl_matrix *A, int kernel, int kind, const void *x, void *y, boo
     const bool st = stream < 0 ? stream_reads(batched_stream_bytes(A, kernel, kind)) : stream != 0;
     switch (kind) {
         case FL_VAL_F64:
-            if (win) st ? launch_win<double, double, double, kPlain | kStream>(A, A->val64.p, (const double *)x, (double *)y, assign, s)
-                        : launch_win<double, double, double, kPlain>(A, A->val64.p, (const double *)x, (double *)y, assign, s);
+            if (win) st ? launch_win<double, double, double, kPlain | kStream>(A, A->val64.p, (const double *)x, (double *)y, assign, s, dot)
+                        : launch_win<double, double, double, kPlain>(A, A->val64.p, (const double *)x, (double *)y, assign, s, dot);
             else st ? launch_pb<double, double, double, double, kPlain | kStream>(A, A->val64.p, (const double *)x, bins64, (double *)y, assign, s, fold)
                     : launch_pb<double, double, double, double, kPlain>(A, A->val64.p, (const double *)x, bins64, (double *)y, assign, s, fold);
             return FL_OK;
         case FL_VAL_F32:
-            if (win) st ? launch_win<float, float, float, kPlain | kStream>(A, A->val32.p, (const float *)x, (float *)y, assign, s)
-                        : launch_win<float, float, float, kPlain>(A, A->val32.p, (const float *)x, (float *)y, assign, s);
+            if (win) st ? launch_win<float, float, float, kPlain | kStream>(A, A->val32.p, (const float *)x, (float *)y, assign, s, dot)
+                        : launch_win<float, float, float, kPlain>(A, A->val32.p, (const float *)x, (float *)y, assign, s, dot);
             else st ? launch_pb<float, float, float, float, kPlain | kStream>(A, A->val32.p, (const float *)x, bins32, (float *)y, assign, s, fold)
                     : launch_pb<float, float, float, float, kPlain>(A, A->val32.p, (const float *)x, bins32, (float *)y, assign, s, fold);
             return FL_OK;

@@ -442,7 +442,7 @@ static int spmv_check(const fl_matrix *A, int kernel, int kind, const void *work
 // clearing; the other kernels accumulate, so y is cleared with a fill kernel first (WIN and
 // WINR then store the rows a single batch owns and add the shared ones atomically).
 int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work, bool assign, hipStream_t s,
-         void *pb_bins, bool cleared) {
+         void *pb_bins, bool cleared, const DotWith *dot) {
     const int rc = spmv_check(A, kernel, kind, work);
     if (rc) return rc;
     if (assign && !cleared && kernel == FL_KERNEL_DROPIN && A->tilenum && dropin_small(A, kind)) {
@@ -462,7 +462,7 @@ int spmv(fl_matrix *A, int kernel, int kind, const void *x, void *y, void *work,
     if (A->tilenum == 0) return FL_OK;
     if (kernel == FL_KERNEL_HYB) return spmv_hyb(A, kind, x, y, assign, s, pb_bins);
     if (kernel == FL_KERNEL_WIN || kernel == FL_KERNEL_WINR || kernel == FL_KERNEL_PB)
-        return spmv_batched(A, kernel, kind, x, y, assign, s, pb_bins);
+        return spmv_batched(A, kernel, kind, x, y, assign, s, pb_bins, nullptr, -1, dot);
     if (kernel == FL_KERNEL_DROPIN) {
         if (kind == FL_VAL_F64) {
             if (A->W == 32) launch_dropin<double, 32>(A, (const double *)x, (double *)y, s);
