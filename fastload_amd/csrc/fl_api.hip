@@ -15,6 +15,8 @@ void csr2csc_device(int m, int n, int nnz, const int *d_rowptr, const int *d_col
 void sorted_copy(int n, const int *d_perm, const int *d_sortnnz, const int *d_P, const int *d_colptr,
                  const int *d_rowidx, const double *d_val, int *d_tmp_row, double *d_tmp_val, hipStream_t s);
 int check_compressed(const int *d_ptr, int count, const int *d_idx, int nnz, int limit, hipStream_t s);
+void check_begin(const int *d_ptr, int count, const int *d_idx, int nnz, int limit, HostInts &h, hipStream_t s);
+int check_result(const HostInts &h);
 void prepare_values(fl_matrix *A, int kind, hipStream_t s);
 void permute_x(const fl_matrix *A, const void *x, void *sx, bool dbl, hipStream_t s);
 void permute_raw(const int *perm, int n, const void *x, void *sx, bool dbl, hipStream_t s);
@@ -469,7 +471,22 @@ int fl_matrix_create(fl_matrix **out, int m, int n, int nnz, const int *d_colptr
     if (width != 32 && width != 64) return invalid("fl_matrix_create: width must be 32 or 64");
     if (!d_colptr || (nnz && (!d_rowidx || !d_val))) return invalid("fl_matrix_create: NULL pointer");
     hipStream_t s = (hipStream_t)stream;
-    const int bad = check_compressed(d_colptr, n, d_rowidx, nnz, m, s);
+    // the check and the longest column (of column pointers that need not be sound yet) with one wait
+    TmpBuf<int> counts(std::max(n, 1), s);
+    int longest = 0, bad = 0;
+    {
+        HostInts checked(s), lengths(s);
+        check_begin(d_colptr, n, d_rowidx, nnz, m, checked, s);
+        if (n > 0) {
+            k_col_counts<<<std::max(1u, std::min<unsigned>(grid_for(n), 65536u)), kBlock, 0, s>>>(d_colptr, n, counts.p);
+            FL_LAUNCH_CHECK();
+        }
+        max_i32_begin(counts.p, n, lengths, s);
+        (void)lengths.wait();
+        (void)checked.wait();
+        bad = check_result(checked);
+        longest = max_i32_end(lengths);
+    }
     if (bad & 2) {
         set_error("fl_matrix_create: row index out of range");
         return FL_ERR_RANGE;
@@ -481,14 +498,9 @@ int fl_matrix_create(fl_matrix **out, int m, int n, int nnz, const int *d_colptr
         A->n = n;
         A->nnz = nnz;
         A->W = width;
-        DevBuf<int> counts(std::max(n, 1));
         A->perm.alloc(std::max(n, 1));
         A->sortnnz.alloc(std::max(n, 1));
-        if (n > 0) {
-            k_col_counts<<<std::max(1u, std::min<unsigned>(grid_for(n), 65536u)), kBlock, 0, s>>>(d_colptr, n, counts.p);
-            FL_LAUNCH_CHECK();
-        }
-        A->max_col_nnz = device_max_i32(counts.p, n, s);
+        A->max_col_nnz = longest;
         colsort_device(n, counts.p, A->perm.p, A->sortnnz.p, A->max_col_nnz, s);
         A->iperm.alloc(std::max(n, 1));
         invert_perm(A->perm.p, n, A->iperm.p, s);
@@ -498,6 +510,7 @@ int fl_matrix_create(fl_matrix **out, int m, int n, int nnz, const int *d_colptr
         src.rowidx = d_rowidx;
         src.val = d_val;
         transform_device(A, A->sortnnz.p, src, s, nullptr, nullptr);
+        FL_HIP(hipStreamSynchronize(s));
     } catch (...) {
         delete A;
         throw;
@@ -574,6 +587,7 @@ int fl_matrix_prepare_values(fl_matrix *A, int val_kind, void *stream) {
     if (!A) return invalid("fl_matrix_prepare_values: NULL");
     if (val_kind < FL_VAL_F64 || val_kind > FL_VAL_PACKED) return invalid("fl_matrix_prepare_values: bad kind");
     prepare_values(A, val_kind, (hipStream_t)stream);
+    FL_HIP(hipStreamSynchronize((hipStream_t)stream));
     return FL_OK;
     FL_API_END
 }
@@ -618,6 +632,7 @@ int fl_matrix_prepare_hyb(fl_matrix *A, int heavy_cols, int batch_tiles, int ban
     const int rc = hyb_args(A, heavy_cols, batch_tiles, band_rows, "fl_matrix_prepare_hyb");
     if (rc) return rc;
     hyb_prepare(A, heavy_cols, batch_tiles, band_rows, (hipStream_t)stream);
+    FL_HIP(hipStreamSynchronize((hipStream_t)stream));
     return FL_OK;
     FL_API_END
 }
@@ -638,6 +653,7 @@ int fl_matrix_prepare_schedule(fl_matrix *A, int kernel, int batch_tiles, int ba
         const int rc = hyb_args(A, H, batch_tiles, band_rows, "fl_matrix_prepare_schedule");
         if (rc) return rc;
         hyb_prepare(A, H, batch_tiles, band_rows, (hipStream_t)stream);
+        FL_HIP(hipStreamSynchronize((hipStream_t)stream));
         return FL_OK;
     }
     if (kernel != FL_KERNEL_WIN && kernel != FL_KERNEL_WINR && kernel != FL_KERNEL_PB)
@@ -650,6 +666,7 @@ int fl_matrix_prepare_schedule(fl_matrix *A, int kernel, int batch_tiles, int ba
     hipStream_t s = (hipStream_t)stream;
     if (kernel == FL_KERNEL_WIN || kernel == FL_KERNEL_WINR) win_prepare(A, batch_tiles, kernel == FL_KERNEL_WINR, s);
     else pb_prepare(A, batch_tiles, band_rows, s);
+    FL_HIP(hipStreamSynchronize(s));
     return FL_OK;
     FL_API_END
 }

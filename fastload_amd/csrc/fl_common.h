@@ -182,10 +182,42 @@ struct TmpBuf {
     DevBlock block;
 };
 
+// Up to kHostInts ints in pinned host memory, zero at first, for what a preparation step has to know on the
+// host: kernels on stream s write them, wait() returns them after the stream. A copy of one int to
+// ordinary memory costs a copy kernel and a wait of its own, 15 to 20 us; 46 of them took a quarter of the
+// 2.9 ms that a new matrix of 8.8 M entries needs. The blocks are kept for later (one per thread in
+// preparation, and never more than kHostBlocks idle ones).
+constexpr int kHostInts = 256;
+constexpr int kHostBlocks = 64;
+class HostInts {
+  public:
+    explicit HostInts(hipStream_t st);
+    ~HostInts();
+    HostInts(const HostInts &) = delete;
+    HostInts &operator=(const HostInts &) = delete;
+    // for a kernel's argument: where int i goes
+    int *out(int i = 0) {
+        pending = true;
+        return p + i;
+    }
+    const int *wait() {
+        if (pending) FL_HIP(hipStreamSynchronize(s));
+        pending = false;
+        return p;
+    }
+    int operator[](int i) const { return p[i]; }  // after wait()
+
+  private:
+    int *p = nullptr;
+    hipStream_t s;
+    bool pending = false;
+};
+
 // ----------------------------------------------------------------- device-side primitives
 // Exclusive prefix sum: out[0]=0, out[i]=sum(in[0..i-1]), out[count]=total. in may equal out
-// only when in has count+1 entries. Returns nothing; total is on the device at out[count].
-void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s);
+// only when in has count+1 entries. Returns nothing; total is on the device at out[count], and
+// in *total (of a HostInts) when that is given.
+void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s, int *total = nullptr);
 
 // Stable LSD radix sort of (key, value) pairs by the low `bits` bits of key.
 // keys/vals are sorted in place (ping-pong through internal scratch).
@@ -198,6 +230,9 @@ void radix_partition(const uint32_t *keys, uint32_t *out, int count, int shift, 
 
 // Device reduction helpers.
 int device_max_i32(const int *in, int count, hipStream_t s);
+// The same in two steps: the kernel, and the maximum after h.wait().
+void max_i32_begin(const int *in, int count, HostInts &h, hipStream_t s);
+int max_i32_end(const HostInts &h);
 int bits_for(uint32_t v);
 
 }  // namespace fl

@@ -43,13 +43,6 @@ constexpr int kHybPairs = 2;
 
 static unsigned hg(long long threads) { return std::max(1u, std::min<unsigned>(grid_for(threads), 65536u)); }
 
-static int hread(const int *d, hipStream_t s) {
-    int h = 0;
-    FL_HIP(hipMemcpyAsync(&h, d, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    return h;
-}
-
 // ------------------------------------------------------------------------ preparation
 __global__ void k_hyb_iota(int *__restrict__ v, int count) {
     HSTRIDE(i, count) v[i] = (int)i;
@@ -145,6 +138,15 @@ __global__ void k_hyb_slot_base(const int *__restrict__ pscan, int count, long l
     HSTRIDE(i, (long long)count + 1) sb[i] = 64LL * pscan[i];
 }
 
+// the entries of the nl light columns (cps: entries before each sorted column) and the longest one, to the host
+__global__ void k_hyb_light(const int *__restrict__ cps, const int *__restrict__ sortnnz, int nl,
+                            int *__restrict__ host) {
+    if (threadIdx.x == 0) {
+        host[0] = cps[nl];
+        host[1] = sortnnz[nl - 1];
+    }
+}
+
 __global__ void k_hyb_f32(const double *__restrict__ in, float *__restrict__ out, long long count) {
     HSTRIDE(i, count) out[i] = (float)in[i];
 }
@@ -166,7 +168,6 @@ void hyb_values(fl_matrix *A, int kind, hipStream_t s) {
         FL_LAUNCH_CHECK();
     }
     if (kind == FL_VAL_F32 || kind == FL_VAL_PACKED) prepare_values(L, kind, s);
-    FL_HIP(hipStreamSynchronize(s));
 }
 
 void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
@@ -179,7 +180,12 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     const int m = A->m, n = A->n, nnz = A->nnz, nl = n - H;
     TmpBuf<int> cps((size_t)n + 1, s);  // entries of the sorted columns before each
     exclusive_scan_i32(A->sortnnz.p, cps.p, n, s);
-    const int nnz_l = nl > 0 ? hread(cps.p + nl, s) : 0;
+    HostInts h(s);  // light entries, longest light column; pair rows, a row out of its window
+    if (nl > 0) {
+        k_hyb_light<<<1, 64, 0, s>>>(cps.p, A->sortnnz.p, nl, h.out(0));
+        FL_LAUNCH_CHECK();
+    }
+    const int nnz_l = h.wait()[0];
     const int nnz_h = nnz - nnz_l;
 
     // light sub-matrix: sorted columns [0, nl) in the same order, its own tiles and PB schedule
@@ -194,7 +200,7 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         k_hyb_iota<<<hg(nl), kBlock, 0, s>>>(L->perm.p, nl);
         FL_LAUNCH_CHECK();
         FL_HIP(hipMemcpyAsync(L->sortnnz.p, A->sortnnz.p, sizeof(int) * (size_t)nl, hipMemcpyDeviceToDevice, s));
-        L->max_col_nnz = hread(A->sortnnz.p + nl - 1, s);
+        L->max_col_nnz = h[1];
     }
     {
         ElemSource src;
@@ -213,11 +219,10 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     A->hyb_iperm.alloc(std::max(m, 1));
     A->hyb_perm.alloc(std::max(m, 1));
     long long slots = 0;
-    TmpBuf<int> hptr((size_t)m + 1, s), rows(std::max(m, 1), s), flag(1, s);
+    TmpBuf<int> hptr((size_t)m + 1, s), rows(std::max(m, 1), s);
     TmpBuf<uint32_t> rkey(std::max(nnz_h, 1), s);
     TmpBuf<int> ridx(std::max(nnz_h, 1), s);
     TmpBuf<ColEntry> ents(std::max(nnz_h, 1), s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
     FL_HIP(hipMemsetAsync(A->hyb_sb.p, 0, sizeof(long long) * ((size_t)nslice + 1), s));
     if (m > 0) {
         if (nnz_h > 0) {  // heavy entries by row (stable: inside a row by column)
@@ -234,15 +239,15 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         k_hyb_winkey<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, wkey.p);
         FL_LAUNCH_CHECK();
         radix_sort_pairs(wkey.p, rows.p, m, bits_for((uint32_t)((m - 1) / win)), s);
-        k_hyb_pos<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, A->hyb_iperm.p, A->hyb_perm.p, flag.p);
+        k_hyb_pos<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, A->hyb_iperm.p, A->hyb_perm.p, h.out(3));
         TmpBuf<int> pairs(std::max(nslice, 1), s), pscan((size_t)nslice + 1, s);
         k_hyb_pairs<<<hg(nslice), kBlock, 0, s>>>(rows.p, hptr.p, m, nslice, A->hyb_np.p, pairs.p);
         FL_LAUNCH_CHECK();
-        exclusive_scan_i32(pairs.p, pscan.p, nslice, s);
+        exclusive_scan_i32(pairs.p, pscan.p, nslice, s, h.out(2));
         k_hyb_slot_base<<<hg((long long)nslice + 1), kBlock, 0, s>>>(pscan.p, nslice, A->hyb_sb.p);
         FL_LAUNCH_CHECK();
-        slots = 64LL * hread(pscan.p + nslice, s);
-        if (hread(flag.p, s)) {
+        slots = 64LL * h.wait()[2];
+        if (h[3]) {
             set_error("HYB schedule: preprocessing moved a row out of its window");
             throw HipError{hipErrorInvalidValue};
         }
@@ -264,7 +269,6 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
                                                                  (double2 *)A->hyb_val64.p);
         FL_LAUNCH_CHECK();
     }
-    FL_HIP(hipStreamSynchronize(s));
     A->hyb_light = std::move(L);
     A->hyb_H = H;
     A->hyb_bt = bt;
@@ -272,7 +276,6 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     A->hyb_grid = cu_count();
     if (A->val32.p) hyb_values(A, FL_VAL_F32, s);
     if (A->pack_wanted) hyb_values(A, FL_VAL_PACKED, s);
-    FL_HIP(hipStreamSynchronize(s));
     A->hyb_ready = true;
 }
 

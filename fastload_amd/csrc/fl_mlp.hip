@@ -13,6 +13,7 @@
 // FP32 (Adam), the forward/backward operands are their BF16 copies. Loss: cross-entropy against
 // soft targets (a distribution over schedules derived from measured times).
 #include <cmath>
+#include <cstring>
 #include <random>
 #include <vector>
 
@@ -369,11 +370,11 @@ int fl_features(int m, int n, int nnz, const int *d_colptr, const int *d_rowidx,
         set_error("fl_features: malformed CSC (column pointers not monotone from 0 to nnz, or a row index outside [0, m))");
         return FL_ERR_RANGE;
     }
-    DevBuf<double> acc(40);
-    DevBuf<int> rc(std::max(m, 1)), maxrc(1);
-    FL_HIP(hipMemsetAsync(acc.p, 0, sizeof(double) * 40, s));
-    FL_HIP(hipMemsetAsync(rc.p, 0, sizeof(int) * std::max(m, 1), s));
-    FL_HIP(hipMemsetAsync(maxrc.p, 0, sizeof(int), s));
+    // 40 sums, the largest row count, and the row counts
+    const size_t words = 41 + ((size_t)std::max(m, 1) + 1) / 2;
+    TmpBuf<double> acc(words, s);
+    int *const maxrc = reinterpret_cast<int *>(acc.p + 40), *const rc = reinterpret_cast<int *>(acc.p + 41);
+    FL_HIP(hipMemsetAsync(acc.p, 0, sizeof(double) * words, s));
     if (n > 0) {
         k_feat_cols<<<std::min(sgm(n), kFeatGroups), kBlock, 0, s>>>(d_colptr, d_rowidx, n, m, acc.p);
         FL_LAUNCH_CHECK();
@@ -387,21 +388,21 @@ int fl_features(int m, int n, int nnz, const int *d_colptr, const int *d_rowidx,
             const size_t lds = sizeof(int) << shift;
             FL_HIP(hipFuncSetAttribute((const void *)k_feat_rowcount_bins, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds));
-            k_feat_rowcount_bins<<<div_up(nnz, kFeatChunk), 1024, lds, s>>>(rows.p, nnz, shift, start.p, m, rc.p);
+            k_feat_rowcount_bins<<<div_up(nnz, kFeatChunk), 1024, lds, s>>>(rows.p, nnz, shift, start.p, m, rc);
         } else {
-            k_feat_rowcount<<<sgm(nnz), kBlock, 0, s>>>(d_rowidx, nnz, rc.p);
+            k_feat_rowcount<<<sgm(nnz), kBlock, 0, s>>>(d_rowidx, nnz, rc);
         }
         FL_LAUNCH_CHECK();
     }
     if (m > 0) {
-        k_feat_rows<<<std::min(sgm(m), kFeatGroups), kBlock, 0, s>>>(rc.p, m, acc.p, maxrc.p);
+        k_feat_rows<<<std::min(sgm(m), kFeatGroups), kBlock, 0, s>>>(rc, m, acc.p, maxrc);
         FL_LAUNCH_CHECK();
     }
+    HostInts out(s);
+    FL_HIP(hipMemcpyAsync(out.out(), acc.p, sizeof(double) * 41, hipMemcpyDeviceToHost, s));
     double h[40];
-    int hmax = 0;
-    FL_HIP(hipMemcpyAsync(h, acc.p, sizeof(double) * 40, hipMemcpyDeviceToHost, s));
-    FL_HIP(hipMemcpyAsync(&hmax, maxrc.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
+    std::memcpy(h, out.wait(), sizeof h);
+    const int hmax = out[80];
     for (int b = 0; b < 32; ++b) features[b] = n ? (float)(h[b] / n) : 0.f;
     const double mean = m ? h[34] / m : 0.0;
     const double var = m ? std::max(h[35] / m - mean * mean, 0.0) : 0.0;
@@ -553,8 +554,14 @@ int fl_mlp_predict(fl_mlp *P, const float *d_X, int batch, int *classes, float *
     P->forward(d_X, batch, s);
     const int C = P->d[3];
     std::vector<float> z((size_t)batch * C);
-    FL_HIP(hipMemcpyAsync(z.data(), P->Z[2].p, sizeof(float) * z.size(), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
+    if (z.size() <= (size_t)kHostInts) {
+        HostInts out(s);
+        FL_HIP(hipMemcpyAsync(out.out(), P->Z[2].p, sizeof(float) * z.size(), hipMemcpyDeviceToHost, s));
+        std::memcpy(z.data(), out.wait(), sizeof(float) * z.size());
+    } else {
+        FL_HIP(hipMemcpyAsync(z.data(), P->Z[2].p, sizeof(float) * z.size(), hipMemcpyDeviceToHost, s));
+        FL_HIP(hipStreamSynchronize(s));
+    }
     for (int r = 0; r < batch; ++r) {
         const float *zr = z.data() + (size_t)r * C;
         int best = 0;

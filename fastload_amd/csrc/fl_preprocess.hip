@@ -19,11 +19,6 @@
 namespace fl {
 
 // ----------------------------------------------------------------------- small kernels
-__global__ void k_iota(int *__restrict__ v, int count) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
-        v[i] = (int)i;
-}
-
 __global__ void k_copy_keys(const int *__restrict__ in, uint32_t *__restrict__ out, int count) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
         out[i] = (uint32_t)in[i];
@@ -43,40 +38,36 @@ __global__ void k_gather(const T *__restrict__ src, const int *__restrict__ idx,
 static unsigned stride_grid(long long count) { return std::max(1u, std::min<unsigned>(grid_for(count), 65536u)); }
 
 // ---------------------------------------------------------------------- input checks
-// flag bit 0: colptr not monotone / wrong ends; bit 1: row index out of range.
-__global__ void k_check_ptr(const int *__restrict__ ptr, int count, int nnz, int *__restrict__ flag) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x) {
+// bad[0] (host memory): ptr not monotone / wrong ends; bad[1]: index out of range. Nothing is written for a
+// sound matrix.
+__global__ void k_check(const int *__restrict__ ptr, int count, const int *__restrict__ idx, int nnz, int limit,
+                        int *__restrict__ bad) {
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+    for (long long i = t; i < count; i += step) {
         const int a = ptr[i], b = ptr[i + 1];
-        if (a > b || a < 0 || b > nnz) atomicOr(flag, 1);
+        if (a > b || a < 0 || b > nnz) bad[0] = 1;
     }
-}
-
-__global__ void k_check_idx(const int *__restrict__ idx, int count, int limit, int *__restrict__ flag) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x) {
+    if (t == 0 && (ptr[0] != 0 || ptr[count] != nnz)) bad[0] = 1;
+    for (long long i = t; i < nnz; i += step) {
         const int r = idx[i];
-        if (r < 0 || r >= limit) atomicOr(flag, 2);
+        if (r < 0 || r >= limit) bad[1] = 1;
     }
 }
 
-// Returns 0 if ptr[0]==0, ptr[count]==nnz, ptr monotone and every idx in [0, limit).
+// Starts the check that ptr[0]==0, ptr[count]==nnz, ptr is monotone and every idx in [0, limit); after h.wait(),
+// check_result is 0 if so, else bit 0: ptr, bit 1: idx.
+void check_begin(const int *d_ptr, int count, const int *d_idx, int nnz, int limit, HostInts &h, hipStream_t s) {
+    k_check<<<stride_grid(std::max(count, nnz)), kBlock, 0, s>>>(d_ptr, count, d_idx, nnz, limit, h.out());
+    FL_LAUNCH_CHECK();
+}
+
+int check_result(const HostInts &h) { return (h[0] ? 1 : 0) | (h[1] ? 2 : 0); }
+
 int check_compressed(const int *d_ptr, int count, const int *d_idx, int nnz, int limit, hipStream_t s) {
-    TmpBuf<int> flag(1, s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
-    if (count > 0) {
-        k_check_ptr<<<stride_grid(count), kBlock, 0, s>>>(d_ptr, count, nnz, flag.p);
-        FL_LAUNCH_CHECK();
-    }
-    if (nnz > 0) {
-        k_check_idx<<<stride_grid(nnz), kBlock, 0, s>>>(d_idx, nnz, limit, flag.p);
-        FL_LAUNCH_CHECK();
-    }
-    int ends[2] = {0, 0}, h = 0;
-    FL_HIP(hipMemcpyAsync(&ends[0], d_ptr, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipMemcpyAsync(&ends[1], d_ptr + count, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipMemcpyAsync(&h, flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    if (ends[0] != 0 || ends[1] != nnz) h |= 1;
-    return h;
+    HostInts h(s);
+    check_begin(d_ptr, count, d_idx, nnz, limit, h, s);
+    (void)h.wait();
+    return check_result(h);
 }
 
 // ------------------------------------------------------------------------------ csr2csc
@@ -108,10 +99,9 @@ void csr2csc_device(int m, int n, int nnz, const int *d_rowptr, const int *d_col
         TmpBuf<uint32_t> keys(nnz, s);
         TmpBuf<int> order(nnz, s), row_of(nnz, s);
         k_copy_keys<<<stride_grid(nnz), kBlock, 0, s>>>(d_colind, keys.p, nnz);
-        k_iota<<<stride_grid(nnz), kBlock, 0, s>>>(order.p, nnz);
         k_row_of<<<stride_grid(m), kBlock, 0, s>>>(d_rowptr, m, row_of.p);
         FL_LAUNCH_CHECK();
-        radix_sort_pairs(keys.p, order.p, nnz, bits_for((uint32_t)std::max(n - 1, 0)), s);
+        radix_sort_positions(keys.p, order.p, nnz, bits_for((uint32_t)std::max(n - 1, 0)), s);
         k_csc_fill<<<stride_grid(nnz), kBlock, 0, s>>>(order.p, row_of.p, d_val, d_cscrow, d_cscval, nnz);
         k_count<<<stride_grid(nnz), kBlock, 0, s>>>(keys.p, nnz, d_nnzpercol);
         FL_LAUNCH_CHECK();
@@ -125,9 +115,8 @@ void colsort_device(int n, const int *d_counts, int *d_perm, int *d_sortnnz, int
     if (n <= 0) return;
     TmpBuf<uint32_t> keys(n, s);
     k_copy_keys<<<stride_grid(n), kBlock, 0, s>>>(d_counts, keys.p, n);
-    k_iota<<<stride_grid(n), kBlock, 0, s>>>(d_perm, n);
     FL_LAUNCH_CHECK();
-    radix_sort_pairs(keys.p, d_perm, n, bits_for((uint32_t)max_key), s);
+    radix_sort_positions(keys.p, d_perm, n, bits_for((uint32_t)max_key), s);
     k_keys_to_int<<<stride_grid(n), kBlock, 0, s>>>(keys.p, d_sortnnz, n);
     FL_LAUNCH_CHECK();
 }
@@ -177,12 +166,10 @@ __global__ void k_lower_bound(const int *__restrict__ sorted, int n, int key, in
 void sorted_copy(int n, const int *d_perm, const int *d_sortnnz, const int *d_P, const int *d_colptr,
                  const int *d_rowidx, const double *d_val, int *d_tmp_row, double *d_tmp_val, hipStream_t s) {
     if (n <= 0) return;
-    TmpBuf<int> lf(1, s);
-    k_lower_bound<<<1, 64, 0, s>>>(d_sortnnz, n, 64, lf.p);
+    HostInts lf(s);
+    k_lower_bound<<<1, 64, 0, s>>>(d_sortnnz, n, 64, lf.out());
     FL_LAUNCH_CHECK();
-    int long_from = n;
-    FL_HIP(hipMemcpyAsync(&long_from, lf.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
+    const int long_from = *lf.wait();
     if (long_from > 0) {
         k_sorted_copy_short<<<stride_grid(long_from), kBlock, 0, s>>>(n, long_from, d_perm, d_P, d_colptr, d_rowidx,
                                                                        d_val, d_tmp_row, d_tmp_val);
@@ -596,21 +583,18 @@ __global__ void k_group_level(int T, int L, const int *__restrict__ tileoff, int
         group_level[gidx] = find_level(tileoff, L, (int)(gidx * 64));
 }
 
-static int read_int(const int *d, hipStream_t s) {
-    int h = 0;
-    FL_HIP(hipMemcpyAsync(&h, d, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    return h;
-}
-
 void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src, hipStream_t s, float *t_tran_ms,
                       float *t_clas_ms, bool classify) {
     const int n = A->n, nnz = A->nnz, W = A->W;
-    hipEvent_t e0, e1, e2;
-    FL_HIP(hipEventCreate(&e0));
-    FL_HIP(hipEventCreate(&e1));
-    FL_HIP(hipEventCreate(&e2));
-    FL_HIP(hipEventRecord(e0, s));
+    HostInts h(s);  // levels; tiles and entries they cover; segments
+    const bool timed = t_tran_ms || t_clas_ms;
+    hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
+    if (timed) {
+        FL_HIP(hipEventCreate(&e0));
+        FL_HIP(hipEventCreate(&e1));
+        FL_HIP(hipEventCreate(&e2));
+        FL_HIP(hipEventRecord(e0, s));
+    }
 
     // levels
     TmpBuf<int> flags(std::max(n, 1), s), lidx((size_t)n + 1, s);
@@ -618,8 +602,8 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
         k_level_flags<<<stride_grid(n), kBlock, 0, s>>>(d_sortnnz, n, flags.p);
         FL_LAUNCH_CHECK();
     }
-    exclusive_scan_i32(flags.p, lidx.p, n, s);
-    const int L = read_int(lidx.p + n, s);
+    exclusive_scan_i32(flags.p, lidx.p, n, s, h.out(0));
+    const int L = h.wait()[0];
     A->L = L;
     A->lvl_col.alloc(std::max(L, 1));
     A->lvl_base.alloc(std::max(L, 1));
@@ -632,10 +616,10 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
                                                        A->lvl_tall.p, lvl_tiles.p, lvl_nnz.p);
         FL_LAUNCH_CHECK();
     }
-    exclusive_scan_i32(lvl_tiles.p, A->lvl_tileoff.p, L, s);
-    exclusive_scan_i32(lvl_nnz.p, A->lvl_nnzoff.p, L, s);
-    const int T = read_int(A->lvl_tileoff.p + L, s);
-    const int total = read_int(A->lvl_nnzoff.p + L, s);
+    exclusive_scan_i32(lvl_tiles.p, A->lvl_tileoff.p, L, s, h.out(1));
+    exclusive_scan_i32(lvl_nnz.p, A->lvl_nnzoff.p, L, s, h.out(2));
+    const int T = h.wait()[1];
+    const int total = h[2];
     if (total != nnz) {
         set_error("formatTransform: level table covers %d elements, expected nnz=%d", total, nnz);
         throw HipError{hipErrorInvalidValue};
@@ -673,7 +657,7 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
     } else {
         FL_HIP(hipMemsetAsync(A->tile_ptr.p, 0, sizeof(int), s));
     }
-    FL_HIP(hipEventRecord(e1, s));
+    if (timed) FL_HIP(hipEventRecord(e1, s));
 
     // classification
     if (classify) {
@@ -690,8 +674,8 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
                                                     seg_count.p, A->tile_format.p);
             FL_LAUNCH_CHECK();
         }
-        exclusive_scan_i32(seg_count.p, A->countrow.p, T, s);
-        A->segsum = read_int(A->countrow.p + T, s);
+        exclusive_scan_i32(seg_count.p, A->countrow.p, T, s, h.out(3));
+        A->segsum = h.wait()[3];
         A->segmentoffset.alloc((size_t)A->segsum + 1);
         FL_HIP(hipMemsetAsync(A->segmentoffset.p + A->segsum, 0, sizeof(int), s));
         if (T > 0) {
@@ -706,7 +690,7 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
             FL_LAUNCH_CHECK();
         }
     }
-    FL_HIP(hipEventRecord(e2, s));
+    if (timed) FL_HIP(hipEventRecord(e2, s));
 
     // group -> level hints for the FAST kernel
     const long long groups = ((long long)T + 63) / 64;
@@ -715,6 +699,7 @@ void transform_device(fl_matrix *A, const int *d_sortnnz, const ElemSource &src,
         k_group_level<<<stride_grid(groups), kBlock, 0, s>>>(T, L, A->lvl_tileoff.p, A->group_level.p);
         FL_LAUNCH_CHECK();
     }
+    if (!timed) return;
     FL_HIP(hipEventSynchronize(e2));
     FL_HIP(hipStreamSynchronize(s));
     float a = 0.f, b = 0.f;

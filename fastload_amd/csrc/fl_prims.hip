@@ -13,9 +13,18 @@
 namespace fl {
 
 // --------------------------------------------------------------------------------- scan
+// A scan is bound by its launches: the largest of a preparation, 8.8 M flags, moves 105 MB in 23 us, most have
+// below 100 K elements, and a launch and the gap before it take about 5 us. One workgroup scans up to
+// kScanSmall elements; above that the tiles' sums are one launch, and each tile then adds up the sums before
+// its own itself, instead of a third launch that scans them (up to kScanTiles tiles; 4,096 sums are 16 loads per
+// thread). A radix pass: 5 launches -> 4, and 3 for up to 262,144 keys.
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;  // 2048 elements per block
+constexpr int kScanTiles = 4096;
+constexpr int kScanBig = 1024, kScanBigItems = 16;
+constexpr int kScanSmall = kScanBig * kScanBigItems;
 
+template <int NT>
 __device__ __forceinline__ int block_exclusive_scan(int v, int *lds_wave, int &block_total) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int incl = wave_inclusive_scan(v);
@@ -23,7 +32,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *lds_wave, int &b
     __syncthreads();
     int prefix = 0, total = 0;
 #pragma unroll
-    for (int i = 0; i < kBlock / kWave; ++i) {
+    for (int i = 0; i < NT / kWave; ++i) {
         const int x = lds_wave[i];
         prefix += (i < w) ? x : 0;
         total += x;
@@ -42,57 +51,117 @@ __global__ __launch_bounds__(kBlock) void k_tile_sums(const int *__restrict__ in
         s += (i < count) ? in[i] : 0;
     }
     int total;
-    (void)block_exclusive_scan(s, lds_wave, total);
+    (void)block_exclusive_scan<kBlock>(s, lds_wave, total);
     if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kBlock) void k_scan_tiles(const int *__restrict__ in, int *__restrict__ out, int count,
-                                                       const int *__restrict__ carry_in) {
-    __shared__ int lds_wave[kBlock / kWave];
-    const long long base = (long long)blockIdx.x * kScanTile + (long long)threadIdx.x * kScanItems;
-    int v[kScanItems];
+// sums: the tiles' sums, scanned (SCANNED) or as they are; null with one tile. host: also gets the total, or null.
+template <int NT, int ITEMS, bool SCANNED>
+__global__ __launch_bounds__(NT) void k_scan_tiles(const int *__restrict__ in, int *__restrict__ out, int count,
+                                                   const int *__restrict__ sums, int *__restrict__ host) {
+    __shared__ int lds_wave[NT / kWave], lds_carry[NT / kWave];
+    const long long base = ((long long)blockIdx.x * NT + threadIdx.x) * ITEMS;
+    int v[ITEMS];
     int s = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const long long i = base + k;
         v[k] = (i < count) ? in[i] : 0;
         s += v[k];
     }
+    int carry = 0;
+    if (SCANNED) {
+        carry = sums[blockIdx.x];
+    } else if (sums) {
+        int c = 0;
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += NT) c += sums[i];
+        (void)block_exclusive_scan<NT>(c, lds_carry, carry);
+    }
     int total;
-    const int excl = block_exclusive_scan(s, lds_wave, total);
-    const int carry = carry_in ? carry_in[blockIdx.x] : 0;
+    const int excl = block_exclusive_scan<NT>(s, lds_wave, total);
     int run = carry + excl;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < ITEMS; ++k) {
         const long long i = base + k;
         if (i < count) out[i] = run;
         run += v[k];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[count] = carry + total;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        out[count] = carry + total;
+        if (host) *host = carry + total;
+    }
 }
 
-void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s) {
+void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s, int *total) {
     if (count <= 0) {
         FL_HIP(hipMemsetAsync(out, 0, sizeof(int), s));
         return;
     }
     const int nb = div_up(count, kScanTile);
-    if (nb == 1) {
-        k_scan_tiles<<<1, kBlock, 0, s>>>(in, out, count, nullptr);
+    if (count <= kScanSmall) {
+        if (nb == 1) k_scan_tiles<kBlock, kScanItems, false><<<1, kBlock, 0, s>>>(in, out, count, nullptr, total);
+        else k_scan_tiles<kScanBig, kScanBigItems, false><<<1, kScanBig, 0, s>>>(in, out, count, nullptr, total);
         FL_LAUNCH_CHECK();
         return;
     }
-    TmpBuf<int> partial(nb, s), partial_scan((size_t)nb + 1, s);
+    TmpBuf<int> partial(nb, s);
     k_tile_sums<<<nb, kBlock, 0, s>>>(in, count, partial.p);
     FL_LAUNCH_CHECK();
+    if (nb <= kScanTiles) {
+        k_scan_tiles<kBlock, kScanItems, false><<<nb, kBlock, 0, s>>>(in, out, count, partial.p, total);
+        FL_LAUNCH_CHECK();
+        return;
+    }
+    TmpBuf<int> partial_scan((size_t)nb + 1, s);
     exclusive_scan_i32(partial.p, partial_scan.p, nb, s);
-    k_scan_tiles<<<nb, kBlock, 0, s>>>(in, out, count, partial_scan.p);
+    k_scan_tiles<kBlock, kScanItems, true><<<nb, kBlock, 0, s>>>(in, out, count, partial_scan.p, total);
     FL_LAUNCH_CHECK();
 }
 
+// ------------------------------------------------------------------------------ ints read by the host
+namespace {
+struct HostBlocks {
+    std::mutex mu;
+    std::vector<int *> idle;
+};
+// never destroyed: see block_store
+HostBlocks &host_blocks() {
+    static HostBlocks &b = *new HostBlocks();
+    return b;
+}
+}  // namespace
+
+HostInts::HostInts(hipStream_t st) : s(st) {
+    {
+        HostBlocks &b = host_blocks();
+        std::lock_guard<std::mutex> g(b.mu);
+        if (!b.idle.empty()) {
+            p = b.idle.back();
+            b.idle.pop_back();
+        }
+    }
+    if (!p) FL_HIP(hipHostMalloc((void **)&p, sizeof(int) * kHostInts, hipHostMallocPortable));
+    std::fill_n(p, kHostInts, 0);
+}
+
+HostInts::~HostInts() {
+    // kernels may still be writing when an error took the caller past its wait
+    bool keep = !pending || hipStreamSynchronize(s) == hipSuccess;
+    if (keep) {
+        HostBlocks &b = host_blocks();
+        std::lock_guard<std::mutex> g(b.mu);
+        keep = b.idle.size() < (size_t)kHostBlocks;
+        if (keep) try {
+                b.idle.push_back(p);
+            } catch (...) {
+                keep = false;
+            }
+    }
+    if (!keep) (void)hipHostFree(p);
+}
+
 // ------------------------------------------------------------------------------ max-reduce
-// One atomic per workgroup, and at most 256 workgroups: atomics on one address run one after another, about
-// 10 ns each (600 K values with one per wave of 2,048 workgroups: 96 us; now 6).
+// One value per workgroup, at most kHostInts workgroups, and the host takes the largest.
 __global__ __launch_bounds__(kBlock) void k_max_i32(const int *__restrict__ in, int count, int *__restrict__ out) {
     __shared__ int part[kBlock / kWave];
     int m = 0;
@@ -103,21 +172,29 @@ __global__ __launch_bounds__(kBlock) void k_max_i32(const int *__restrict__ in, 
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < kBlock / kWave; ++w) m = max(m, part[w]);
-        atomicMax(out, m);
+        out[blockIdx.x] = m;
     }
+}
+
+void max_i32_begin(const int *in, int count, HostInts &h, hipStream_t s) {
+    if (count <= 0) return;
+    const unsigned g = std::min<unsigned>(grid_for(count), (unsigned)kHostInts);
+    k_max_i32<<<g, kBlock, 0, s>>>(in, count, h.out());
+    FL_LAUNCH_CHECK();
+}
+
+int max_i32_end(const HostInts &h) {
+    int m = 0;
+    for (int i = 0; i < kHostInts; ++i) m = std::max(m, h[i]);
+    return m;
 }
 
 int device_max_i32(const int *in, int count, hipStream_t s) {
     if (count <= 0) return 0;
-    DevBuf<int> d(1);
-    FL_HIP(hipMemsetAsync(d.p, 0, sizeof(int), s));
-    const unsigned g = std::min<unsigned>(grid_for(count), 256u);
-    k_max_i32<<<g, kBlock, 0, s>>>(in, count, d.p);
-    FL_LAUNCH_CHECK();
-    int h = 0;
-    FL_HIP(hipMemcpyAsync(&h, d.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    return h;
+    HostInts h(s);
+    max_i32_begin(in, count, h, s);
+    (void)h.wait();
+    return max_i32_end(h);
 }
 
 int bits_for(uint32_t v) {
@@ -240,6 +317,14 @@ __global__ void k_positions(int *__restrict__ v, int count) {
         v[i] = (int)i;
 }
 
+__global__ void k_copy_pairs(const uint32_t *__restrict__ k, const int *__restrict__ v, uint32_t *__restrict__ keys,
+                             int *__restrict__ vals, int count) {
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x) {
+        keys[i] = k[i];
+        vals[i] = v[i];
+    }
+}
+
 static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool positions, hipStream_t s) {
     if (count <= 1 || bits <= 0) {
         if (positions && count > 0) {
@@ -255,13 +340,17 @@ static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool posi
         throw HipError{hipErrorInvalidValue};
     }
     TmpBuf<int> hist((size_t)hcount, s), offs((size_t)hcount + 1, s);
-    TmpBuf<uint32_t> k2(count, s);
-    TmpBuf<int> v2(count, s);
+    const int passes = (bits + kRadixBits - 1) / kRadixBits;
+    // an odd number of passes ends in the caller's arrays by way of a third pair
+    const bool third = passes >= 3 && passes % 2 == 1;
+    TmpBuf<uint32_t> k2(count, s), k3(third ? count : 0, s);
+    TmpBuf<int> v2(count, s), v3(third ? count : 0, s);
     uint32_t *kin = keys, *kout = k2.p;
     int *vin = vals, *vout = v2.p;
-    const int passes = (bits + kRadixBits - 1) / kRadixBits;
     for (int p = 0; p < passes; ++p) {
         const int shift = p * kRadixBits;
+        if (third && p == 1) kout = k3.p, vout = v3.p;
+        if (third && p == 2) kout = keys, vout = vals;
         k_radix_hist<<<nb, kBlock, 0, s>>>(kin, count, shift, nb, hist.p);
         FL_LAUNCH_CHECK();
         exclusive_scan_i32(hist.p, offs.p, (int)hcount, s);
@@ -270,9 +359,9 @@ static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool posi
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
-    if (kin != keys) {
-        FL_HIP(hipMemcpyAsync(keys, kin, sizeof(uint32_t) * count, hipMemcpyDeviceToDevice, s));
-        FL_HIP(hipMemcpyAsync(vals, vin, sizeof(int) * count, hipMemcpyDeviceToDevice, s));
+    if (kin != keys) {  // one pass
+        k_copy_pairs<<<std::min(grid_for(count), 65536u), kBlock, 0, s>>>(kin, vin, keys, vals, count);
+        FL_LAUNCH_CHECK();
     }
     // no wait here: the temporaries are freed in stream order, and the caller's later work on s
     // (or its own readback) comes after the sort

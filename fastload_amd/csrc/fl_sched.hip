@@ -28,7 +28,6 @@
 
 namespace fl {
 
-void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s);
 
 static unsigned sg(long long count) { return std::max(1u, std::min<unsigned>(grid_for(count), 65536u)); }
 
@@ -87,10 +86,6 @@ __global__ void k_batch_sizes(int T, int bt, int nb, int n, const int *__restric
     }
 }
 
-__global__ void k_iota2(int *__restrict__ v, int count) {
-    GRID_STRIDE(i, count) v[i] = (int)i;
-}
-
 __global__ void k_key_gather(const int *__restrict__ src, const int *__restrict__ order, uint32_t *__restrict__ key,
                              int count) {
     GRID_STRIDE(i, count) key[i] = (uint32_t)src[order[i]];
@@ -142,8 +137,11 @@ __global__ void k_win_heads(const uint32_t *__restrict__ kb, const int *__restri
 }
 
 __global__ void k_win_off(const uint32_t *__restrict__ kb, const int *__restrict__ d, int *__restrict__ win_off,
-                          int count) {
-    GRID_STRIDE(i, count) if (i == 0 || kb[i] != kb[i - 1]) win_off[kb[i]] = d[i];
+                          int count, int nb) {
+    GRID_STRIDE(i, count) {
+        if (i == 0 || kb[i] != kb[i - 1]) win_off[kb[i]] = d[i];
+        if (i == 0) win_off[nb] = d[count];
+    }
 }
 
 __global__ void k_win_slot(const uint32_t *__restrict__ kb, const int *__restrict__ order, const int *__restrict__ row,
@@ -170,9 +168,16 @@ __global__ void k_pb_dest(const int *__restrict__ orderA, const int *__restrict_
 }
 
 // chunk_off[c] = first band-major position of chunk c, rounded down to a multiple of 4 (keeps
-// the 16-byte alignment of phase 2's vector loads in the reused product array)
-__global__ void k_chunk_off(const int *__restrict__ band_start, int nbands, int C, int *__restrict__ chunk_off) {
-    GRID_STRIDE(c, C) chunk_off[c] = band_start[(size_t)c * nbands] & ~3;
+// the 16-byte alignment of phase 2's vector loads in the reused product array); the same and the C + 1
+// starts to the host (one workgroup)
+constexpr int kMaxChunks = 2;
+__global__ void k_chunk_off(const int *__restrict__ band_start, int nbands, int C, int *__restrict__ chunk_off,
+                            int *__restrict__ host_off, int *__restrict__ host_start) {
+    GRID_STRIDE(c, (long long)C + 1) {
+        const int b = band_start[(size_t)c * nbands];
+        host_start[c] = b;
+        if (c < C) chunk_off[c] = host_off[c] = b & ~3;
+    }
 }
 
 // start[b] = first position of key b in the sorted keys (lower bound); start[nb] = count.
@@ -211,8 +216,13 @@ __global__ void k_pb_runs(const uint32_t *__restrict__ kb, const int *__restrict
     }
 }
 
-__global__ void k_run_len(const int *__restrict__ run_pos, int nruns, int total, int *__restrict__ run_len) {
-    GRID_STRIDE(r, nruns) run_len[r] = ((r + 1 < nruns) ? run_pos[r + 1] : total) - run_pos[r];
+// and the end of the last batch's runs
+__global__ void k_run_len(const int *__restrict__ run_pos, int nruns, int total, int *__restrict__ run_len,
+                          int *__restrict__ run_end) {
+    GRID_STRIDE(r, nruns) {
+        run_len[r] = ((r + 1 < nruns) ? run_pos[r + 1] : total) - run_pos[r];
+        if (r == 0) *run_end = nruns;
+    }
 }
 
 __global__ void k_adjdiff(const int *__restrict__ in, int count, int *__restrict__ out) {
@@ -220,18 +230,19 @@ __global__ void k_adjdiff(const int *__restrict__ in, int count, int *__restrict
 }
 
 // Every entry's destination must be its run's destination plus its offset inside the run (the
-// phase-1 copy moves whole runs).
+// phase-1 copy moves whole runs). flag: as for the validators below.
 __global__ void k_check_runs(const int *__restrict__ orderB, const int *__restrict__ head,
                              const int *__restrict__ runidx, const int *__restrict__ run_pos,
                              const int *__restrict__ run_dest, const int *__restrict__ dest, int count,
                              int *__restrict__ flag) {
     GRID_STRIDE(i, count) {
         const int r = runidx[i] + head[i] - 1;
-        if (dest[orderB[i]] != run_dest[r] + ((int)i - run_pos[r])) atomicOr(flag, 16);
+        if (dest[orderB[i]] != run_dest[r] + ((int)i - run_pos[r])) *flag = 1;
     }
 }
 
-// Validators: every index the kernels will use must be inside the buffers they assume.
+// Validators: every index the kernels will use must be inside the buffers they assume. flag is in host memory,
+// written only when something is wrong.
 __global__ void k_check_win(const int *__restrict__ batch_of, const uint16_t *__restrict__ slot,
                             const int *__restrict__ win_off, int cap, int nnz, int m,
                             const int *__restrict__ win_rows, int *__restrict__ flag) {
@@ -239,11 +250,11 @@ __global__ void k_check_win(const int *__restrict__ batch_of, const uint16_t *__
         const int b = batch_of[g];
         const int ns = win_off[b + 1] - win_off[b];
         if (ns <= 0 || ns > cap || (int)slot[g] >= ns) {
-            atomicOr(flag, 1);
+            *flag = 1;
             continue;
         }
         const int r = win_rows[win_off[b] + slot[g]] & 0x7fffffff;  // high bit: row shared with other batches
-        if (r >= m) atomicOr(flag, 2);
+        if (r >= m) *flag = 1;
     }
 }
 
@@ -255,7 +266,7 @@ __global__ void k_check_pb(const int *__restrict__ batch_of, const uint16_t *__r
     GRID_STRIDE(g, nnz) {
         const int b = batch_of[g];
         const int bsize = batch_start[b + 1] - batch_start[b];
-        if (bsize > cap || (int)lslot[g] >= bsize) atomicOr(flag, 4);
+        if (bsize > cap || (int)lslot[g] >= bsize) *flag = 1;
     }
     GRID_STRIDE(t, (long long)nb * 64) {  // a wave per batch
         const long long b = t >> 6;
@@ -263,20 +274,8 @@ __global__ void k_check_pb(const int *__restrict__ batch_of, const uint16_t *__r
         for (int r = run_off[b] + (int)(t & 63); r < run_off[b + 1]; r += 64)
             if (run_len[r] <= 0 || run_lstart[r] < 0 || run_lstart[r] + run_len[r] > bsize || run_dest[r] < 0 ||
                 run_dest[r] + run_len[r] > ring)
-                atomicOr(flag, 8);
+                *flag = 1;
     }
-}
-
-static int read1(const int *d, hipStream_t s) {
-    int h = 0;
-    FL_HIP(hipMemcpyAsync(&h, d, sizeof(int), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    return h;
-}
-
-static void write1(int *d, int v, hipStream_t s) {
-    FL_HIP(hipMemcpyAsync(d, &v, sizeof(int), hipMemcpyHostToDevice, s));
-    FL_HIP(hipStreamSynchronize(s));
 }
 
 static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
@@ -293,14 +292,12 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
             TmpBuf<int> order(T, s);
             if (kind == 1) k_tile_rowkey<<<sg(T), kBlock, 0, s>>>(A->tile_ptr.p, A->sortrowidx.p, T, key.p);
             else k_tile_bucket<<<sg(T), kBlock, 0, s>>>(A->tile_colidx.p, T, key.p);
-            k_iota2<<<sg(T), kBlock, 0, s>>>(order.p, T);
             FL_LAUNCH_CHECK();
             const int top = kind == 1 ? (A->m - 1) >> 6 : (A->n - 1) >> 8;
-            radix_sort_pairs(key.p, order.p, T, bits_for((uint32_t)std::max(top, 0)), s);
+            radix_sort_positions(key.p, order.p, T, bits_for((uint32_t)std::max(top, 0)), s);
             k_tile_reorder<<<sg(T), kBlock, 0, s>>>(order.p, A->tile_ptr.p, A->tile_colidx.p, T, A->ord_ptr.p,
                                                     A->ord_cx.p);
             FL_LAUNCH_CHECK();
-            FL_HIP(hipStreamSynchronize(s));
         }
     }
     if (A->bt == bt && A->batch_of.p) return;
@@ -318,7 +315,6 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
         FL_LAUNCH_CHECK();
     }
     exclusive_scan_i32(sizes.p, A->batch_start.p, A->nbatches, s);
-    FL_HIP(hipStreamSynchronize(s));
 }
 
 void pack_schedules(fl_matrix *A, hipStream_t s);
@@ -341,29 +337,26 @@ void win_prepare(fl_matrix *A, int bt, bool rows, hipStream_t s) {
     TmpBuf<int> order(nnz, s), head(nnz, s), d((size_t)nnz + 1, s);
     // (row, g) order, then stable by batch -> (batch, row, g)
     k_key_copy<<<sg(nnz), kBlock, 0, s>>>(A->sortrowidx.p, key.p, nnz, 1);
-    k_iota2<<<sg(nnz), kBlock, 0, s>>>(order.p, nnz);
     FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
     k_key_gather<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, order.p, key.p, nnz);
     FL_LAUNCH_CHECK();
     radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(nb - 1, 0)), s);
     k_win_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, nnz);
     FL_LAUNCH_CHECK();
-    exclusive_scan_i32(head.p, d.p, nnz, s);
-    const int D = read1(d.p + nnz, s);
+    HostInts h(s);  // distinct rows; out-of-range slots
+    exclusive_scan_i32(head.p, d.p, nnz, s, h.out(0));
+    const int D = h.wait()[0];
     A->win_rows.alloc(std::max(D, 1));
-    k_win_off<<<sg(nnz), kBlock, 0, s>>>(key.p, d.p, A->win_off.p, nnz);
+    k_win_off<<<sg(nnz), kBlock, 0, s>>>(key.p, d.p, A->win_off.p, nnz, nb);
     FL_LAUNCH_CHECK();
-    write1(A->win_off.p + nb, D, s);
     k_win_slot<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, d.p, A->win_off.p, A->win_slot.p,
                                           A->win_rows.p, nnz);
     FL_LAUNCH_CHECK();
-    TmpBuf<int> flag(1, s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
     k_check_win<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->win_slot.p, A->win_off.p, bt * 64, nnz, A->m,
-                                           A->win_rows.p, flag.p);
+                                           A->win_rows.p, h.out(1));
     FL_LAUNCH_CHECK();
-    if (read1(flag.p, s)) {
+    if (h.wait()[1]) {
         set_error("WIN schedule: preprocessing produced out-of-range slots");
         throw HipError{hipErrorInvalidValue};
     }
@@ -373,7 +366,6 @@ void win_prepare(fl_matrix *A, int bt, bool rows, hipStream_t s) {
         k_row_batches<<<sg(D), kBlock, 0, s>>>(A->win_rows.p, D, cnt.p);
         k_mark_shared<<<sg(D), kBlock, 0, s>>>(A->win_rows.p, D, cnt.p);
         FL_LAUNCH_CHECK();
-        FL_HIP(hipStreamSynchronize(s));
     }
     TmpBuf<int> per_batch(nb, s);
     k_adjdiff<<<sg(nb), kBlock, 0, s>>>(A->win_off.p, nb, per_batch.p);
@@ -448,7 +440,7 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     // is small next to them (every chunk after the first re-reads and re-writes y). On the
     // 67 M-entry power-law matrix two chunks are 7 % faster than one; three or more are slower
     // (each chunk adds a pass over y and two launch tails).
-    const int want = (nnz >= (1 << 25) && (long long)m * 8 <= nnz) ? 2 : 1;
+    const int want = (nnz >= (1 << 25) && (long long)m * 8 <= nnz) ? kMaxChunks : 1;
     const std::vector<int> cb = pb_chunk_batches(A, want, s);
     const int C = (int)cb.size() - 1;
     if ((long long)C * nbands > 0x7fffffffLL) {
@@ -465,34 +457,33 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     // range of the product array
     const int per_xcd = (nb + 7) / 8;
     k_key_batch_xcd<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, per_xcd, key.p, nnz);
-    k_iota2<<<sg(nnz), kBlock, 0, s>>>(order.p, nnz);
     FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
     k_key_chunk_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, order.p, R, nbands, d_cb.p, C, key.p,
                                                 nnz);
     FL_LAUNCH_CHECK();
     radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)(C * nbands - 1)), s);
     k_key_bounds<<<sg((long long)C * nbands + 1), kBlock, 0, s>>>(key.p, nnz, C * nbands, A->pb_band_start.p);
-    k_chunk_off<<<sg(C), kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p);
+    HostInts h(s);  // runs; bad runs or slots; the chunks' offsets and starts
+    static_assert(2 + 2 * kMaxChunks + 1 <= kHostInts, "chunk offsets fit the host block");
+    k_chunk_off<<<1, kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p, h.out(2), h.out(2 + C));
     k_pb_dest<<<sg(nnz), kBlock, 0, s>>>(order.p, A->sortrowidx.p, R, key.p, nbands, d_off.p, dest.p,
                                          A->pb_rowlocal.p, nnz);
     FL_LAUNCH_CHECK();
-    std::vector<int> off(C), cstart((size_t)C + 1);
-    FL_HIP(hipMemcpyAsync(off.data(), d_off.p, sizeof(int) * C, hipMemcpyDeviceToHost, s));
-    FL_HIP(hipStreamSynchronize(s));
-    int ring = 0;
-    for (int c = 0; c <= C; ++c) cstart[c] = read1(A->pb_band_start.p + (size_t)c * nbands, s);
-    for (int c = 0; c < C; ++c) ring = std::max(ring, cstart[c + 1] - off[c]);
     // B: (batch, band, g) order -> LDS staging slots and runs
     k_key_batch_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, R, nbands, key.p, nnz);
-    k_iota2<<<sg(nnz), kBlock, 0, s>>>(order.p, nnz);
     FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)(nb * nbands - 1)), s);
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)(nb * nbands - 1)), s);
     k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, head.p, nnz);
     FL_LAUNCH_CHECK();
-    exclusive_scan_i32(head.p, runidx.p, nnz, s);
-    const int nruns = read1(runidx.p + nnz, s);
+    exclusive_scan_i32(head.p, runidx.p, nnz, s, h.out(0));
+    const int nruns = h.wait()[0];
     A->nruns = nruns;
+    std::vector<int> off(C), cstart((size_t)C + 1);
+    int ring = 0;
+    for (int c = 0; c < C; ++c) off[c] = h[2 + c];
+    for (int c = 0; c <= C; ++c) cstart[c] = h[2 + C + c];
+    for (int c = 0; c < C; ++c) ring = std::max(ring, cstart[c + 1] - off[c]);
     A->pb_run_lstart.alloc(nruns);
     A->pb_run_dest.alloc(nruns);
     A->pb_run_len.alloc(nruns);
@@ -500,18 +491,15 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, head.p, runidx.p, dest.p, A->batch_start.p, nbands,
                                          A->pb_lslot.p, A->pb_run_lstart.p, A->pb_run_dest.p, run_pos.p,
                                          A->pb_run_off.p, nnz);
-    k_run_len<<<sg(nruns), kBlock, 0, s>>>(run_pos.p, nruns, nnz, A->pb_run_len.p);
+    k_run_len<<<sg(nruns), kBlock, 0, s>>>(run_pos.p, nruns, nnz, A->pb_run_len.p, A->pb_run_off.p + nb);
     FL_LAUNCH_CHECK();
-    write1(A->pb_run_off.p + nb, nruns, s);
-    TmpBuf<int> flag(1, s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
     k_check_pb<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->pb_lslot.p, A->batch_start.p, A->bt * 64, nnz, ring,
                                           A->pb_run_off.p, A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p, nb,
-                                          flag.p);
+                                          h.out(1));
     k_check_runs<<<sg(nnz), kBlock, 0, s>>>(order.p, head.p, runidx.p, run_pos.p, A->pb_run_dest.p, dest.p, nnz,
-                                            flag.p);
+                                            h.out(1));
     FL_LAUNCH_CHECK();
-    if (read1(flag.p, s) || cstart[C] != nnz || ring > nnz) {
+    if (h.wait()[1] || cstart[C] != nnz || ring > nnz) {
         set_error("PB schedule: preprocessing produced out-of-range runs or slots");
         throw HipError{hipErrorInvalidValue};
     }
@@ -632,7 +620,6 @@ void pack_schedules(fl_matrix *A, hipStream_t s) {
             A->pb_pf = f;
         }
     }
-    FL_HIP(hipStreamSynchronize(s));
 }
 
 // ----------------------------------------------------------- schedules read back from a file
@@ -670,13 +657,12 @@ int win_install(fl_matrix *A, int bt, bool rows, int nb_file, const uint16_t *sl
     upload_to(A->win_slot, slot, nnz, s);
     upload_to(A->win_rows, win_rows, (size_t)D, s);
     upload_to(A->win_off, off, (size_t)nb + 1, s);
-    TmpBuf<int> flag(1, s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
+    HostInts bad(s);
     if (nnz)
         k_check_win<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->win_slot.p, A->win_off.p, bt * 64, nnz, A->m,
-                                               A->win_rows.p, flag.p);
+                                               A->win_rows.p, bad.out());
     FL_LAUNCH_CHECK();
-    if (read1(flag.p, s)) {
+    if (bad.wait()[0]) {
         A->win_slot.release();
         A->win_rows.release();
         A->win_off.release();
@@ -721,14 +707,13 @@ int pb_install(fl_matrix *A, int bt, int R, int nb_file, int C, const int *chunk
     upload_to(A->pb_run_lstart, run_lstart, (size_t)nruns, s);
     upload_to(A->pb_run_dest, run_dest, (size_t)nruns, s);
     upload_to(A->pb_run_len, run_len, (size_t)nruns, s);
-    TmpBuf<int> flag(1, s);
-    FL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), s));
+    HostInts bad(s);
     if (nnz)
         k_check_pb<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->pb_lslot.p, A->batch_start.p, bt * 64, nnz, (int)ring,
                                               A->pb_run_off.p, A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p,
-                                              nb, flag.p);
+                                              nb, bad.out());
     FL_LAUNCH_CHECK();
-    if (read1(flag.p, s)) {
+    if (bad.wait()[0]) {
         A->pb_ready = false;
         return bad_file("PB schedule: staging slots or runs out of range");
     }

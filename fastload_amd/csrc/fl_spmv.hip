@@ -320,7 +320,6 @@ void prepare_values(fl_matrix *A, int kind, hipStream_t s) {
         FL_LAUNCH_CHECK();
     }
     if (A->hyb_light) hyb_values(A, kind, s);
-    FL_HIP(hipStreamSynchronize(s));
 }
 
 void permute_raw(const int *perm, int n, const void *x, void *sx, bool dbl, hipStream_t s) {
