@@ -79,8 +79,8 @@ __global__ void k_feat_rowcount(const int *__restrict__ rowidx, int nnz, int *__
 
 // Entries per row from row indices grouped by row >> shift (start: 257 group bounds). A workgroup counts
 // kFeatChunk consecutive indices, group by group, in LDS (1 << shift counters) and adds what it has
-// seen of a group to rc. Global atomics on random rows run at about 28 G/s (10 M entries, 600 K rows:
-// 350 us); grouped (radix_partition, 65 us) and counted here (22 us) it is LDS work, and the adds to
+// seen of a group to rc. Global atomics on random rows run at about 28 G/s (8.8 M entries, 600 K rows:
+// 310 us); grouped (radix_partition, 69 us) and counted here (22 us) it is LDS work, and the adds to
 // rc are coalesced.
 constexpr int kFeatChunk = 1 << 16, kFeatMaxShift = 15;
 __global__ __launch_bounds__(1024) void k_feat_rowcount_bins(const uint32_t *__restrict__ rows, int nnz, int shift,
