@@ -121,11 +121,6 @@ __global__ void k_key_chunk_band(const int *__restrict__ batch_of, const int *__
     }
 }
 
-__global__ void k_key_batch_band(const int *__restrict__ batch_of, const int *__restrict__ row, int R, int nbands,
-                                 uint32_t *__restrict__ key, int count) {
-    GRID_STRIDE(i, count) key[i] = (uint32_t)batch_of[i] * (uint32_t)nbands + (uint32_t)(row[i] / R);
-}
-
 // WIN: heads of (batch, row) runs in (batch, row, g) order
 __global__ void k_win_heads(const uint32_t *__restrict__ kb, const int *__restrict__ order, const int *__restrict__ row,
                             int *__restrict__ head, int count) {
@@ -155,15 +150,66 @@ __global__ void k_win_slot(const uint32_t *__restrict__ kb, const int *__restric
     }
 }
 
-// PB: dest[g] = product-array position (band-major position minus its chunk's offset);
-// rowlocal[pos] = row - band*R at the band-major position
-__global__ void k_pb_dest(const int *__restrict__ orderA, const int *__restrict__ row, int R,
-                          const uint32_t *__restrict__ key, int nbands, const int *__restrict__ chunk_off,
-                          int *__restrict__ dest, uint16_t *__restrict__ rowlocal, int count) {
+// PB, entries in (chunk, band, batch, g) order: a run is one batch's entries of one band. head[i] = 1 where one
+// starts; rowlocal[i] = the entry's row inside its band.
+__global__ void k_pb_heads(const uint32_t *__restrict__ key, const int *__restrict__ order,
+                           const int *__restrict__ batch_of, const int *__restrict__ row, int R,
+                           int *__restrict__ head, uint16_t *__restrict__ rowlocal, int count) {
     GRID_STRIDE(i, count) {
-        const int g = orderA[i];
-        dest[g] = (int)i - chunk_off[key[i] / (uint32_t)nbands];
+        const int g = order[i];
+        head[i] = i == 0 || key[i] != key[i - 1] || batch_of[g] != batch_of[order[i - 1]];
         rowlocal[i] = (uint16_t)(row[g] % R);
+    }
+}
+
+// first entry of every run, and its (batch, band)
+__global__ void k_pb_runs(const int *__restrict__ head, const int *__restrict__ runidx,
+                          const uint32_t *__restrict__ key, const int *__restrict__ order,
+                          const int *__restrict__ batch_of, int nbands, int *__restrict__ run_pos,
+                          uint32_t *__restrict__ run_key, int count) {
+    GRID_STRIDE(i, count) {
+        if (!head[i]) continue;
+        const int r = runidx[i];
+        run_pos[r] = (int)i;
+        run_key[r] = (uint32_t)batch_of[order[i]] * (uint32_t)nbands + key[i] % (uint32_t)nbands;
+    }
+}
+
+// lengths of the runs in (batch, band) order (by: the k-th run in that order)
+__global__ void k_pb_run_len(const int *__restrict__ by, const int *__restrict__ run_pos, int nruns, int total,
+                             int *__restrict__ run_len) {
+    GRID_STRIDE(k, nruns) {
+        const int r = by[k];
+        run_len[k] = (r + 1 < nruns ? run_pos[r + 1] : total) - run_pos[r];
+    }
+}
+
+// The k-th run's place in its batch's staging area (start: entries of the runs before it; also by run, for
+// k_pb_slots) and in the product array, and the first run of every batch.
+__global__ void k_pb_run_place(const uint32_t *__restrict__ key, const int *__restrict__ by,
+                               const int *__restrict__ run_pos, const int *__restrict__ start,
+                               const int *__restrict__ batch_start, const int *__restrict__ chunk_batch, int C,
+                               const int *__restrict__ chunk_off, int nbands, int nruns, int nb,
+                               int *__restrict__ run_lstart, int *__restrict__ run_dest, int *__restrict__ run_off,
+                               int *__restrict__ lstart_of) {
+    GRID_STRIDE(k, nruns) {
+        const int r = by[k], batch = (int)(key[k] / (uint32_t)nbands);
+        int c = 0;
+        while (c + 1 < C && batch >= chunk_batch[c + 1]) ++c;
+        const int ls = start[k] - batch_start[batch];
+        run_lstart[k] = lstart_of[r] = ls;
+        run_dest[k] = run_pos[r] - chunk_off[c];
+        if (k == 0 || batch != (int)(key[k - 1] / (uint32_t)nbands)) run_off[batch] = (int)k;
+        if (k == 0) run_off[nb] = nruns;
+    }
+}
+
+__global__ void k_pb_slots(const int *__restrict__ head, const int *__restrict__ runidx,
+                           const int *__restrict__ order, const int *__restrict__ run_pos,
+                           const int *__restrict__ lstart_of, uint16_t *__restrict__ lslot, int count) {
+    GRID_STRIDE(i, count) {
+        const int r = runidx[i] + head[i] - 1;
+        lslot[order[i]] = (uint16_t)(lstart_of[r] + (int)i - run_pos[r]);
     }
 }
 
@@ -192,53 +238,8 @@ __global__ void k_key_bounds(const uint32_t *__restrict__ k, int count, int nb, 
     }
 }
 
-__global__ void k_pb_heads(const uint32_t *__restrict__ kb, int *__restrict__ head, int count) {
-    GRID_STRIDE(i, count) head[i] = (i == 0) || (kb[i] != kb[i - 1]);
-}
-
-__global__ void k_pb_runs(const uint32_t *__restrict__ kb, const int *__restrict__ orderB, const int *__restrict__ head,
-                          const int *__restrict__ runidx, const int *__restrict__ dest,
-                          const int *__restrict__ batch_start, int nbands, uint16_t *__restrict__ lslot,
-                          int *__restrict__ run_lstart, int *__restrict__ run_dest, int *__restrict__ run_pos,
-                          int *__restrict__ run_off, int count) {
-    GRID_STRIDE(i, count) {
-        const int batch = (int)(kb[i] / (uint32_t)nbands);
-        const int bstart = batch_start[batch];
-        const int g = orderB[i];
-        lslot[g] = (uint16_t)(i - bstart);
-        if (head[i]) {
-            const int r = runidx[i];
-            run_lstart[r] = (int)i - bstart;
-            run_dest[r] = dest[g];
-            run_pos[r] = (int)i;
-            if (i == 0 || kb[i] / (uint32_t)nbands != kb[i - 1] / (uint32_t)nbands) run_off[batch] = r;
-        }
-    }
-}
-
-// and the end of the last batch's runs
-__global__ void k_run_len(const int *__restrict__ run_pos, int nruns, int total, int *__restrict__ run_len,
-                          int *__restrict__ run_end) {
-    GRID_STRIDE(r, nruns) {
-        run_len[r] = ((r + 1 < nruns) ? run_pos[r + 1] : total) - run_pos[r];
-        if (r == 0) *run_end = nruns;
-    }
-}
-
 __global__ void k_adjdiff(const int *__restrict__ in, int count, int *__restrict__ out) {
     GRID_STRIDE(i, count) out[i] = in[i + 1] - in[i];
-}
-
-// Every entry's destination must be its run's destination plus its offset inside the run (the
-// phase-1 copy moves whole runs). flag: as for the validators below.
-__global__ void k_check_runs(const int *__restrict__ orderB, const int *__restrict__ head,
-                             const int *__restrict__ runidx, const int *__restrict__ run_pos,
-                             const int *__restrict__ run_dest, const int *__restrict__ dest, int count,
-                             int *__restrict__ flag) {
-    GRID_STRIDE(i, count) {
-        const int r = runidx[i] + head[i] - 1;
-        if (dest[orderB[i]] != run_dest[r] + ((int)i - run_pos[r])) *flag = 1;
-    }
 }
 
 // Validators: every index the kernels will use must be inside the buffers they assume. flag is in host memory,
@@ -451,8 +452,8 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     TmpBuf<int> d_cb(cb.size(), s), d_off(C, s);
     FL_HIP(hipMemcpyAsync(d_cb.p, cb.data(), sizeof(int) * cb.size(), hipMemcpyHostToDevice, s));
     TmpBuf<uint32_t> key(nnz, s);
-    TmpBuf<int> order(nnz, s), dest(nnz, s), head(nnz, s), runidx((size_t)nnz + 1, s);
-    // A: chunk-major, then band-major order (chunk, band, batch, g): stable by batch (batches in
+    TmpBuf<int> order(nnz, s), head(nnz, s), runidx((size_t)nnz + 1, s);
+    // chunk-major, then band-major order (chunk, band, batch, g): stable by batch (batches in
     // XCD order), then stable by (chunk, band), so each (batch, band) run occupies one contiguous
     // range of the product array
     const int per_xcd = (nb + 7) / 8;
@@ -467,14 +468,8 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     HostInts h(s);  // runs; bad runs or slots; the chunks' offsets and starts
     static_assert(2 + 2 * kMaxChunks + 1 <= kHostInts, "chunk offsets fit the host block");
     k_chunk_off<<<1, kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p, h.out(2), h.out(2 + C));
-    k_pb_dest<<<sg(nnz), kBlock, 0, s>>>(order.p, A->sortrowidx.p, R, key.p, nbands, d_off.p, dest.p,
-                                         A->pb_rowlocal.p, nnz);
-    FL_LAUNCH_CHECK();
-    // B: (batch, band, g) order -> LDS staging slots and runs
-    k_key_batch_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, R, nbands, key.p, nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)(nb * nbands - 1)), s);
-    k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, head.p, nnz);
+    k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->batch_of.p, A->sortrowidx.p, R, head.p,
+                                          A->pb_rowlocal.p, nnz);
     FL_LAUNCH_CHECK();
     exclusive_scan_i32(head.p, runidx.p, nnz, s, h.out(0));
     const int nruns = h.wait()[0];
@@ -484,20 +479,29 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     for (int c = 0; c < C; ++c) off[c] = h[2 + c];
     for (int c = 0; c <= C; ++c) cstart[c] = h[2 + C + c];
     for (int c = 0; c < C; ++c) ring = std::max(ring, cstart[c + 1] - off[c]);
+    // The runs by (batch, band), and with their lengths the entries' staging slots. There are 20 to 60 times
+    // fewer runs than entries, and inside a run both orders are the same, so only the runs are sorted again.
+    // (Sorting the entries again was up to four passes over all of them and three gathers: the preparation of
+    // 18 M uniform entries 1,556 us, so 1,121; 9.6 M power-law entries 909 and 709; 1.8 M 289 and 289.)
     A->pb_run_lstart.alloc(nruns);
     A->pb_run_dest.alloc(nruns);
     A->pb_run_len.alloc(nruns);
-    TmpBuf<int> run_pos(nruns, s);
-    k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, head.p, runidx.p, dest.p, A->batch_start.p, nbands,
-                                         A->pb_lslot.p, A->pb_run_lstart.p, A->pb_run_dest.p, run_pos.p,
-                                         A->pb_run_off.p, nnz);
-    k_run_len<<<sg(nruns), kBlock, 0, s>>>(run_pos.p, nruns, nnz, A->pb_run_len.p, A->pb_run_off.p + nb);
+    TmpBuf<int> run_pos(nruns, s), by(nruns, s), start((size_t)nruns + 1, s), lstart_of(nruns, s);
+    TmpBuf<uint32_t> run_key(nruns, s);
+    k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, key.p, order.p, A->batch_of.p, nbands, run_pos.p, run_key.p,
+                                         nnz);
     FL_LAUNCH_CHECK();
+    radix_sort_positions(run_key.p, by.p, nruns, bits_for((uint32_t)(nb * nbands - 1)), s);
+    k_pb_run_len<<<sg(nruns), kBlock, 0, s>>>(by.p, run_pos.p, nruns, nnz, A->pb_run_len.p);
+    FL_LAUNCH_CHECK();
+    exclusive_scan_i32(A->pb_run_len.p, start.p, nruns, s);
+    k_pb_run_place<<<sg(nruns), kBlock, 0, s>>>(run_key.p, by.p, run_pos.p, start.p, A->batch_start.p, d_cb.p, C,
+                                                d_off.p, nbands, nruns, nb, A->pb_run_lstart.p, A->pb_run_dest.p,
+                                                A->pb_run_off.p, lstart_of.p);
+    k_pb_slots<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, order.p, run_pos.p, lstart_of.p, A->pb_lslot.p, nnz);
     k_check_pb<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->pb_lslot.p, A->batch_start.p, A->bt * 64, nnz, ring,
                                           A->pb_run_off.p, A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p, nb,
                                           h.out(1));
-    k_check_runs<<<sg(nnz), kBlock, 0, s>>>(order.p, head.p, runidx.p, run_pos.p, A->pb_run_dest.p, dest.p, nnz,
-                                            h.out(1));
     FL_LAUNCH_CHECK();
     if (h.wait()[1] || cstart[C] != nnz || ring > nnz) {
         set_error("PB schedule: preprocessing produced out-of-range runs or slots");
