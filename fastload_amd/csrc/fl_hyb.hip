@@ -57,35 +57,100 @@ __global__ void k_hyb_bounds(const uint32_t *__restrict__ key, int count, int nb
     }
 }
 
-__global__ void k_hyb_lenkey(const int *__restrict__ hptr, int m, uint32_t *__restrict__ key, int *__restrict__ rows) {
-    HSTRIDE(r, m) {
-        key[r] = 65535u - (uint32_t)(hptr[r + 1] - hptr[r]);
-        rows[r] = (int)r;
+// Rows by (window, heavy count descending, row), and the pair rows of every slice (half its first, longest
+// row, rounded up). One workgroup per window: a stable radix sort of the counts in LDS, 8 bits at a time, the
+// second pass only where a row has 256 heavy entries or more. Each wave ranks a contiguous part of the rows, as in
+// the radix sort of the whole device; one sort of all rows there, by count and then by window, was
+// 17 launches and 75 us for 600 K rows, this is one of 9 us.
+constexpr int kOrderThreads = 1024, kOrderWaves = kOrderThreads / 64;
+constexpr int kOrderRounds = 16;  // of 64 rows per wave: windows of up to 16,384 rows
+__global__ __launch_bounds__(kOrderThreads) void k_hyb_order(const int *__restrict__ hptr, int m, int win, int rounds,
+                                                             int *__restrict__ rows, uint16_t *__restrict__ iperm,
+                                                             uint16_t *__restrict__ perm, int *__restrict__ np,
+                                                             int *__restrict__ pairs) {
+    extern __shared__ double order_lds[];
+    const int cap = rounds * kOrderThreads;
+    uint16_t *ka = reinterpret_cast<uint16_t *>(order_lds), *ia = ka + cap, *kb = ia + cap, *ib = kb + cap;
+    int(*wcnt)[256] = reinterpret_cast<int(*)[256]>(ib + cap);  // a wave's rows per digit, then where they go
+    __shared__ int wsum[4];
+    const int base = (int)blockIdx.x * win, n = min(win, m - base);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int big = 0;
+    for (int i = threadIdx.x; i < n; i += kOrderThreads) {
+        const int c = hptr[base + i + 1] - hptr[base + i];
+        big |= c >= 256;
+        ka[i] = (uint16_t)(65535 - c);
+        ia[i] = (uint16_t)i;
     }
-}
-
-__global__ void k_hyb_winkey(const int *__restrict__ rows, int m, int win, uint32_t *__restrict__ key) {
-    HSTRIDE(p, m) key[p] = (uint32_t)(rows[p] / win);
-}
-
-__global__ void k_hyb_pos(const int *__restrict__ rows, int m, int win, uint16_t *__restrict__ iperm,
-                          uint16_t *__restrict__ perm, int *__restrict__ flag) {
-    HSTRIDE(p, m) {
-        const int r = rows[p], w0 = r / win * win;
-        iperm[r] = (uint16_t)(p - w0);
-        perm[p] = (uint16_t)(r - w0);
-        if (p < w0 || p - w0 >= win) *flag = 1;  // a row left its window
+    const int passes = __syncthreads_or(big) ? 2 : 1;
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    for (int p = 0; p < passes; ++p) {
+        const int shift = 8 * p;
+        for (int i = threadIdx.x; i < kOrderWaves * 256; i += kOrderThreads) wcnt[i >> 8][i & 255] = 0;
+        __syncthreads();
+        int at[kOrderRounds];  // rank among the wave's rows of the same digit
+#pragma unroll
+        for (int r = 0; r < kOrderRounds; ++r) {
+            if (r >= rounds) break;
+            const int i = (w * rounds + r) * 64 + lane;
+            const bool valid = i < n;
+            const int d = valid ? (ka[i] >> shift) & 255 : 0;
+            uint64_t peers = ballot64(valid);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const bool bit = (d >> k) & 1;
+                const uint64_t b = ballot64(bit);
+                peers &= bit ? b : ~b;
+            }
+            const int rank = __popcll(peers & lt_mask);
+            int o = 0;
+            if (valid && rank == 0) o = atomicAdd(&wcnt[w][d], __popcll(peers));
+            at[r] = __shfl(o, valid ? __ffsll((unsigned long long)peers) - 1 : lane, 64) + rank;
+        }
+        __syncthreads();
+        // where each wave's rows of a digit start
+        int sum = 0, v = 0;
+        if (w < 4) {
+            for (int q = 0; q < kOrderWaves; ++q) sum += wcnt[q][threadIdx.x];
+            v = wave_inclusive_scan(sum);
+            if (lane == 63) wsum[w] = v;
+        }
+        __syncthreads();
+        if (w < 4) {
+            int before = v - sum;
+            for (int q = 0; q < w; ++q) before += wsum[q];
+            for (int q = 0; q < kOrderWaves; ++q) {
+                const int t = wcnt[q][threadIdx.x];
+                wcnt[q][threadIdx.x] = before;
+                before += t;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kOrderRounds; ++r) {
+            if (r >= rounds) break;
+            const int i = (w * rounds + r) * 64 + lane;
+            if (i < n) {
+                const int pos = wcnt[w][(ka[i] >> shift) & 255] + at[r];
+                kb[pos] = ka[i];
+                ib[pos] = ia[i];
+            }
+        }
+        __syncthreads();
+        uint16_t *t = ka;
+        ka = kb, kb = t;
+        t = ia, ia = ib, ib = t;
     }
-}
-
-// pair rows of every slice: half the longest row, rounded up (the first lane's: longest first)
-__global__ void k_hyb_pairs(const int *__restrict__ rows, const int *__restrict__ hptr, int m, int nslice,
-                            int *__restrict__ np, int *__restrict__ slots) {
-    HSTRIDE(s, nslice) {
-        const int r = rows[s * 64];
-        const int p = (hptr[r + 1] - hptr[r] + 1) / 2;
-        np[s] = p;
-        slots[s] = p;
+    for (int p = threadIdx.x; p < n; p += kOrderThreads) {
+        const int r = ia[p];
+        rows[base + p] = base + r;
+        perm[base + p] = (uint16_t)r;
+        iperm[base + r] = (uint16_t)p;
+        if ((p & 63) == 0) {
+            const int q = (65535 - ka[p] + 1) / 2;
+            np[(base + p) / 64] = q;
+            pairs[(base + p) / 64] = q;
+        }
     }
 }
 
@@ -94,7 +159,8 @@ __global__ void k_hyb_pairs(const int *__restrict__ rows, const int *__restrict_
 // gathers of the entries, one line each; two pair rows at a time keep four in flight per lane.
 __global__ void k_hyb_fill(int m, int nslice, int H, const int *__restrict__ rows, const int *__restrict__ np,
                            const long long *__restrict__ sb, const int *__restrict__ hptr, const int *__restrict__ ridx,
-                           const ColEntry *__restrict__ ents, uint32_t *__restrict__ col2, double2 *__restrict__ val2) {
+                           const ColEntry *__restrict__ ents, uint32_t *__restrict__ col2, double2 *__restrict__ val2,
+                           float2 *__restrict__ val2f) {
     // one position per thread; consecutive workgroups of an XCD take consecutive slices, so the lines of the
     // entries that a sorting window's rows share are fetched once (7.4 M heavy entries: 195 us with the slices dealt round-robin, 148 so; the three
     // dependent reads per entry before that took 545)
@@ -125,6 +191,7 @@ __global__ void k_hyb_fill(int m, int nslice, int H, const int *__restrict__ row
                 const long long slot = sb[s] + 64LL * (q + h) + lane;
                 col2[slot] = (uint32_t)e[2 * h].col | ((uint32_t)e[2 * h + 1].col << 16);
                 val2[slot] = make_double2(e[2 * h].val, e[2 * h + 1].val);
+                if (val2f) val2f[slot] = make_float2((float)e[2 * h].val, (float)e[2 * h + 1].val);
             }
         }
     }
@@ -180,7 +247,7 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     const int m = A->m, n = A->n, nnz = A->nnz, nl = n - H;
     TmpBuf<int> cps((size_t)n + 1, s);  // entries of the sorted columns before each
     exclusive_scan_i32(A->sortnnz.p, cps.p, n, s);
-    HostInts h(s);  // light entries, longest light column; pair rows, a row out of its window
+    HostInts h(s);  // light entries, longest light column; pair rows
     if (nl > 0) {
         k_hyb_light<<<1, 64, 0, s>>>(cps.p, A->sortnnz.p, nl, h.out(0));
         FL_LAUNCH_CHECK();
@@ -231,26 +298,18 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
         }
         k_hyb_bounds<<<hg((long long)nnz_h + 1), kBlock, 0, s>>>(rkey.p, nnz_h, m, hptr.p);
         FL_LAUNCH_CHECK();
-        // rows by (window, heavy count descending, row): two stable passes
-        TmpBuf<uint32_t> wkey(m, s);
-        k_hyb_lenkey<<<hg(m), kBlock, 0, s>>>(hptr.p, m, wkey.p, rows.p);
-        FL_LAUNCH_CHECK();
-        radix_sort_pairs(wkey.p, rows.p, m, 16, s);
-        k_hyb_winkey<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, wkey.p);
-        FL_LAUNCH_CHECK();
-        radix_sort_pairs(wkey.p, rows.p, m, bits_for((uint32_t)((m - 1) / win)), s);
-        k_hyb_pos<<<hg(m), kBlock, 0, s>>>(rows.p, m, win, A->hyb_iperm.p, A->hyb_perm.p, h.out(3));
+        // rows by (window, heavy count descending, row)
         TmpBuf<int> pairs(std::max(nslice, 1), s), pscan((size_t)nslice + 1, s);
-        k_hyb_pairs<<<hg(nslice), kBlock, 0, s>>>(rows.p, hptr.p, m, nslice, A->hyb_np.p, pairs.p);
+        const int rounds = div_up(win, kOrderThreads);
+        const size_t lds = sizeof(uint16_t) * 4 * rounds * kOrderThreads + sizeof(int) * kOrderWaves * 256;
+        FL_HIP(hipFuncSetAttribute((const void *)k_hyb_order, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        k_hyb_order<<<div_up(m, win), kOrderThreads, lds, s>>>(hptr.p, m, win, rounds, rows.p, A->hyb_iperm.p,
+                                                              A->hyb_perm.p, A->hyb_np.p, pairs.p);
         FL_LAUNCH_CHECK();
         exclusive_scan_i32(pairs.p, pscan.p, nslice, s, h.out(2));
         k_hyb_slot_base<<<hg((long long)nslice + 1), kBlock, 0, s>>>(pscan.p, nslice, A->hyb_sb.p);
         FL_LAUNCH_CHECK();
         slots = 64LL * h.wait()[2];
-        if (h[3]) {
-            set_error("HYB schedule: preprocessing moved a row out of its window");
-            throw HipError{hipErrorInvalidValue};
-        }
     }
     // slots past the last slice: the kernel's look-ahead loads past a wave's last slice read
     // kHybPairs pair rows at hyb_slots, and those past a slice's end up to kHybPairs - 1 pair
@@ -263,10 +322,15 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
                                                          padded - slots);
     FL_LAUNCH_CHECK();
     FL_HIP(hipMemsetAsync(A->hyb_val64.p + 2 * slots, 0, sizeof(double) * 2 * (size_t)(padded - slots), s));
+    if (A->val32.p) {  // FP32 values along with the others
+        A->hyb_val32.alloc((size_t)padded * 2);
+        FL_HIP(hipMemsetAsync(A->hyb_val32.p + 2 * slots, 0, sizeof(float) * 2 * (size_t)(padded - slots), s));
+    }
     if (slots > 0) {
         k_hyb_fill<<<(grid_for((long long)nslice * 64) + 7u) & ~7u, kBlock, 0, s>>>(m, nslice, H, rows.p, A->hyb_np.p, A->hyb_sb.p, hptr.p,
                                                                  ridx.p, ents.p, A->hyb_col2.p,
-                                                                 (double2 *)A->hyb_val64.p);
+                                                                 (double2 *)A->hyb_val64.p,
+                                                                 (float2 *)A->hyb_val32.p);
         FL_LAUNCH_CHECK();
     }
     A->hyb_light = std::move(L);
