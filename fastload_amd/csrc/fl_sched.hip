@@ -242,6 +242,188 @@ __global__ void k_adjdiff(const int *__restrict__ in, int count, int *__restrict
     GRID_STRIDE(i, count) out[i] = in[i + 1] - in[i];
 }
 
+// ---- PB places without a sort
+// A batch's entries of one band are a run, and a run's place in the product array is where the runs before it
+// end: with the lengths of all (band, batch) runs in a table in that order, its prefix sums are the places, and a
+// batch's entries find theirs by counting. That is one pass of a radix sort with the batch as tile and
+// the band as digit, in place of a sort by batch, one by band and one of the runs with the kernels between them
+// (33 launches). Bound by the two reads of the rows and the writes of 4 bytes per entry. Preparation, sorted -> this:
+// 67 M power-law entries 4,400 -> 1,045 us, 18 M uniform ones 1,500 -> 300, 3.5 M power-law ones 418 -> 150. The
+// arrays are the same bit for bit.
+constexpr int kPlaceThreads = 512, kPlaceWaves = kPlaceThreads / kWave;
+// Bands of the table: a workgroup keeps each wave's count of every band in LDS (144 KB at the most). At 16,384 rows a
+// band this covers 67 M rows.
+constexpr int kPlaceBands = 4096;
+constexpr int kPlaceTiles = 256;  // the largest batch
+
+// The table's order: chunk, band, then the chunk's batches by XCD (k_key_batch_xcd; a chunk starts at a multiple
+// of 8 batches).
+struct PbCells {
+    const int *__restrict__ cb;  // [C + 1] first batch of every chunk
+    int C, nbands;
+    // batch b's chunk, its cell of band 0 and the distance of its cells
+    __device__ __forceinline__ int find(int b, int &first, int &stride) const {
+        int c = 0;
+        while (c + 1 < C && b >= cb[c + 1]) ++c;
+        const int b0 = cb[c], n = cb[c + 1] - b0, q = b - b0, x = q & 7;
+        first = nbands * b0 + x * (n >> 3) + min(x, n & 7) + (q >> 3);
+        stride = n;
+        return c;
+    }
+};
+
+// A batch's run lengths into the table, and how many are not zero.
+__global__ __launch_bounds__(kPlaceThreads) void k_pb_count(int T, int bt, int n, const int *__restrict__ ord_ptr,
+                                                            const int *__restrict__ ord_cx, const int *__restrict__ row,
+                                                            int R, PbCells pc, int *__restrict__ len,
+                                                            int *__restrict__ nonzero) {
+    extern __shared__ int cnt[];
+    constexpr int U = 4;
+    const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i1 = (int)min((long long)(b + 1) * bt, (long long)T);
+    for (int k = threadIdx.x; k < pc.nbands; k += kPlaceThreads) cnt[k] = 0;
+    __syncthreads();
+    for (int i = b * bt + w * U; i < i1; i += kPlaceWaves * U) {
+        int r[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            r[u] = i + u < i1 && lane < n - ord_cx[i + u] ? row[ord_ptr[i + u] + lane] : -1;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (r[u] >= 0) atomicAdd(&cnt[r[u] / R], 1);
+    }
+    __syncthreads();
+    int first, stride, some = 0;
+    (void)pc.find(b, first, stride);
+    for (int k = threadIdx.x; k < pc.nbands; k += kPlaceThreads) {
+        const int c = cnt[k];
+        len[first + (long long)k * stride] = c;
+        some += c > 0;
+    }
+    for (int o = 32; o > 0; o >>= 1) some += __shfl_down(some, o, 64);
+    __shared__ int part[kPlaceWaves];
+    if (lane == 0) part[w] = some;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kPlaceWaves; ++q) some += part[q];
+        nonzero[b] = some;
+    }
+}
+
+// The bands' starts in the product array, and to the host every chunk's offset (k_chunk_off) and start.
+__global__ void k_pb_bands(const int *__restrict__ pos, PbCells pc, int cells, int *__restrict__ band_start,
+                           int *__restrict__ host_off, int *__restrict__ host_start) {
+    GRID_STRIDE(i, (long long)pc.C * pc.nbands + 1) {
+        const int c = (int)(i / pc.nbands), k = (int)(i % pc.nbands);
+        const int at = c < pc.C ? pos[pc.nbands * pc.cb[c] + k * (pc.cb[c + 1] - pc.cb[c])] : pos[cells];
+        band_start[i] = at;
+        if (k == 0) {
+            host_start[c] = at;
+            if (c < pc.C) host_off[c] = at & ~3;
+        }
+    }
+}
+
+// A batch's runs and the places of its entries: their slots in the batch's staging area, run by run, and their rows
+// by place. The entries of a run keep the order of the tile layout: the batch's tiles are put in that order, each
+// wave takes consecutive ones, and the lanes of a tile with the same band are ranked by ballots, as in the radix sort.
+__global__ __launch_bounds__(kPlaceThreads) void k_pb_place(int T, int bt, int n, const int *__restrict__ ord_ptr,
+                                                            const int *__restrict__ ord_cx, const int *__restrict__ row,
+                                                            int R, PbCells pc, int band_bits,
+                                                            const int *__restrict__ pos, const int *__restrict__ run_off,
+                                                            int *__restrict__ run_lstart, int *__restrict__ run_dest,
+                                                            int *__restrict__ run_len, uint16_t *__restrict__ lslot,
+                                                            uint16_t *__restrict__ rowlocal) {
+    extern __shared__ int place_lds[];
+    __shared__ int raw_ptr[kPlaceTiles], raw_len[kPlaceTiles], tile_ptr[kPlaceTiles], tile_len[kPlaceTiles];
+    __shared__ int wsum[kPlaceWaves];
+    const int nbands = pc.nbands;
+    const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int *wcnt = place_lds + w * nbands;                 // this wave's entries by band, then its next slots
+    int *shift = place_lds + kPlaceWaves * nbands;      // place of an entry minus its slot, by band
+    const int tiles = (int)min((long long)bt, (long long)T - (long long)b * bt);
+    for (int k = threadIdx.x; k < kPlaceWaves * nbands; k += kPlaceThreads) place_lds[k] = 0;
+    if ((int)threadIdx.x < tiles) {
+        const int i = b * bt + (int)threadIdx.x;
+        raw_ptr[threadIdx.x] = ord_ptr[i];
+        raw_len[threadIdx.x] = min(64, n - ord_cx[i]);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < tiles) {
+        const int p = raw_ptr[threadIdx.x];
+        int before = 0;
+        for (int j = 0; j < tiles; ++j) before += raw_ptr[j] < p;  // no two tiles start at the same entry
+        tile_ptr[before] = p;
+        tile_len[before] = raw_len[threadIdx.x];
+    }
+    __syncthreads();
+    const int per = (tiles + kPlaceWaves - 1) / kPlaceWaves;
+    const int t0 = w * per, t1 = min(tiles, t0 + per);
+    for (int t = t0; t < t1; ++t)
+        if (lane < tile_len[t]) atomicAdd(&wcnt[row[tile_ptr[t] + lane] / R], 1);
+    // the runs before each band's, and the entries in them: each thread has consecutive bands
+    int first, stride;
+    const int c = pc.find(b, first, stride);
+    const int off = pos[pc.nbands * pc.cb[c]] & ~3;
+    const int each = (nbands + kPlaceThreads - 1) / kPlaceThreads;
+    const int k0 = min((int)threadIdx.x * each, nbands), k1 = min(k0 + each, nbands);
+    int entries = 0, runs = 0;
+    for (int k = k0; k < k1; ++k) {
+        const long long cell = first + (long long)k * stride;
+        const int len = pos[cell + 1] - pos[cell];
+        entries += len;
+        runs += len > 0;
+    }
+    const int both = (runs << 16) | entries;  // at most 16,384 entries and 4,096 runs
+    int sum = wave_inclusive_scan(both);
+    if (lane == 63) wsum[w] = sum;
+    __syncthreads();  // also: every wave has counted
+    sum -= both;
+    for (int q = 0; q < w; ++q) sum += wsum[q];
+    int slot = sum & 0xffff, run = run_off[b] + (sum >> 16);
+    for (int k = k0; k < k1; ++k) {
+        const long long cell = first + (long long)k * stride;
+        const int at = pos[cell], len = pos[cell + 1] - at;
+        shift[k] = at - slot;
+        if (len > 0) {
+            run_lstart[run] = slot;
+            run_dest[run] = at - off;
+            run_len[run] = len;
+            ++run;
+        }
+        int next = slot;
+        for (int q = 0; q < kPlaceWaves; ++q) {
+            const int v = place_lds[q * nbands + k];
+            place_lds[q * nbands + k] = next;
+            next += v;
+        }
+        slot += len;
+    }
+    __syncthreads();
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    int r = t0 < t1 && lane < tile_len[t0] ? row[tile_ptr[t0] + lane] : 0;
+    for (int t = t0; t < t1; ++t) {
+        const int g = tile_ptr[t] + lane, here = r;
+        const bool valid = lane < tile_len[t];
+        r = t + 1 < t1 && lane < tile_len[t + 1] ? row[tile_ptr[t + 1] + lane] : 0;
+        const int band = here / R;
+        uint64_t peers = ballot64(valid);
+        for (int k = 0; k < band_bits; ++k) {
+            const bool bit = (band >> k) & 1;
+            const uint64_t m = ballot64(bit);
+            peers &= bit ? m : ~m;
+        }
+        const int rank = __popcll(peers & lt_mask);
+        int o = 0;
+        if (valid && rank == 0) o = atomicAdd(&wcnt[band], __popcll(peers));
+        o = __shfl(o, valid ? __ffsll((unsigned long long)peers) - 1 : lane, 64) + rank;
+        if (valid) {
+            lslot[g] = (uint16_t)o;
+            rowlocal[shift[band] + o] = (uint16_t)(here - band * R);
+        }
+    }
+}
+
 // Validators: every index the kernels will use must be inside the buffers they assume. flag is in host memory,
 // written only when something is wrong.
 __global__ void k_check_win(const int *__restrict__ batch_of, const uint16_t *__restrict__ slot,
@@ -408,6 +590,85 @@ static int pb_band_rows(int m, int bt, int R) {
     return std::min(R, std::max(1024, (per + 1023) / 1024 * 1024));
 }
 
+template <typename K>
+static void allow_lds(K kern, size_t bytes) {
+    FL_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+}
+
+static void pb_alloc_runs(fl_matrix *A, int nruns) {
+    A->nruns = nruns;
+    A->pb_run_lstart.alloc(nruns);
+    A->pb_run_dest.alloc(nruns);
+    A->pb_run_len.alloc(nruns);
+}
+
+// Runs and places from a table of the runs' lengths (k_pb_count, k_pb_place): nothing is sorted.
+static void pb_place_table(fl_matrix *A, int R, const int *d_cb, int C, HostInts &h, hipStream_t s) {
+    const int T = A->tilenum, nb = A->nbatches, nbands = A->nbands, cells = nb * nbands;
+    TmpBuf<int> len(cells, s), pos((size_t)cells + 1, s), nonzero(nb, s);
+    const PbCells pc{d_cb, C, nbands};
+    const size_t lds1 = sizeof(int) * nbands, lds2 = sizeof(int) * nbands * (kPlaceWaves + 1);
+    allow_lds(k_pb_count, lds1);
+    allow_lds(k_pb_place, lds2);
+    k_pb_count<<<nb, kPlaceThreads, lds1, s>>>(T, A->bt, A->n, A->ord_ptr.p, A->ord_cx.p, A->sortrowidx.p, R, pc, len.p,
+                                               nonzero.p);
+    FL_LAUNCH_CHECK();
+    exclusive_scan_i32(nonzero.p, A->pb_run_off.p, nb, s, h.out(0));
+    exclusive_scan_i32(len.p, pos.p, cells, s);
+    k_pb_bands<<<sg((long long)C * nbands + 1), kBlock, 0, s>>>(pos.p, pc, cells, A->pb_band_start.p, h.out(2),
+                                                               h.out(2 + C));
+    FL_LAUNCH_CHECK();
+    pb_alloc_runs(A, h.wait()[0]);
+    k_pb_place<<<nb, kPlaceThreads, lds2, s>>>(T, A->bt, A->n, A->ord_ptr.p, A->ord_cx.p, A->sortrowidx.p, R, pc,
+                                               bits_for((uint32_t)(nbands - 1)), pos.p, A->pb_run_off.p,
+                                               A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p, A->pb_lslot.p,
+                                               A->pb_rowlocal.p);
+    FL_LAUNCH_CHECK();
+}
+
+// The same by sorting the entries, for more bands than a workgroup counts in LDS.
+static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInts &h, hipStream_t s) {
+    const int nnz = A->nnz, nb = A->nbatches, nbands = A->nbands;
+    TmpBuf<int> d_off(C, s);
+    TmpBuf<uint32_t> key(nnz, s);
+    TmpBuf<int> order(nnz, s), head(nnz, s), runidx((size_t)nnz + 1, s);
+    // stable by batch (batches in XCD order), then stable by (chunk, band)
+    const int per_xcd = (nb + 7) / 8;
+    k_key_batch_xcd<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, per_xcd, key.p, nnz);
+    FL_LAUNCH_CHECK();
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
+    k_key_chunk_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, order.p, R, nbands, d_cb, C, key.p,
+                                                nnz);
+    FL_LAUNCH_CHECK();
+    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)(C * nbands - 1)), s);
+    k_key_bounds<<<sg((long long)C * nbands + 1), kBlock, 0, s>>>(key.p, nnz, C * nbands, A->pb_band_start.p);
+    k_chunk_off<<<1, kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p, h.out(2), h.out(2 + C));
+    k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->batch_of.p, A->sortrowidx.p, R, head.p,
+                                          A->pb_rowlocal.p, nnz);
+    FL_LAUNCH_CHECK();
+    exclusive_scan_i32(head.p, runidx.p, nnz, s, h.out(0));
+    const int nruns = h.wait()[0];
+    // The runs by (batch, band), and with their lengths the entries' staging slots. There are 20 to 60 times
+    // fewer runs than entries, and inside a run both orders are the same, so only the runs are sorted again.
+    // (Sorting the entries again was up to four passes over all of them and three gathers: the preparation of
+    // 18 M uniform entries 1,556 us, so 1,121; 9.6 M power-law entries 909 and 709; 1.8 M 289 and 289.)
+    pb_alloc_runs(A, nruns);
+    TmpBuf<int> run_pos(nruns, s), by(nruns, s), start((size_t)nruns + 1, s), lstart_of(nruns, s);
+    TmpBuf<uint32_t> run_key(nruns, s);
+    k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, key.p, order.p, A->batch_of.p, nbands, run_pos.p, run_key.p,
+                                         nnz);
+    FL_LAUNCH_CHECK();
+    radix_sort_positions(run_key.p, by.p, nruns, bits_for((uint32_t)(nb * nbands - 1)), s);
+    k_pb_run_len<<<sg(nruns), kBlock, 0, s>>>(by.p, run_pos.p, nruns, nnz, A->pb_run_len.p);
+    FL_LAUNCH_CHECK();
+    exclusive_scan_i32(A->pb_run_len.p, start.p, nruns, s);
+    k_pb_run_place<<<sg(nruns), kBlock, 0, s>>>(run_key.p, by.p, run_pos.p, start.p, A->batch_start.p, d_cb, C,
+                                                d_off.p, nbands, nruns, nb, A->pb_run_lstart.p, A->pb_run_dest.p,
+                                                A->pb_run_off.p, lstart_of.p);
+    k_pb_slots<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, order.p, run_pos.p, lstart_of.p, A->pb_lslot.p, nnz);
+    FL_LAUNCH_CHECK();
+}
+
 void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     ensure_batches(A, bt, 0, s);
     R = pb_band_rows(A->m, bt, R);
@@ -449,56 +710,21 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
         throw HipError{hipErrorInvalidValue};
     }
     A->pb_band_start.alloc((size_t)C * nbands + 1);
-    TmpBuf<int> d_cb(cb.size(), s), d_off(C, s);
+    TmpBuf<int> d_cb(cb.size(), s);
     FL_HIP(hipMemcpyAsync(d_cb.p, cb.data(), sizeof(int) * cb.size(), hipMemcpyHostToDevice, s));
-    TmpBuf<uint32_t> key(nnz, s);
-    TmpBuf<int> order(nnz, s), head(nnz, s), runidx((size_t)nnz + 1, s);
-    // chunk-major, then band-major order (chunk, band, batch, g): stable by batch (batches in
-    // XCD order), then stable by (chunk, band), so each (batch, band) run occupies one contiguous
-    // range of the product array
-    const int per_xcd = (nb + 7) / 8;
-    k_key_batch_xcd<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, per_xcd, key.p, nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
-    k_key_chunk_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, order.p, R, nbands, d_cb.p, C, key.p,
-                                                nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)(C * nbands - 1)), s);
-    k_key_bounds<<<sg((long long)C * nbands + 1), kBlock, 0, s>>>(key.p, nnz, C * nbands, A->pb_band_start.p);
     HostInts h(s);  // runs; bad runs or slots; the chunks' offsets and starts
     static_assert(2 + 2 * kMaxChunks + 1 <= kHostInts, "chunk offsets fit the host block");
-    k_chunk_off<<<1, kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p, h.out(2), h.out(2 + C));
-    k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->batch_of.p, A->sortrowidx.p, R, head.p,
-                                          A->pb_rowlocal.p, nnz);
-    FL_LAUNCH_CHECK();
-    exclusive_scan_i32(head.p, runidx.p, nnz, s, h.out(0));
-    const int nruns = h.wait()[0];
-    A->nruns = nruns;
+    // The places of the entries, chunk-major, then band-major (chunk, band, batch, g), the batches in XCD
+    // order: each (batch, band) run is one contiguous range of the product array.
+    // The table while its counts fit LDS, and while it is not much larger than the entries (few entries in many
+    // batches of short tiles), which it then costs less than sorting them.
+    if (nbands <= kPlaceBands && (long long)nb * nbands <= 4LL * nnz) pb_place_table(A, R, d_cb.p, C, h, s);
+    else pb_place_sorted(A, R, d_cb.p, C, h, s);
     std::vector<int> off(C), cstart((size_t)C + 1);
     int ring = 0;
     for (int c = 0; c < C; ++c) off[c] = h[2 + c];
     for (int c = 0; c <= C; ++c) cstart[c] = h[2 + C + c];
     for (int c = 0; c < C; ++c) ring = std::max(ring, cstart[c + 1] - off[c]);
-    // The runs by (batch, band), and with their lengths the entries' staging slots. There are 20 to 60 times
-    // fewer runs than entries, and inside a run both orders are the same, so only the runs are sorted again.
-    // (Sorting the entries again was up to four passes over all of them and three gathers: the preparation of
-    // 18 M uniform entries 1,556 us, so 1,121; 9.6 M power-law entries 909 and 709; 1.8 M 289 and 289.)
-    A->pb_run_lstart.alloc(nruns);
-    A->pb_run_dest.alloc(nruns);
-    A->pb_run_len.alloc(nruns);
-    TmpBuf<int> run_pos(nruns, s), by(nruns, s), start((size_t)nruns + 1, s), lstart_of(nruns, s);
-    TmpBuf<uint32_t> run_key(nruns, s);
-    k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, key.p, order.p, A->batch_of.p, nbands, run_pos.p, run_key.p,
-                                         nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(run_key.p, by.p, nruns, bits_for((uint32_t)(nb * nbands - 1)), s);
-    k_pb_run_len<<<sg(nruns), kBlock, 0, s>>>(by.p, run_pos.p, nruns, nnz, A->pb_run_len.p);
-    FL_LAUNCH_CHECK();
-    exclusive_scan_i32(A->pb_run_len.p, start.p, nruns, s);
-    k_pb_run_place<<<sg(nruns), kBlock, 0, s>>>(run_key.p, by.p, run_pos.p, start.p, A->batch_start.p, d_cb.p, C,
-                                                d_off.p, nbands, nruns, nb, A->pb_run_lstart.p, A->pb_run_dest.p,
-                                                A->pb_run_off.p, lstart_of.p);
-    k_pb_slots<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, order.p, run_pos.p, lstart_of.p, A->pb_lslot.p, nnz);
     k_check_pb<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->pb_lslot.p, A->batch_start.p, A->bt * 64, nnz, ring,
                                           A->pb_run_off.p, A->pb_run_lstart.p, A->pb_run_dest.p, A->pb_run_len.p, nb,
                                           h.out(1));
@@ -1140,11 +1366,6 @@ static OrdTiles ord_tiles(const fl_matrix *A) {
     ot.n = A->n;
     ot.T = A->tilenum;
     return ot;
-}
-
-template <typename K>
-static void allow_lds(K kern, size_t bytes) {
-    FL_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
 template <typename V, typename X, typename Y, int MODE, int NT, bool ASSIGN, bool DOT>
