@@ -424,6 +424,85 @@ __global__ __launch_bounds__(kPlaceThreads) void k_pb_place(int T, int bt, int n
     }
 }
 
+// ---- WIN slots without a sort
+// A batch's slots are its distinct rows in ascending order. A workgroup marks the batch's rows (held in registers,
+// U tiles to a wave) in a bitmap in LDS, kWinSeg rows at a time from the lowest one not yet done, and a row's slot
+// is the number of marks below its own. Counts the distinct rows (PLACE false: distinct), or writes the slots and rows.
+// A batch of neighbouring rows takes one or two bitmaps, one of rows all over the matrix m / kWinSeg of them, 2 us
+// each. The sorts by row and by batch that this replaces are four or five passes over all entries, whatever m is.
+// Preparation, sorted -> this: 128^3 grid, 56 M entries 3,030 -> 1,200 us, 40^3 240 -> 140; 10 M power-law entries,
+// 600 K rows 1,160 -> 650; 36 M uniform ones, 3 M rows 5,000 -> 3,900; 25 M, 8.4 M rows (32 bitmaps) 3,600 -> 5,100:
+// the line is at 16 bitmaps for rows all over the matrix. The arrays are the same bit for bit.
+constexpr int kWinSeg = 1 << 18, kWinSegs = 16;
+template <int U, bool PLACE>
+__global__ __launch_bounds__(kPlaceThreads) void k_win_rows(int T, int bt, int n, const int *__restrict__ ord_ptr,
+                                                            const int *__restrict__ ord_cx, const int *__restrict__ row,
+                                                            const int *__restrict__ win_off, int *__restrict__ distinct,
+                                                            uint16_t *__restrict__ win_slot,
+                                                            int *__restrict__ win_rows) {
+    constexpr int kWords = kWinSeg / 32, kEach = kWords / kPlaceThreads;
+    __shared__ uint32_t bits[kWords];
+    __shared__ uint16_t below[kWords];  // marks in the words before
+    __shared__ int wred[2][kPlaceWaves];
+    const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i0 = b * bt + w * U;
+    int r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = i0 + u < T && lane < n - ord_cx[i0 + u] ? row[ord_ptr[i0 + u] + lane] : -1;
+    const int out = PLACE ? win_off[b] : 0;
+    int seen = 0;
+    for (int from = 0;;) {
+        int base = 0x7fffffff;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (r[u] >= from) base = min(base, r[u]);
+        for (int o = 32; o > 0; o >>= 1) base = min(base, __shfl_xor(base, o));
+        if (lane == 0) wred[0][w] = base;
+        for (int i = threadIdx.x; i < kWords; i += kPlaceThreads) bits[i] = 0;
+        __syncthreads();
+        for (int q = 0; q < kPlaceWaves; ++q) base = min(base, wred[0][q]);
+        if (base == 0x7fffffff) break;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int d = r[u] - base;
+            if (r[u] >= base && d < kWinSeg) atomicOr(&bits[d >> 5], 1u << (d & 31));
+        }
+        __syncthreads();
+        const int w0 = (int)threadIdx.x * kEach;
+        int marks = 0;
+        for (int i = 0; i < kEach; ++i) marks += __popc(bits[w0 + i]);
+        const int upto = wave_inclusive_scan(marks);
+        if (lane == 63) wred[1][w] = upto;
+        __syncthreads();
+        int at = upto - marks, total = 0;
+        for (int q = 0; q < kPlaceWaves; ++q) {
+            at += q < w ? wred[1][q] : 0;
+            total += wred[1][q];
+        }
+        if constexpr (PLACE) {
+            for (int i = 0; i < kEach; ++i) {
+                below[w0 + i] = (uint16_t)at;
+                for (uint32_t m = bits[w0 + i]; m; m &= m - 1)
+                    win_rows[out + seen + at++] = base + (w0 + i) * 32 + __ffs((int)m) - 1;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int d = r[u] - base;
+                if (r[u] >= base && d < kWinSeg)
+                    win_slot[ord_ptr[i0 + u] + lane] =
+                        (uint16_t)(seen + below[d >> 5] + __popc(bits[d >> 5] & ((1u << (d & 31)) - 1u)));
+            }
+            __syncthreads();  // the bitmap is cleared next
+        }
+        seen += total;
+        from = base + kWinSeg;
+    }
+    if constexpr (!PLACE) {
+        if (threadIdx.x == 0) distinct[b] = seen;
+    }
+}
+
 // Validators: every index the kernels will use must be inside the buffers they assume. flag is in host memory,
 // written only when something is wrong.
 __global__ void k_check_win(const int *__restrict__ batch_of, const uint16_t *__restrict__ slot,
@@ -502,6 +581,49 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
 
 void pack_schedules(fl_matrix *A, hipStream_t s);
 
+// Slots and rows from bitmaps of the batches' rows (k_win_rows).
+static void win_rows_counted(fl_matrix *A, HostInts &h, hipStream_t s) {
+    const int nb = A->nbatches;
+    TmpBuf<int> distinct(nb, s);
+    auto run = [&](auto count, auto place) {
+        count<<<nb, kPlaceThreads, 0, s>>>(A->tilenum, A->bt, A->n, A->ord_ptr.p, A->ord_cx.p, A->sortrowidx.p, nullptr,
+                                           distinct.p, nullptr, nullptr);
+        FL_LAUNCH_CHECK();
+        exclusive_scan_i32(distinct.p, A->win_off.p, nb, s, h.out(0));
+        A->win_rows.alloc(std::max(h.wait()[0], 1));
+        place<<<nb, kPlaceThreads, 0, s>>>(A->tilenum, A->bt, A->n, A->ord_ptr.p, A->ord_cx.p, A->sortrowidx.p,
+                                           A->win_off.p, nullptr, A->win_slot.p, A->win_rows.p);
+        FL_LAUNCH_CHECK();
+    };
+    if (A->bt == 64) run(k_win_rows<64 / kPlaceWaves, false>, k_win_rows<64 / kPlaceWaves, true>);
+    else if (A->bt == 128) run(k_win_rows<128 / kPlaceWaves, false>, k_win_rows<128 / kPlaceWaves, true>);
+    else run(k_win_rows<256 / kPlaceWaves, false>, k_win_rows<256 / kPlaceWaves, true>);
+}
+
+// The same by sorting the entries by (batch, row).
+static void win_rows_sorted(fl_matrix *A, HostInts &h, hipStream_t s) {
+    const int nnz = A->nnz, nb = A->nbatches;
+    TmpBuf<uint32_t> key(nnz, s);
+    TmpBuf<int> order(nnz, s), head(nnz, s), d((size_t)nnz + 1, s);
+    // (row, g) order, then stable by batch -> (batch, row, g)
+    k_key_copy<<<sg(nnz), kBlock, 0, s>>>(A->sortrowidx.p, key.p, nnz, 1);
+    FL_LAUNCH_CHECK();
+    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
+    k_key_gather<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, order.p, key.p, nnz);
+    FL_LAUNCH_CHECK();
+    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(nb - 1, 0)), s);
+    k_win_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, nnz);
+    FL_LAUNCH_CHECK();
+    exclusive_scan_i32(head.p, d.p, nnz, s, h.out(0));
+    const int D = h.wait()[0];
+    A->win_rows.alloc(std::max(D, 1));
+    k_win_off<<<sg(nnz), kBlock, 0, s>>>(key.p, d.p, A->win_off.p, nnz, nb);
+    FL_LAUNCH_CHECK();
+    k_win_slot<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, d.p, A->win_off.p, A->win_slot.p,
+                                          A->win_rows.p, nnz);
+    FL_LAUNCH_CHECK();
+}
+
 void win_prepare(fl_matrix *A, int bt, bool rows, hipStream_t s) {
     ensure_batches(A, bt, rows ? 1 : 0, s);
     if (A->win_ready) return;
@@ -516,26 +638,10 @@ void win_prepare(fl_matrix *A, int bt, bool rows, hipStream_t s) {
         A->win_ready = true;
         return;
     }
-    TmpBuf<uint32_t> key(nnz, s);
-    TmpBuf<int> order(nnz, s), head(nnz, s), d((size_t)nnz + 1, s);
-    // (row, g) order, then stable by batch -> (batch, row, g)
-    k_key_copy<<<sg(nnz), kBlock, 0, s>>>(A->sortrowidx.p, key.p, nnz, 1);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
-    k_key_gather<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, order.p, key.p, nnz);
-    FL_LAUNCH_CHECK();
-    radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(nb - 1, 0)), s);
-    k_win_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, nnz);
-    FL_LAUNCH_CHECK();
     HostInts h(s);  // distinct rows; out-of-range slots
-    exclusive_scan_i32(head.p, d.p, nnz, s, h.out(0));
-    const int D = h.wait()[0];
-    A->win_rows.alloc(std::max(D, 1));
-    k_win_off<<<sg(nnz), kBlock, 0, s>>>(key.p, d.p, A->win_off.p, nnz, nb);
-    FL_LAUNCH_CHECK();
-    k_win_slot<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->sortrowidx.p, head.p, d.p, A->win_off.p, A->win_slot.p,
-                                          A->win_rows.p, nnz);
-    FL_LAUNCH_CHECK();
+    if (A->m <= kWinSegs * kWinSeg) win_rows_counted(A, h, s);
+    else win_rows_sorted(A, h, s);
+    const int D = h[0];
     k_check_win<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->win_slot.p, A->win_off.p, bt * 64, nnz, A->m,
                                            A->win_rows.p, h.out(1));
     FL_LAUNCH_CHECK();
