@@ -71,7 +71,7 @@ void row_prepare(fl_matrix *A, hipStream_t s) {
     FL_LAUNCH_CHECK();
     exclusive_scan_i32(len.p, colptr.p, n, s);
     columns_from_tiles(A, 0, colptr.p, 0, A->perm.p, key.p, ents.p, s);
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(m - 1, 0)), s);
+    radix_sort_positions(key.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(m - 1, 0)), s);
     k_rows_fill<<<sgb(nnz), kBlock, 0, s>>>(order.p, ents.p, A->row_col.p, A->row_val64.p, A->row_val32.p, nnz);
     k_row_bounds<<<sgb((long long)nnz + 1), kBlock, 0, s>>>(key.p, nnz, m, A->row_ptr.p);
     FL_LAUNCH_CHECK();

@@ -223,7 +223,8 @@ void exclusive_scan_i32(const int *in, int *out, int count, hipStream_t s, int *
 // keys/vals are sorted in place (ping-pong through internal scratch).
 void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_t s);
 // The same with the values 0 .. count - 1: order[i] = input position of the i-th key (order is output only).
-void radix_sort_positions(uint32_t *keys, int *order, int count, int bits, hipStream_t s);
+// The keys come from in, which may be keys itself.
+void radix_sort_positions(const uint32_t *in, uint32_t *keys, int *order, int count, int bits, hipStream_t s);
 
 // Keys grouped by their top 8 bits [shift, shift + 8), and where each of the 256 groups starts.
 void radix_partition(const uint32_t *keys, uint32_t *out, int count, int shift, int *start, hipStream_t s);

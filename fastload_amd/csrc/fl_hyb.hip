@@ -294,7 +294,7 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     if (m > 0) {
         if (nnz_h > 0) {  // heavy entries by row (stable: inside a row by column)
             columns_from_tiles(A, nl, cps.p, nnz_l, nullptr, rkey.p, ents.p, s);
-            radix_sort_positions(rkey.p, ridx.p, nnz_h, bits_for((uint32_t)(m - 1)), s);
+            radix_sort_positions(rkey.p, rkey.p, ridx.p, nnz_h, bits_for((uint32_t)(m - 1)), s);
         }
         k_hyb_bounds<<<hg((long long)nnz_h + 1), kBlock, 0, s>>>(rkey.p, nnz_h, m, hptr.p);
         FL_LAUNCH_CHECK();

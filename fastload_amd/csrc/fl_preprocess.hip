@@ -19,16 +19,6 @@
 namespace fl {
 
 // ----------------------------------------------------------------------- small kernels
-__global__ void k_copy_keys(const int *__restrict__ in, uint32_t *__restrict__ out, int count) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
-        out[i] = (uint32_t)in[i];
-}
-
-__global__ void k_keys_to_int(const uint32_t *__restrict__ in, int *__restrict__ out, int count) {
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
-        out[i] = (int)in[i];
-}
-
 template <typename T>
 __global__ void k_gather(const T *__restrict__ src, const int *__restrict__ idx, T *__restrict__ dst, int count) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
@@ -98,10 +88,10 @@ void csr2csc_device(int m, int n, int nnz, const int *d_rowptr, const int *d_col
     if (nnz > 0) {
         TmpBuf<uint32_t> keys(nnz, s);
         TmpBuf<int> order(nnz, s), row_of(nnz, s);
-        k_copy_keys<<<stride_grid(nnz), kBlock, 0, s>>>(d_colind, keys.p, nnz);
         k_row_of<<<stride_grid(m), kBlock, 0, s>>>(d_rowptr, m, row_of.p);
         FL_LAUNCH_CHECK();
-        radix_sort_positions(keys.p, order.p, nnz, bits_for((uint32_t)std::max(n - 1, 0)), s);
+        radix_sort_positions((const uint32_t *)d_colind, keys.p, order.p, nnz,
+                             bits_for((uint32_t)std::max(n - 1, 0)), s);
         k_csc_fill<<<stride_grid(nnz), kBlock, 0, s>>>(order.p, row_of.p, d_val, d_cscrow, d_cscval, nnz);
         k_count<<<stride_grid(nnz), kBlock, 0, s>>>(keys.p, nnz, d_nnzpercol);
         FL_LAUNCH_CHECK();
@@ -113,12 +103,7 @@ void csr2csc_device(int m, int n, int nnz, const int *d_rowptr, const int *d_col
 // ------------------------------------------------------------------------ column sort
 void colsort_device(int n, const int *d_counts, int *d_perm, int *d_sortnnz, int max_key, hipStream_t s) {
     if (n <= 0) return;
-    TmpBuf<uint32_t> keys(n, s);
-    k_copy_keys<<<stride_grid(n), kBlock, 0, s>>>(d_counts, keys.p, n);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(keys.p, d_perm, n, bits_for((uint32_t)max_key), s);
-    k_keys_to_int<<<stride_grid(n), kBlock, 0, s>>>(keys.p, d_sortnnz, n);
-    FL_LAUNCH_CHECK();
+    radix_sort_positions((const uint32_t *)d_counts, (uint32_t *)d_sortnnz, d_perm, n, bits_for((uint32_t)max_key), s);
 }
 
 // Concatenate the sorted columns (Pre4SortIdxVal, ColSort_GPU.h:21-43): one lane per column

@@ -374,12 +374,18 @@ __global__ void k_copy_pairs(const uint32_t *__restrict__ k, const int *__restri
     }
 }
 
-static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool positions, hipStream_t s) {
+// in: the keys, in another array than `keys` or in it. From another array the passes alternate between the scratch pair
+// and the caller's arrays so that the last one ends there; in place that takes a third pair for an odd
+// number of passes, and a copy for a single one.
+static void sort_pairs(const uint32_t *in, uint32_t *keys, int *vals, int count, int bits, bool positions, hipStream_t s) {
+    const bool inplace = in == keys;
     if (count <= 1 || bits <= 0) {
         if (positions && count > 0) {
             k_positions<<<std::min(grid_for(count), 65536u), kBlock, 0, s>>>(vals, count);
             FL_LAUNCH_CHECK();
         }
+        if (!inplace && count > 0)
+            FL_HIP(hipMemcpyAsync(keys, in, sizeof(uint32_t) * (size_t)count, hipMemcpyDeviceToDevice, s));
         return;
     }
     const int nb = div_up(count, kSortTile);
@@ -390,25 +396,27 @@ static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool posi
     }
     TmpBuf<int> hist((size_t)hcount, s), offs((size_t)hcount + 1, s);
     const int passes = (bits + kRadixBits - 1) / kRadixBits;
-    // an odd number of passes ends in the caller's arrays by way of a third pair
-    const bool third = passes >= 3 && passes % 2 == 1;
-    TmpBuf<uint32_t> k2(count, s), k3(third ? count : 0, s);
-    TmpBuf<int> v2(count, s), v3(third ? count : 0, s);
-    uint32_t *kin = keys, *kout = k2.p;
-    int *vin = vals, *vout = v2.p;
+    const bool third = inplace && passes >= 3 && passes % 2 == 1;
+    const bool scratch = inplace || passes > 1;
+    TmpBuf<uint32_t> k2(scratch ? count : 0, s), k3(third ? count : 0, s);
+    TmpBuf<int> v2(scratch ? count : 0, s), v3(third ? count : 0, s);
+    const uint32_t *kin = in;
+    const int *vin = vals;
     for (int p = 0; p < passes; ++p) {
         const int shift = p * kRadixBits;
+        uint32_t *kout = (passes - 1 - p) % 2 == 0 ? keys : k2.p;
+        int *vout = (passes - 1 - p) % 2 == 0 ? vals : v2.p;
         if (third && p == 1) kout = k3.p, vout = v3.p;
-        if (third && p == 2) kout = keys, vout = vals;
+        if (inplace && p == 0) kout = k2.p, vout = v2.p;
         k_radix_hist<<<sort_grid(nb), kBlock, 0, s>>>(kin, count, shift, nb, hist.p);
         FL_LAUNCH_CHECK();
         exclusive_scan_i32(hist.p, offs.p, (int)hcount, s);
         k_radix_scatter<true><<<sort_grid(nb), kBlock, 0, s>>>(kin, positions && p == 0 ? nullptr : vin, kout, vout, count, shift, nb, offs.p);
         FL_LAUNCH_CHECK();
-        std::swap(kin, kout);
-        std::swap(vin, vout);
+        kin = kout;
+        vin = vout;
     }
-    if (kin != keys) {  // one pass
+    if (kin != keys) {  // one pass in place
         k_copy_pairs<<<std::min(grid_for(count), 65536u), kBlock, 0, s>>>(kin, vin, keys, vals, count);
         FL_LAUNCH_CHECK();
     }
@@ -417,11 +425,11 @@ static void sort_pairs(uint32_t *keys, int *vals, int count, int bits, bool posi
 }
 
 void radix_sort_pairs(uint32_t *keys, int *vals, int count, int bits, hipStream_t s) {
-    sort_pairs(keys, vals, count, bits, false, s);
+    sort_pairs(keys, keys, vals, count, bits, false, s);
 }
 
-void radix_sort_positions(uint32_t *keys, int *order, int count, int bits, hipStream_t s) {
-    sort_pairs(keys, order, count, bits, true, s);
+void radix_sort_positions(const uint32_t *in, uint32_t *keys, int *order, int count, int bits, hipStream_t s) {
+    sort_pairs(in, keys, order, count, bits, true, s);
 }
 
 __global__ void k_bin_starts(const int *__restrict__ offs, int nblocks, int count, int *__restrict__ start) {

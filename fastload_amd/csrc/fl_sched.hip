@@ -556,7 +556,7 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
             else k_tile_bucket<<<sg(T), kBlock, 0, s>>>(A->tile_colidx.p, T, key.p);
             FL_LAUNCH_CHECK();
             const int top = kind == 1 ? (A->m - 1) >> 6 : (A->n - 1) >> 8;
-            radix_sort_positions(key.p, order.p, T, bits_for((uint32_t)std::max(top, 0)), s);
+            radix_sort_positions(key.p, key.p, order.p, T, bits_for((uint32_t)std::max(top, 0)), s);
             k_tile_reorder<<<sg(T), kBlock, 0, s>>>(order.p, A->tile_ptr.p, A->tile_colidx.p, T, A->ord_ptr.p,
                                                     A->ord_cx.p);
             FL_LAUNCH_CHECK();
@@ -608,7 +608,7 @@ static void win_rows_sorted(fl_matrix *A, HostInts &h, hipStream_t s) {
     // (row, g) order, then stable by batch -> (batch, row, g)
     k_key_copy<<<sg(nnz), kBlock, 0, s>>>(A->sortrowidx.p, key.p, nnz, 1);
     FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
+    radix_sort_positions(key.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
     k_key_gather<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, order.p, key.p, nnz);
     FL_LAUNCH_CHECK();
     radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(nb - 1, 0)), s);
@@ -742,7 +742,7 @@ static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInt
     const int per_xcd = (nb + 7) / 8;
     k_key_batch_xcd<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, per_xcd, key.p, nnz);
     FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
+    radix_sort_positions(key.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(8 * per_xcd - 1, 0)), s);
     k_key_chunk_band<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, A->sortrowidx.p, order.p, R, nbands, d_cb, C, key.p,
                                                 nnz);
     FL_LAUNCH_CHECK();
@@ -764,7 +764,7 @@ static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInt
     k_pb_runs<<<sg(nnz), kBlock, 0, s>>>(head.p, runidx.p, key.p, order.p, A->batch_of.p, nbands, run_pos.p, run_key.p,
                                          nnz);
     FL_LAUNCH_CHECK();
-    radix_sort_positions(run_key.p, by.p, nruns, bits_for((uint32_t)(nb * nbands - 1)), s);
+    radix_sort_positions(run_key.p, run_key.p, by.p, nruns, bits_for((uint32_t)(nb * nbands - 1)), s);
     k_pb_run_len<<<sg(nruns), kBlock, 0, s>>>(by.p, run_pos.p, nruns, nnz, A->pb_run_len.p);
     FL_LAUNCH_CHECK();
     exclusive_scan_i32(A->pb_run_len.p, start.p, nruns, s);
