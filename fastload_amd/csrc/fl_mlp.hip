@@ -78,16 +78,17 @@ __global__ void k_feat_rowcount(const int *__restrict__ rowidx, int nnz, int *__
 }
 
 // Entries per row from row indices grouped by row >> shift (start: 257 group bounds). A workgroup counts
-// kFeatChunk consecutive indices, group by group, in LDS (1 << shift counters) and adds what it has
+// a chunk of kFeatChunkMin to kFeatChunk consecutive indices, group by group, in LDS (1 << shift counters) and adds what it has
 // seen of a group to rc. Global atomics on random rows run at about 28 G/s (8.8 M entries, 600 K rows:
-// 310 us); grouped (radix_partition, 69 us) and counted here (22 us) it is LDS work, and the adds to
-// rc are coalesced.
-constexpr int kFeatChunk = 1 << 16, kFeatMaxShift = 15;
-__global__ __launch_bounds__(1024) void k_feat_rowcount_bins(const uint32_t *__restrict__ rows, int nnz, int shift,
+// 310 us); grouped (radix_partition, 69 us) and counted here (15 us) it is LDS work, and the adds to
+// rc are coalesced. Chunks are shorter where there are few entries, so that most compute units get one (1.8 M
+// entries: 25 us with 28 chunks, 11 with 110).
+constexpr int kFeatChunk = 1 << 16, kFeatChunkMin = 1 << 14, kFeatMaxShift = 15;
+__global__ __launch_bounds__(1024) void k_feat_rowcount_bins(const uint32_t *__restrict__ rows, int nnz, int chunk, int shift,
                                                              const int *__restrict__ start, int m,
                                                              int *__restrict__ rc) {
     extern __shared__ int cnt[];
-    const int c0 = (int)blockIdx.x * kFeatChunk, c1 = min(nnz - c0, kFeatChunk) + c0;
+    const int c0 = (int)blockIdx.x * chunk, c1 = min(nnz - c0, chunk) + c0;
     const int w = 1 << shift;
     for (int b = (int)(rows[c0] >> shift); b < 256 && start[b] < c1; ++b) {
         const int i0 = max(start[b], c0), i1 = min(start[b + 1], c1);
@@ -452,7 +453,8 @@ int fl_features(int m, int n, int nnz, const int *d_colptr, const int *d_rowidx,
             const size_t lds = sizeof(int) << shift;
             FL_HIP(hipFuncSetAttribute((const void *)k_feat_rowcount_bins, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds));
-            k_feat_rowcount_bins<<<div_up(nnz, kFeatChunk), 1024, lds, s>>>(rows.p, nnz, shift, start.p, m, rc);
+            const int chunk = std::min(std::max(nnz / 256, kFeatChunkMin), kFeatChunk);
+            k_feat_rowcount_bins<<<div_up(nnz, chunk), 1024, lds, s>>>(rows.p, nnz, chunk, shift, start.p, m, rc);
         } else {
             k_feat_rowcount<<<sgm(nnz), kBlock, 0, s>>>(d_rowidx, nnz, rc);
         }
