@@ -76,13 +76,16 @@ __global__ void k_tile_reorder(const int *__restrict__ order, const int *__restr
     }
 }
 
-// entry count of each batch (sum of its re-ordered tiles' lengths)
+// entry count of each batch (sum of its re-ordered tiles' lengths), a wave per batch (with a thread per batch
+// 14 us for 170 batches of 128 tiles, the loads of one after another)
 __global__ void k_batch_sizes(int T, int bt, int nb, int n, const int *__restrict__ ord_cx, int *__restrict__ sizes) {
-    GRID_STRIDE(b, nb) {
+    GRID_STRIDE(t, (long long)nb * 64) {
+        const int b = (int)(t >> 6), lane = (int)(t & 63);
         int s = 0;
-        const int i1 = min((int)(b + 1) * bt, T);
-        for (int i = (int)b * bt; i < i1; ++i) s += min(64, n - ord_cx[i]);
-        sizes[b] = s;
+        const long long i1 = min((long long)(b + 1) * bt, (long long)T);
+        for (long long i = (long long)b * bt + lane; i < i1; i += 64) s += min(64, n - ord_cx[i]);
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+        if (lane == 0) sizes[b] = s;
     }
 }
 
@@ -573,7 +576,7 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
     TmpBuf<int> sizes(std::max(A->nbatches, 1), s);
     if (T > 0) {
         k_batch_of<<<sg((long long)T * 64), kBlock, 0, s>>>(T, bt, A->n, A->ord_ptr.p, A->ord_cx.p, A->batch_of.p);
-        k_batch_sizes<<<sg(A->nbatches), kBlock, 0, s>>>(T, bt, A->nbatches, A->n, A->ord_cx.p, sizes.p);
+        k_batch_sizes<<<sg((long long)A->nbatches * 64), kBlock, 0, s>>>(T, bt, A->nbatches, A->n, A->ord_cx.p, sizes.p);
         FL_LAUNCH_CHECK();
     }
     exclusive_scan_i32(sizes.p, A->batch_start.p, A->nbatches, s);
