@@ -1479,9 +1479,13 @@ static OrdTiles ord_tiles(const fl_matrix *A) {
 
 template <typename V, typename X, typename Y, int MODE, int NT, bool ASSIGN, bool DOT>
 static auto win_kernel(int bt) {
-    constexpr int U = sizeof(X) == 4 ? 8 : 4;  // tiles per group: 8 keeps the 4-byte-x kinds within 64 VGPRs
+    // Tiles per group. FP64, 4 -> 8 (16): 80^3 27-point grid 33.8 -> 33.2 us (36.4), 127^3 150.2 -> 148.3 (160.0), a CG
+    // solve on 80^3 7,630 -> 7,510 (8,550); FP32 on 60^3 13.8 with 8, 14.7 with 16. In FP64 batches of 128 tiles keep 4,
+    // as 8 leave fewer of their 512-thread workgroups on a compute unit (WIN on 80^3: 64 tiles 33.3 with 4 and 8,
+    // 128 30.5 and 33.3, 256, where LDS decides that, 34.6 and 34.2).
+    constexpr int U = 8, U128 = sizeof(X) == 4 ? 8 : 4;
     return (bt == 256) ? k_win<V, X, Y, MODE, U, 256, NT, ASSIGN, DOT>
-           : (bt == 128) ? k_win<V, X, Y, MODE, U, 128, NT, ASSIGN, DOT> : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN, DOT>;
+           : (bt == 128) ? k_win<V, X, Y, MODE, U128, 128, NT, ASSIGN, DOT> : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN, DOT>;
 }
 
 template <typename V, typename X, typename Y, int MODE>
@@ -1514,7 +1518,8 @@ static void launch_win(const fl_matrix *A, const V *val, const X *x, Y *y, bool 
 template <typename V, typename X, typename P, typename Y, int MODE>
 static void launch_pb(const fl_matrix *A, const V *val, const X *x, P *bins, Y *y, bool assign,
                       hipStream_t s, const PbFold *fold) {
-    constexpr int U = sizeof(X) == 4 ? 8 : 4;  // tiles per group, as in WIN
+    // Tiles per group. FP64, 4 -> 8: 18 M uniform entries 119.7 -> 117.0 us; FP32 70.3 with 8, 77.9 with 16.
+    constexpr int U = 8;
     const PackFmt pf = A->pb_pf;
     const uint16_t *lslot = mode_kind(MODE) == kPacked ? nullptr : A->pb_lslot.p;
     constexpr bool S = (MODE & kStream) != 0;
