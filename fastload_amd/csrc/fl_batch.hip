@@ -319,6 +319,53 @@ __global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const in
     if (live && j == 0) Y[r] = accumulate ? (T)((ACC)Y[r] + acc) : (T)acc;
 }
 
+// The same sums for short rows, two lanes per row (32 rows per wave): lane j takes the fours j and j + 2 of every
+// sixteen, so each sum and their order are those of the four lanes above, bit for bit. Of rows of up to four
+// entries one lane in four has work there, and a wave half as many rows.
+template <typename T, typename ACC>
+__global__ __launch_bounds__(kBlock) void k_spmv_row1_short(int m, int chunk, const int *__restrict__ row_ptr,
+                                                            const int *__restrict__ row_col,
+                                                            const T *__restrict__ row_val, const T *__restrict__ X,
+                                                            T *__restrict__ Y, int accumulate) {
+    constexpr int RPW = 32;
+    const int idx = blockIdx.x >> 3;
+    const long long wg = (long long)(idx / chunk * 8 + (int)(blockIdx.x & 7)) * chunk + idx % chunk;
+    const int lane = threadIdx.x & 63, j = lane & 1;
+    const long long r = (wg * (kBlock / 64) + (threadIdx.x >> 6)) * RPW + (lane >> 1);
+    const bool live = r < m;  // all lanes reach the exchange
+    int e0 = 0, left = 0;     // entries from this lane's next four to the row's end
+    if (live) {
+        e0 = row_ptr[r];
+        left = row_ptr[r + 1] - e0 - 4 * j;
+    }
+    const int *__restrict__ pc = row_col + e0 + 4 * j;
+    const T *__restrict__ pv = row_val + e0 + 4 * j;
+    ACC acc[2] = {0, 0};
+    auto four = [&](ACC &a) {
+        int c[4];
+        T v[4], x[4];
+        load_quad(pc, c);
+        load_quad(pv, v);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = X[u < left ? c[u] : c[0]];
+        ACC q = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (u < left) q += (ACC)v[u] * (ACC)x[u];
+        a += q;
+        left -= 8;
+        pc += 8;
+        pv += 8;
+    };
+    while (left > 0) {
+        four(acc[0]);
+        if (left > 0) four(acc[1]);
+    }
+    ACC sum = acc[0] + acc[1];
+    sum += __shfl_xor(sum, 1, 64);
+    if (live && j == 0) Y[r] = accumulate ? (T)((ACC)Y[r] + sum) : (T)sum;
+}
+
 // Workgroups of `rows` rows each for m rows: chunks of kRowChunk rows, shorter where that would leave an
 // XCD fewer than eight of them, and a grid of whole chunks for each XCD.
 struct RowGrid {
@@ -330,8 +377,21 @@ static RowGrid row_grid(int m, int rows) {
     return {chunk, 8 * chunk * div_up(wgs, 8 * chunk)};
 }
 
+// Entries per row, on average, up to which rows take two lanes. Two lanes / four (every fourth entry per lane, before both), us:
+// 800 K rows in diagonal blocks, FP32, 3 entries 9.0 / 12.8 (9.8), 6 12.2 / 15.2 (17.1), 9 15.4 / 17.0 (21.5), FP64 at 9
+// 20.3 / 19.7 (34.3); 800 K rows of 3 uniform entries 16.1 / 17.8 (18.6), 6 28.7 / 26.5 (31.3), FP64 51.4 / 47.2 (58.3);
+// 60 stacked Zipf(2) matrices, 7 entries, 64.6 / 61.1 (75.9). From 7 on four lanes are ahead of both
+// on all of them but the blocks in FP32.
+constexpr long long kShortRow = 6;
 template <typename T, typename ACC>
 static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
+    if ((long long)A->nnz <= kShortRow * A->m) {
+        const RowGrid g = row_grid(A->m, 32 * (kBlock / 64));
+        k_spmv_row1_short<T, ACC><<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y,
+                                                            accumulate);
+        FL_LAUNCH_CHECK();
+        return;
+    }
     const RowGrid g = row_grid(A->m, 64 / kRowLanes * (kBlock / 64));
     const bool pre = (long long)A->nnz > 4LL * kRowLanes * A->m;  // rows of more than one step on average
     auto k = pre ? k_spmv_row1<T, ACC, true> : k_spmv_row1<T, ACC, false>;
