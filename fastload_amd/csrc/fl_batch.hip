@@ -486,6 +486,7 @@ int fl_matrix_prepare_rows(fl_matrix *A, void *stream) {
         return FL_ERR_INVALID;
     }
     row_prepare(A, (hipStream_t)stream);
+    FL_HIP(hipStreamSynchronize((hipStream_t)stream));  // products may follow on any stream
     return FL_OK;
     FL_API_END
 }
