@@ -209,6 +209,7 @@ struct CgState {
     hipGraphExec_t graph = nullptr;
     void *graph_x = nullptr;
     int graph_iters = 0;
+    unsigned graph_built = 0;  // A->built at the capture: the graph holds the schedule's addresses and sizes
     ~CgState() {
         if (s) (void)hipStreamSynchronize(s);
         if (graph) (void)hipGraphExecDestroy(graph);
@@ -296,7 +297,7 @@ static int cg_solve(CgState *c, const T *b, T *x, int max_iter, double rtol, int
         return FL_OK;
     }
     // capture `every` iterations (even, so every replay starts on scalar slot 0)
-    if (!c->graph || c->graph_x != (void *)x || c->graph_iters != every) {
+    if (!c->graph || c->graph_x != (void *)x || c->graph_iters != every || c->graph_built != c->A->built) {
         if (c->graph) FL_HIP(hipGraphExecDestroy(c->graph));
         c->graph = nullptr;
         FL_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
@@ -313,6 +314,7 @@ static int cg_solve(CgState *c, const T *b, T *x, int max_iter, double rtol, int
         FL_HIP(e);
         c->graph_x = x;
         c->graph_iters = every;
+        c->graph_built = c->A->built;
     }
     const double *hist = c->hist;
     while (done < max_iter) {

@@ -239,6 +239,7 @@ void hyb_values(fl_matrix *A, int kind, hipStream_t s) {
 
 void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
     if (A->hyb_ready && A->hyb_H == H && A->hyb_bt == bt && A->hyb_R == R) return;
+    ++A->built;
     A->hyb_ready = false;
     A->hyb_light.reset();
     A->hyb_val32.release();

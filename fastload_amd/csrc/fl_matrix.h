@@ -26,6 +26,7 @@ __device__ __forceinline__ float pack_decode(uint32_t w, const PackFmt &p) {
 
 struct fl_matrix {
     int m = 0, n = 0, nnz = 0, W = 32;
+    unsigned built = 0;  // raised before a schedule's arrays are built anew: launches recorded until then read the old ones
     int L = 0;        // levels (h_count)
     int tilenum = 0;
     int segsum = 0;

@@ -548,6 +548,7 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
     if (!A->ord_ptr.p || A->ord_kind != kind) {
         // stable sort of the tiles by 256-column bucket of their first sorted column (kind 0) or
         // by the 64-row window of their first entry (kind 1)
+        ++A->built;
         A->ord_ptr.alloc(std::max(T, 1));
         A->ord_cx.alloc(std::max(T, 1));
         A->ord_kind = kind;
@@ -566,6 +567,7 @@ static void ensure_batches(fl_matrix *A, int bt, int kind, hipStream_t s) {
         }
     }
     if (A->bt == bt && A->batch_of.p) return;
+    ++A->built;
     A->bt = bt;
     A->nbatches = (T + bt - 1) / bt;
     A->win_ready = A->pb_ready = false;
@@ -630,6 +632,7 @@ static void win_rows_sorted(fl_matrix *A, HostInts &h, hipStream_t s) {
 void win_prepare(fl_matrix *A, int bt, bool rows, hipStream_t s) {
     ensure_batches(A, bt, rows ? 1 : 0, s);
     if (A->win_ready) return;
+    ++A->built;
     A->win_pack.release();
     const int nnz = A->nnz, nb = A->nbatches;
     A->win_slot.alloc(std::max(nnz, 1));
@@ -782,6 +785,7 @@ void pb_prepare(fl_matrix *A, int bt, int R, hipStream_t s) {
     ensure_batches(A, bt, 0, s);
     R = pb_band_rows(A->m, bt, R);
     if (A->pb_ready && A->pb_R == R) return;
+    ++A->built;
     A->pb_ready = false;
     A->pb_pack.release();
     const int nnz = A->nnz, nb = A->nbatches, m = A->m;

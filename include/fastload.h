@@ -335,7 +335,7 @@ int fl_spmm(fl_matrix *A, int val_kind, int k, const void *d_X, void *d_Y, int a
  * src/FastLoad_GPU.h:349-374). The product uses one prepared schedule: kernel as for fl_spmv, or
  * FL_KERNEL_ROW (the row-ordered kernel, after fl_matrix_prepare_rows); val_kind FL_VAL_F64
  * (double b, x and vectors) or FL_VAL_F32 (float; dot products summed in FP64). A must outlive the
- * solver. fl_cg_solve starts from the x it is given, runs iterations in groups of check_every
+ * solver; its schedule may be prepared again between two solves, which then use the new one. fl_cg_solve starts from the x it is given, runs iterations in groups of check_every
  * (rounded up to even) captured once as a hipGraph, and after each group stops when
  * ||r|| / ||b|| <= rtol or max_iter iterations have run: *iters receives the iterations run (a
  * multiple of the group), *rel_res the final ||r|| / ||b|| (recursive residual). */
