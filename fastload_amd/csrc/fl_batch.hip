@@ -37,15 +37,6 @@ __global__ void k_rows_fill(const int *__restrict__ order, const ColEntry *__res
     }
 }
 
-// start[r] = first position of a key >= r, r in [0, m]; keys ascending
-__global__ void k_row_bounds(const uint32_t *__restrict__ k, int count, int m, int *__restrict__ start) {
-    GSTRIDE(i, (long long)count + 1) {
-        const long long lo = i == 0 ? 0 : (long long)k[i - 1] + 1;
-        const long long hi = i == count ? m : (long long)k[i];
-        for (long long r = lo; r <= hi; ++r) start[r] = (int)i;
-    }
-}
-
 // The row arrays end with kRowPad entries that belong to no row: the k = 1 kernel loads entries four at a time.
 constexpr int kRowPad = 4;
 
@@ -73,8 +64,8 @@ void row_prepare(fl_matrix *A, hipStream_t s) {
     columns_from_tiles(A, 0, colptr.p, 0, A->perm.p, key.p, ents.p, s);
     radix_sort_positions(key.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(m - 1, 0)), s);
     k_rows_fill<<<sgb(nnz), kBlock, 0, s>>>(order.p, ents.p, A->row_col.p, A->row_val64.p, A->row_val32.p, nnz);
-    k_row_bounds<<<sgb((long long)nnz + 1), kBlock, 0, s>>>(key.p, nnz, m, A->row_ptr.p);
     FL_LAUNCH_CHECK();
+    key_bounds(key.p, nnz, m, A->row_ptr.p, s);
     A->row_ready = true;
 }
 

@@ -229,6 +229,9 @@ void radix_sort_positions(const uint32_t *in, uint32_t *keys, int *order, int co
 // Keys grouped by their top 8 bits [shift, shift + 8), and where each of the 256 groups starts.
 void radix_partition(const uint32_t *keys, uint32_t *out, int count, int shift, int *start, hipStream_t s);
 
+// start[b] = first position of a key >= b in the ascending keys, b in [0, nb] (start[nb] = count when all are below nb).
+void key_bounds(const uint32_t *keys, int count, int nb, int *start, hipStream_t s);
+
 // Device reduction helpers.
 int device_max_i32(const int *in, int count, hipStream_t s);
 // The same in two steps: the kernel, and the maximum after h.wait().

@@ -48,15 +48,6 @@ __global__ void k_hyb_iota(int *__restrict__ v, int count) {
     HSTRIDE(i, count) v[i] = (int)i;
 }
 
-// ptr[r] = first i with key[i] >= r, r in [0, nb]; key ascending
-__global__ void k_hyb_bounds(const uint32_t *__restrict__ key, int count, int nb, int *__restrict__ ptr) {
-    HSTRIDE(i, (long long)count + 1) {
-        const long long lo = i == 0 ? 0 : (long long)key[i - 1] + 1;
-        const long long hi = i == count ? nb : (long long)key[i];
-        for (long long r = lo; r <= hi; ++r) ptr[r] = (int)i;
-    }
-}
-
 // Rows by (window, heavy count descending, row), and the pair rows of every slice (half its first, longest
 // row, rounded up). One workgroup per window: a stable radix sort of the counts in LDS, 8 bits at a time, the
 // second pass only where a row has 256 heavy entries or more. Each wave ranks a contiguous part of the rows, as in
@@ -297,8 +288,7 @@ void hyb_prepare(fl_matrix *A, int H, int bt, int R, hipStream_t s) {
             columns_from_tiles(A, nl, cps.p, nnz_l, nullptr, rkey.p, ents.p, s);
             radix_sort_positions(rkey.p, rkey.p, ridx.p, nnz_h, bits_for((uint32_t)(m - 1)), s);
         }
-        k_hyb_bounds<<<hg((long long)nnz_h + 1), kBlock, 0, s>>>(rkey.p, nnz_h, m, hptr.p);
-        FL_LAUNCH_CHECK();
+        key_bounds(rkey.p, nnz_h, m, hptr.p, s);
         // rows by (window, heavy count descending, row)
         TmpBuf<int> pairs(std::max(nslice, 1), s), pscan((size_t)nslice + 1, s);
         const int rounds = div_up(win, kOrderThreads);

@@ -229,18 +229,6 @@ __global__ void k_chunk_off(const int *__restrict__ band_start, int nbands, int 
     }
 }
 
-// start[b] = first position of key b in the sorted keys (lower bound); start[nb] = count.
-__global__ void k_key_bounds(const uint32_t *__restrict__ k, int count, int nb, int *__restrict__ start) {
-    GRID_STRIDE(b, (long long)nb + 1) {
-        int lo = 0, hi = count;
-        while (lo < hi) {
-            const int mid = (int)(((long long)lo + hi) >> 1);
-            if (k[mid] < (uint32_t)b) lo = mid + 1; else hi = mid;
-        }
-        start[b] = lo;
-    }
-}
-
 __global__ void k_adjdiff(const int *__restrict__ in, int count, int *__restrict__ out) {
     GRID_STRIDE(i, count) out[i] = in[i + 1] - in[i];
 }
@@ -753,7 +741,7 @@ static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInt
                                                 nnz);
     FL_LAUNCH_CHECK();
     radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)(C * nbands - 1)), s);
-    k_key_bounds<<<sg((long long)C * nbands + 1), kBlock, 0, s>>>(key.p, nnz, C * nbands, A->pb_band_start.p);
+    key_bounds(key.p, nnz, C * nbands, A->pb_band_start.p, s);
     k_chunk_off<<<1, kBlock, 0, s>>>(A->pb_band_start.p, nbands, C, d_off.p, h.out(2), h.out(2 + C));
     k_pb_heads<<<sg(nnz), kBlock, 0, s>>>(key.p, order.p, A->batch_of.p, A->sortrowidx.p, R, head.p,
                                           A->pb_rowlocal.p, nnz);
