@@ -357,6 +357,17 @@ __global__ __launch_bounds__(kBlock) void k_spmv_row1_short(int m, int chunk, co
     if (live && j == 0) Y[r] = accumulate ? (T)((ACC)Y[r] + sum) : (T)sum;
 }
 
+// A launch has fewer than 2^32 work-items, so the rows run in slices of at most 2^31 lanes each (one launch for all up to
+// 2^25 rows at 64 lanes a row). launch(rows of the slice, their pointers, their Y).
+template <typename T, typename F>
+static void row_slices(const fl_matrix *A, int lanes, int k, T *Y, F &&launch) {
+    const long long most = (1LL << 31) / lanes;
+    for (long long r = 0; r < A->m; r += most) {
+        launch((int)std::min<long long>(most, A->m - r), A->row_ptr.p + r, Y + r * k);
+        FL_LAUNCH_CHECK();
+    }
+}
+
 // Workgroups of `rows` rows each for m rows: chunks of kRowChunk rows, shorter where that would leave an
 // XCD fewer than eight of them, and a grid of whole chunks for each XCD.
 struct RowGrid {
@@ -376,26 +387,22 @@ static RowGrid row_grid(int m, int rows) {
 constexpr long long kShortRow = 6;
 template <typename T, typename ACC>
 static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    if ((long long)A->nnz <= kShortRow * A->m) {
-        const RowGrid g = row_grid(A->m, 32 * (kBlock / 64));
-        k_spmv_row1_short<T, ACC><<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y,
-                                                            accumulate);
-        FL_LAUNCH_CHECK();
-        return;
-    }
-    const RowGrid g = row_grid(A->m, 64 / kRowLanes * (kBlock / 64));
+    const bool small = (long long)A->nnz <= kShortRow * A->m;
     const bool pre = (long long)A->nnz > 4LL * kRowLanes * A->m;  // rows of more than one step on average
-    auto k = pre ? k_spmv_row1<T, ACC, true> : k_spmv_row1<T, ACC, false>;
-    k<<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y, accumulate);
-    FL_LAUNCH_CHECK();
+    const int lanes = small ? 2 : kRowLanes;
+    auto k = small ? k_spmv_row1_short<T, ACC> : pre ? k_spmv_row1<T, ACC, true> : k_spmv_row1<T, ACC, false>;
+    row_slices(A, lanes, 1, Y, [&](int m, const int *row_ptr, T *y) {
+        const RowGrid g = row_grid(m, kBlock / lanes);
+        k<<<g.grid, kBlock, 0, s>>>(m, g.chunk, row_ptr, A->row_col.p, val, X, y, accumulate);
+    });
 }
 
 template <typename T, typename ACC, int K, int VEC>
 static void launch_row_v(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    const RowGrid g = row_grid(A->m, 64 * VEC / K * (kBlock / 64));
-    k_spmm_row<T, ACC, K, VEC><<<g.grid, kBlock, 0, s>>>(A->m, g.chunk, A->row_ptr.p, A->row_col.p, val, X, Y,
-                                                         accumulate);
-    FL_LAUNCH_CHECK();
+    row_slices(A, K / VEC, K, Y, [&](int m, const int *row_ptr, T *y) {
+        const RowGrid g = row_grid(m, kBlock * VEC / K);
+        k_spmm_row<T, ACC, K, VEC><<<g.grid, kBlock, 0, s>>>(m, g.chunk, row_ptr, A->row_col.p, val, X, y, accumulate);
+    });
 }
 
 // Widest vector that keeps at least 4 lanes per row (k >= 4), is at most 16 bytes and that X
