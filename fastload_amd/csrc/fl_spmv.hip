@@ -81,13 +81,18 @@ __global__ __launch_bounds__(kBlock) void k_spmv_dropin(int T_, const int *__res
 // bound by their launches (about 4 us each in a stream of calls, against 1 to 2 us of work): sorting
 // x, clearing y and multiplying are three, this makes them two. permute_x and y = A x, 1,138 rows
 // and 4,094 entries: 12.2 -> 8.2 us in a stream of calls, 21.9 -> 19.6 each waited for.
-// One CU reads 2 to 4 entries per ns, so larger matrices keep the fill kernel and the whole chip.
-// The line lies where a call that is waited for takes as long either way (one launch / two):
-// FP64 10,000 entries 21.5 / 21.9 us, 14,000 23.0 / 21.9; FP32 12,000 21.1 / 21.9, 15,000 22.0 / 22.0.
-// In a stream of calls the one launch is ahead up to 20,000 entries (FP64 12.3 / 12.0, FP32 9.9 / 11.9).
+// One CU does it, so its time grows with the passes over the tiles (16 waves of 4 tiles of 64, or 8 of 32, to a
+// pass, each with three loads that depend on one another) and with the entries of one row inside a tile, whose adds to
+// LDS run in turn; the fill kernel and the whole chip take 6.8 to 7.4 us in a stream whatever the matrix. One launch, us:
+// FP64 2.8 + 1.5 a pass + 0.8 per 1,000 entries that repeat the row of the lane before; FP32 2.1 + 1.0 + 0.9.
+// The lines below are where a call that is waited for takes as long either way (one launch / two, with the sort of x):
+// FP64 131 tiles 19.7 / 20.4, 143 20.6 / 20.6; FP32 175 19.5 / 20.5, 200 20.7 / 20.7; dense 48 x 48 in FP64
+// 20.0 / 20.8, 64 x 64 22.3 / 20.3; without the sort, FP64, 128 tiles of one entry 17.4 / 17.6, 256 20.4 / 17.7. With
+// lines on rows and entries alone a column of 5,000 entries took 117 us in a stream of calls, two launches take 6.5.
 constexpr int kSmallBlock = 1024;
 constexpr int kSmallRows = 8192;  // 64 KB of LDS
-constexpr int kSmallEntries64 = 8192, kSmallEntries32 = 12288;
+constexpr int kSmallTiles64 = 132, kSmallTiles32 = 192;  // of 64 lanes
+constexpr int kSmallSame64 = 27, kSmallSame32 = 17;      // repeated rows that take as long as a tile
 
 template <typename T, int W, int U>
 __global__ __launch_bounds__(kSmallBlock) void k_dropin_small(int T_, int m, const int *__restrict__ tile_ptr,
@@ -370,7 +375,10 @@ static void launch_dropin_small(const fl_matrix *A, const T *x, T *y, hipStream_
 }
 
 static bool dropin_small(const fl_matrix *A, int kind) {
-    return A->m <= kSmallRows && A->nnz <= (kind == FL_VAL_F64 ? kSmallEntries64 : kSmallEntries32);
+    if (A->m > kSmallRows) return false;
+    const bool dbl = kind == FL_VAL_F64;
+    const long long tiles = (long long)A->tilenum * A->W / 64, same = A->nnz - A->segsum;
+    return tiles + same / (dbl ? kSmallSame64 : kSmallSame32) <= (dbl ? kSmallTiles64 : kSmallTiles32);
 }
 
 template <typename V, typename X, typename Y, bool SPLIT>
