@@ -37,7 +37,7 @@ __global__ void k_rows_fill(const int *__restrict__ order, const ColEntry *__res
     }
 }
 
-// The row arrays end with kRowPad entries that belong to no row: the k = 1 kernel loads entries four at a time.
+// The row arrays end with kRowPad entries that belong to no row: the row kernels load entries up to four at a time.
 constexpr int kRowPad = 4;
 
 void row_prepare(fl_matrix *A, hipStream_t s) {
@@ -144,9 +144,13 @@ __device__ __forceinline__ void static_for(F &&f) {
 //
 // Bound by the vector memory path: every distinct line an instruction touches takes a turn in
 // the L1, and a gather touches one per row. So the entries are not loaded once per row and entry
-// (which cost as many turns as the X rows themselves): each lane of a row loads one of the next
-// L * Q entries, and the lanes hand them to each other with DPP moves while the next step's are in
-// flight. X rows come in groups of U, unconditionally: past the row's end the lanes read X row 0
+// (which cost as many turns as the X rows themselves): each lane of a row loads Q consecutive ones of the
+// next L * Q entries, up to four with a load (at the alignment of an entry), and the lanes hand them to each
+// other with DPP moves while the next step's are in flight. Every L-th entry per lane instead, Q loads that touch
+// the same lines while the first is still on its way, fetches each line once per load (us; consecutive
+// entries / every L-th / all loaded by every lane of the row as they are used): k = 2 in FP32, 100 K uniform rows of 32
+// 19.0 / 28.3 / 23.2, 50^3 grid 7.1 / 11.8 / 10.7; k = 8 in FP64, 40^3 grid 9.4 / 10.9 / 9.9.
+// X rows come in groups of U, unconditionally: past the row's end the lanes read X row 0
 // (one line for all of them) and drop it, since a branch around the loads would drain them.
 // Consecutive groups run on one XCD in chunks of kRowChunk rows, dealt round-robin: rows with local
 // columns (bands, grids, block-diagonal batches) share X lines in that XCD's L2, and no XCD gets
@@ -154,8 +158,8 @@ __device__ __forceinline__ void static_for(F &&f) {
 // end unevenly (grid of 64^3, k = 16 in FP64: 58 us with one group, 78 with eight).
 // Y rows of at least a line are stored with the streaming hint: they are written whole and leave the L2
 // to X (k = 32: 287 -> 274 us).
-// Measured, before -> after (one entry load per row, four entries ahead, contiguous row ranges):
-// 128 stacked Zipf(2) matrices (5.2 M rows, 37 M entries) k = 8: 398 -> 291 us; 64 of them, k = 32:
+// Measured, before (one entry load per row, four entries ahead, contiguous row ranges) -> after, still with every
+// L-th entry per lane: 128 stacked Zipf(2) matrices (5.2 M rows, 37 M entries) k = 8: 398 -> 291 us; 64 of them, k = 32:
 // 395 -> 273 us; 64^3 27-point grid, k = 16 in FP64: 79 -> 58 us. With every gather
 // sent to 64 lines of X the k = 8 product takes 238 us, without gathers 121 us. Measured and not
 // kept: the columns that recur in a block of rows staged in LDS (k = 8: 290 us, k = 32: 332 us and
@@ -179,18 +183,26 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
     if (r >= m) return;
     const V *__restrict__ Xv = reinterpret_cast<const V *>(X);
     const int e0 = row_ptr[r];
-    const int *__restrict__ pc = row_col + e0 + j;
-    const T *__restrict__ pv = row_val + e0 + j;
+    const int *__restrict__ pc = row_col + e0 + j * Q;
+    const T *__restrict__ pv = row_val + e0 + j * Q;
     ACC acc[VEC];
 #pragma unroll
     for (int q = 0; q < VEC; ++q) acc[q] = 0;
     int c[Q], nc[Q];
     T v[Q], nv[Q];
     auto fetch = [&](int left, int *cc, T *vv) {  // the next entries of the row, `left` of them to come
+        constexpr int G = Q < 4 ? Q : 4;           // per load: at most G - 1 < kRowPad past the row's end
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            cc[q] = q * L + j < left ? pc[q * L] : 0;
-            vv[q] = q * L + j < left ? pv[q * L] : T(0);
+        for (int q = 0; q < Q; q += G) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                cc[q + g] = 0;
+                vv[q + g] = T(0);
+            }
+            if (j * Q + q < left) {
+                __builtin_memcpy(cc + q, pc + q, sizeof(int) * G);
+                __builtin_memcpy(vv + q, pv + q, sizeof(T) * G);
+            }
         }
         pc += L * Q;
         pv += L * Q;
@@ -198,6 +210,8 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
     int left = row_ptr[r + 1] - e0;
     fetch(left, c, v);
     for (; left > 0; left -= L * Q) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) c[q] = j * Q + q < left ? c[q] : 0;
         fetch(left - L * Q, nc, nv);
         static_for<0, L * Q / U>([&](auto h) {
             constexpr int H = decltype(h)::value * U;
@@ -205,11 +219,11 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
                 V x[U];
                 static_for<0, U>([&](auto u) {
                     constexpr int k = H + decltype(u)::value;
-                    x[u] = Xv[(long long)bcast_u32<L, k % L>((uint32_t)c[k / L]) * L + j];
+                    x[u] = Xv[(long long)bcast_u32<L, k / Q>((uint32_t)c[k % Q]) * L + j];
                 });
                 static_for<0, U>([&](auto u) {
                     constexpr int k = H + decltype(u)::value;
-                    const T a = bcast<L, k % L>(v[k / L]);
+                    const T a = bcast<L, k / Q>(v[k % Q]);
                     if (k < left) {
                         const T *xs = reinterpret_cast<const T *>(&x[u]);
 #pragma unroll
