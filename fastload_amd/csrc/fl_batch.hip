@@ -66,6 +66,10 @@ void row_prepare(fl_matrix *A, hipStream_t s) {
     k_rows_fill<<<sgb(nnz), kBlock, 0, s>>>(order.p, ents.p, A->row_col.p, A->row_val64.p, A->row_val32.p, nnz);
     FL_LAUNCH_CHECK();
     key_bounds(key.p, nnz, m, A->row_ptr.p, s);
+    HostInts longest(s);
+    max_step_begin(A->row_ptr.p, m, longest, s);
+    (void)longest.wait();
+    A->row_longest = max_i32_end(longest);
     A->row_ready = true;
 }
 
@@ -78,7 +82,11 @@ __global__ void k_row_val32(const double *__restrict__ v64, float *__restrict__ 
 int row_install(fl_matrix *A, const int *row_ptr, const int *row_col, const double *row_val, hipStream_t s) {
     const int m = A->m, n = A->n, nnz = A->nnz;
     bool ok = row_ptr[0] == 0 && row_ptr[m] == nnz;
-    for (int r = 0; ok && r < m; ++r) ok = row_ptr[r] <= row_ptr[r + 1];
+    int longest = 0;
+    for (int r = 0; ok && r < m; ++r) {
+        ok = row_ptr[r] <= row_ptr[r + 1];
+        longest = std::max(longest, row_ptr[r + 1] - row_ptr[r]);
+    }
     for (long long i = 0; ok && i < nnz; ++i) ok = row_col[i] >= 0 && row_col[i] < n;
     if (!ok) {
         set_error("fl_matrix_load: row order invalid (row pointers or columns out of range)");
@@ -95,6 +103,7 @@ int row_install(fl_matrix *A, const int *row_ptr, const int *row_col, const doub
         k_row_val32<<<sgb(nnz), kBlock, 0, s>>>(A->row_val64.p, A->row_val32.p, nnz);
         FL_LAUNCH_CHECK();
     }
+    A->row_longest = longest;
     A->row_ready = true;
     return FL_OK;
 }
@@ -156,6 +165,12 @@ __device__ __forceinline__ void static_for(F &&f) {
 // columns (bands, grids, block-diagonal batches) share X lines in that XCD's L2, and no XCD gets
 // all of the large blocks of a batch. One group per wave: waves that loop over several groups
 // end unevenly (grid of 64^3, k = 16 in FP64: 58 us with one group, 78 with eight).
+// HUB: for matrices whose longest row takes longer than all others (hub_rows), where one wave's chain of loads and
+// instructions is the time: 16 X rows in flight, the next step's entries loaded after them (loads come back in order,
+// so loaded before them they would delay every use of X), and no test per entry in whole steps. FP32, 400 K rows of
+// Zipf(2) length up to 50,000, k = 2, 8, 32: 1.05, 1.23, 1.90 ms, without 2.32, 4.60, 6.29, and with four entries ahead
+// loaded by every lane of the row 2.30, 3.91, 4.28. It takes 64 to 124 registers instead of 26 to 84, which costs where
+// rows are of one length: uniform rows of 32, k = 8 in FP64 28 and 40 us.
 // Y rows of at least a line are stored with the streaming hint: they are written whole and leave the L2
 // to X (k = 32: 287 -> 274 us).
 // Measured, before (one entry load per row, four entries ahead, contiguous row ranges) -> after, still with every
@@ -167,14 +182,14 @@ __device__ __forceinline__ void static_for(F &&f) {
 // rows ordered by length in windows of 256 (k = 8: 409 us: entries of a wave's rows no longer share
 // lines).
 constexpr int kRowChunk = 1024;
-template <typename T, typename ACC, int K, int VEC>
+template <typename T, typename ACC, int K, int VEC, bool HUB>
 __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int *__restrict__ row_ptr,
                                                      const int *__restrict__ row_col, const T *__restrict__ row_val,
                                                      const T *__restrict__ X, T *__restrict__ Y, int accumulate) {
     using V = typename RowVec<T, VEC>::type;
     constexpr int L = K / VEC, RPW = 64 / L;  // lanes per row, rows per wave
     constexpr int Q = L < 16 ? 16 / L : 1;    // entries per lane of a step
-    constexpr int U = L * Q < 4 ? L * Q : 4;  // X rows in flight together
+    constexpr int U = HUB ? 16 : 4;           // X rows in flight together
     constexpr bool kStreamY = K * sizeof(T) >= 128;
     const int idx = blockIdx.x >> 3;
     const long long wg = (long long)(idx / chunk * 8 + (int)(blockIdx.x & 7)) * chunk + idx % chunk;
@@ -209,22 +224,22 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
     };
     int left = row_ptr[r + 1] - e0;
     fetch(left, c, v);
-    for (; left > 0; left -= L * Q) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) c[q] = j * Q + q < left ? c[q] : 0;
-        fetch(left - L * Q, nc, nv);
+    auto step = [&](auto whole) {  // whole: the row has all L * Q entries of the step
+        constexpr bool W = decltype(whole)::value;
+        if constexpr (!HUB) fetch(left - L * Q, nc, nv);
         static_for<0, L * Q / U>([&](auto h) {
             constexpr int H = decltype(h)::value * U;
-            if (H < left) {
+            if (W || H < left) {
                 V x[U];
                 static_for<0, U>([&](auto u) {
                     constexpr int k = H + decltype(u)::value;
                     x[u] = Xv[(long long)bcast_u32<L, k / Q>((uint32_t)c[k % Q]) * L + j];
                 });
+                if constexpr (HUB && H == L * Q - U) fetch(left - L * Q, nc, nv);
                 static_for<0, U>([&](auto u) {
                     constexpr int k = H + decltype(u)::value;
                     const T a = bcast<L, k / Q>(v[k % Q]);
-                    if (k < left) {
+                    if (W || k < left) {
                         const T *xs = reinterpret_cast<const T *>(&x[u]);
 #pragma unroll
                         for (int q = 0; q < VEC; ++q) acc[q] += (ACC)a * (ACC)xs[q];
@@ -237,6 +252,15 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
             c[q] = nc[q];
             v[q] = nv[q];
         }
+        left -= L * Q;
+    };
+    if constexpr (HUB) {
+        while (left >= L * Q) step(std::true_type{});
+    }
+    while (left > 0) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) c[q] = j * Q + q < left ? c[q] : 0;
+        step(std::false_type{});
     }
     V *out = reinterpret_cast<V *>(Y) + r * L + j;
     V o;
@@ -393,6 +417,15 @@ static RowGrid row_grid(int m, int rows) {
     return {chunk, 8 * chunk * div_up(wgs, 8 * chunk)};
 }
 
+// Whether the longest row is more than 1 / part of the entries and far from the others' length: its chain, one step
+// after another, then outlasts the rest of the matrix, spread over the chip. With k >= 2 the line lies where the
+// chain of the ordinary kernel begins to show (400 K rows of 4 and one of 100 entries, a 16,000th of all, k = 8 in FP32:
+// ordinary 35.7 us, HUB 26.8, every lane of a row loading its entries 32.0; one of 400, a 4,000th: 73, 30 and 59).
+constexpr long long kHubPart = 24576;
+static bool hub_rows(const fl_matrix *A, long long part) {
+    return A->row_longest * part > A->nnz && (long long)A->row_longest * A->m > 8LL * A->nnz;
+}
+
 // Entries per row, on average, up to which rows take two lanes. Two lanes / four (every fourth entry per lane, before both), us:
 // 800 K rows in diagonal blocks, FP32, 3 entries 9.0 / 12.8 (9.8), 6 12.2 / 15.2 (17.1), 9 15.4 / 17.0 (21.5), FP64 at 9
 // 20.3 / 19.7 (34.3); 800 K rows of 3 uniform entries 16.1 / 17.8 (18.6), 6 28.7 / 26.5 (31.3), FP64 51.4 / 47.2 (58.3);
@@ -413,9 +446,10 @@ static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, in
 
 template <typename T, typename ACC, int K, int VEC>
 static void launch_row_v(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
+    auto k = hub_rows(A, kHubPart) ? k_spmm_row<T, ACC, K, VEC, true> : k_spmm_row<T, ACC, K, VEC, false>;
     row_slices(A, K / VEC, K, Y, [&](int m, const int *row_ptr, T *y) {
         const RowGrid g = row_grid(m, kBlock * VEC / K);
-        k_spmm_row<T, ACC, K, VEC><<<g.grid, kBlock, 0, s>>>(m, g.chunk, row_ptr, A->row_col.p, val, X, y, accumulate);
+        k<<<g.grid, kBlock, 0, s>>>(m, g.chunk, row_ptr, A->row_col.p, val, X, y, accumulate);
     });
 }
 

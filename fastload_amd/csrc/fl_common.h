@@ -236,6 +236,8 @@ void key_bounds(const uint32_t *keys, int count, int nb, int *start, hipStream_t
 int device_max_i32(const int *in, int count, hipStream_t s);
 // The same in two steps: the kernel, and the maximum after h.wait().
 void max_i32_begin(const int *in, int count, HostInts &h, hipStream_t s);
+// the same of in[i + 1] - in[i], i < count
+void max_step_begin(const int *in, int count, HostInts &h, hipStream_t s);
 int max_i32_end(const HostInts &h);
 int bits_for(uint32_t v);
 

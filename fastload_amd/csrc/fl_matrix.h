@@ -95,6 +95,7 @@ struct fl_matrix {
     // ROW (multi-right-hand-side): the entries re-ordered by row (CSR of A, columns in the
     // original numbering, so X needs no permutation): row_ptr [m+1], row_col/row_val [nnz].
     bool row_ready = false;
+    int row_longest = 0;  // entries of the longest row
     fl::DevBuf<int> row_ptr, row_col;
     fl::DevBuf<float> row_val32;
     fl::DevBuf<double> row_val64;

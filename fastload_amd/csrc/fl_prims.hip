@@ -180,11 +180,12 @@ HostInts::~HostInts() {
 
 // ------------------------------------------------------------------------------ max-reduce
 // One value per workgroup, at most kHostInts workgroups, and the host takes the largest.
+template <bool STEP>
 __global__ __launch_bounds__(kBlock) void k_max_i32(const int *__restrict__ in, int count, int *__restrict__ out) {
     __shared__ int part[kBlock / kWave];
     int m = 0;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x)
-        m = max(m, in[i]);
+        m = max(m, STEP ? in[i + 1] - in[i] : in[i]);
     for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -194,12 +195,17 @@ __global__ __launch_bounds__(kBlock) void k_max_i32(const int *__restrict__ in, 
     }
 }
 
-void max_i32_begin(const int *in, int count, HostInts &h, hipStream_t s) {
+template <bool STEP>
+static void max_begin(const int *in, int count, HostInts &h, hipStream_t s) {
     if (count <= 0) return;
     const unsigned g = std::min<unsigned>(grid_for(count), (unsigned)kHostInts);
-    k_max_i32<<<g, kBlock, 0, s>>>(in, count, h.out());
+    k_max_i32<STEP><<<g, kBlock, 0, s>>>(in, count, h.out());
     FL_LAUNCH_CHECK();
 }
+
+void max_i32_begin(const int *in, int count, HostInts &h, hipStream_t s) { max_begin<false>(in, count, h, s); }
+
+void max_step_begin(const int *in, int count, HostInts &h, hipStream_t s) { max_begin<true>(in, count, h, s); }
 
 int max_i32_end(const HostInts &h) {
     int m = 0;

@@ -1,9 +1,8 @@
-"""GPU test: two right-hand sides take about as long as four (100 K uniform rows of 32 entries, FP32: 19 us each); with the
-entries of a row fetched anew by every load they took 28 against 20."""
+"""GPU test: two right-hand sides take no longer than four (27-point grid of 54^3, FP32: 9.7 and 11.2 us; with the entries of
+a row fetched anew by every load 16.8 and 12.8)."""
 import time
 
 import numpy as np
-
 import pytest
 
 import fastload_amd as fl
@@ -13,12 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 def test_two_columns_are_no_slower_than_four(gpu):
-    m = n = 100_000
-    rng = np.random.default_rng(0)
-    rows, cols = np.repeat(np.arange(m), 32), rng.integers(0, n, 32 * m)
-    o = np.lexsort((rows, cols))
-    cp = np.concatenate([[0], np.cumsum(np.bincount(cols, minlength=n))]).astype(np.int32)
-    M = fl.FastLoadMatrix(m, n, cp, rows[o].astype(np.int32), np.ones(rows.size), width=64)
+    m, n, cp, ri, val = fl.gen_matrix(fl.GEN_STENCIL27, 1, 0, 0, (54,))
+    M = fl.FastLoadMatrix(m, n, cp, ri, val, width=64)
     M.prepare_rows()
     best = {2: np.inf, 4: np.inf}
     for _ in range(8):
@@ -31,4 +26,4 @@ def test_two_columns_are_no_slower_than_four(gpu):
                 M.spmm(X, Y, k, fl.VAL_F32)
             fl.synchronize()
             best[k] = min(best[k], time.perf_counter() - t)
-    assert best[2] < 1.2 * best[4]
+    assert best[2] < 1.08 * best[4]  # the middle of 0.87 and 1.31
