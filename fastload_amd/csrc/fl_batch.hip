@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
 // entries come in one 16-byte load of columns and one or two of values (at the alignment of an
 // entry), instead of four loads that each touch the lines of all 16 rows. Loads past the row's end stay
 // inside the arrays (kRowPad); those entries gather the lane's first column again and are dropped.
-// PRE: the next sixteen entries are loaded before the gathers. That pays where rows have more than
+// kRowPre: the next sixteen entries are loaded before the gathers. That pays where rows have more than
 // sixteen entries (100^3 grid: 47 against 50 us) and costs where they do not, since the
 // gathers then wait for loads of few rows (60 stacked Zipf(2) matrices: 85 against 75 us).
 // Measured, before (four entries ahead, every fourth entry per lane) -> after: 524 K rows of diagonal
@@ -287,13 +287,19 @@ __global__ __launch_bounds__(kBlock) void k_spmm_row(int m, int chunk, const int
 // uniform rows of 8: 26 -> 21; 1 M power-law rows: 117 -> 97; 60 stacked Zipf(2) matrices: 113 -> 75.
 // Two lanes per row: 32, 63, 52 us for the first three, 8 for short rows of 6 entries (10); eight: 31, 52,
 // 37 and 17 us.
+// kRowHub: for matrices whose longest row takes longer than all others (hub_rows): four steps of it at a time, 16 gathers
+// of a lane in flight and the next entries loaded after them. FP32, 400 K rows of Zipf(2.2) and Zipf(2) length up to
+// 50,000: 177 and 351 us; plain 374 and 738, four loads of every fourth entry 347 and 703, two lanes per row 634 for the
+// first. Its 100 to 144 registers (plain: 36 to 48) cost 1.4 times the time where the longest row does not decide
+// (800 K rows of 3).
 template <typename T>
 __device__ __forceinline__ void load_quad(const T *p, T *out) {
     __builtin_memcpy(out, p, 4 * sizeof(T));
 }
 
 constexpr int kRowLanes = 4;
-template <typename T, typename ACC, bool PRE>
+enum RowAhead { kRowPlain, kRowPre, kRowHub };
+template <typename T, typename ACC, RowAhead MODE>
 __global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const int *__restrict__ row_ptr,
                                                       const int *__restrict__ row_col, const T *__restrict__ row_val,
                                                       const T *__restrict__ X, T *__restrict__ Y, int accumulate) {
@@ -311,6 +317,42 @@ __global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const in
     const int *__restrict__ pc = row_col + e0 + 4 * j;
     const T *__restrict__ pv = row_val + e0 + 4 * j;
     ACC acc = 0;
+    if constexpr (MODE == kRowHub) {
+        constexpr int S = 4;  // of the row's steps at a time, while the lane's part of them is whole
+        const auto whole = [](int l) { return l >= (S - 1) * kStep + 4; };
+        const auto load = [&](int(*cc)[4], T(*vv)[4]) {
+#pragma unroll
+            for (int i = 0; i < S; ++i) {
+                load_quad(pc + i * kStep, cc[i]);
+                load_quad(pv + i * kStep, vv[i]);
+            }
+        };
+        int c[S][4], nc[S][4];
+        T v[S][4], nv[S][4], x[S][4];
+        if (whole(left)) load(c, v);
+        while (whole(left)) {
+#pragma unroll
+            for (int i = 0; i < S; ++i)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[i][u] = X[c[i][u]];
+            pc += S * kStep;
+            pv += S * kStep;
+            left -= S * kStep;
+            if (whole(left)) load(nc, nv);
+#pragma unroll
+            for (int i = 0; i < S; ++i) {
+                ACC q = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) q += (ACC)v[i][u] * (ACC)x[i][u];
+                acc += q;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    c[i][u] = nc[i][u];
+                    v[i][u] = nv[i][u];
+                }
+            }
+        }
+    }
     int c[4], nc[4];
     T v[4], nv[4];
     if (left > 0) {
@@ -320,7 +362,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const in
     while (left > 0) {
         pc += kStep;
         pv += kStep;
-        if (PRE && left > kStep) {
+        if (MODE == kRowPre && left > kStep) {
             load_quad(pc, nc);
             load_quad(pv, nv);
         }
@@ -333,7 +375,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_row1(int m, int chunk, const in
             if (u < left) q += (ACC)v[u] * (ACC)x[u];
         acc += q;
         left -= kStep;
-        if (!PRE && left > 0) {
+        if (MODE != kRowPre && left > 0) {
             load_quad(pc, nc);
             load_quad(pv, nv);
         }
@@ -431,13 +473,20 @@ static bool hub_rows(const fl_matrix *A, long long part) {
 // 20.3 / 19.7 (34.3); 800 K rows of 3 uniform entries 16.1 / 17.8 (18.6), 6 28.7 / 26.5 (31.3), FP64 51.4 / 47.2 (58.3);
 // 60 stacked Zipf(2) matrices, 7 entries, 64.6 / 61.1 (75.9). From 7 on four lanes are ahead of both
 // on all of them but the blocks in FP32.
-constexpr long long kShortRow = 6;
+// A row longer than 1 / kShortPart of the entries takes four lanes all the same: two take twice as long over it (800 K rows
+// of 3, one of 200 entries, a 12,000th, FP32 17.7 / 16.9, FP64 29.8 / 25.5; one of 100 15.4 / 16.9 and 25.5 / 25.4; 100 K
+// rows of 4, 300 of 200 10.7 / 7.0). From kHubPart1 on it is kRowHub's (four lanes / kRowHub: one of 400, a
+// 6,000th, 20.0 / 23.8; one of 1,000, a 2,400th, 29.2 / 24.0).
+constexpr long long kShortRow = 6, kShortPart = 16384, kHubPart1 = 3072;
 template <typename T, typename ACC>
 static void launch_row_k1(const fl_matrix *A, const T *val, const T *X, T *Y, int accumulate, hipStream_t s) {
-    const bool small = (long long)A->nnz <= kShortRow * A->m;
+    const bool small = (long long)A->nnz <= kShortRow * A->m && !hub_rows(A, kShortPart);
     const bool pre = (long long)A->nnz > 4LL * kRowLanes * A->m;  // rows of more than one step on average
     const int lanes = small ? 2 : kRowLanes;
-    auto k = small ? k_spmv_row1_short<T, ACC> : pre ? k_spmv_row1<T, ACC, true> : k_spmv_row1<T, ACC, false>;
+    auto k = small                     ? k_spmv_row1_short<T, ACC>
+             : hub_rows(A, kHubPart1) ? k_spmv_row1<T, ACC, kRowHub>
+             : pre                     ? k_spmv_row1<T, ACC, kRowPre>
+                                       : k_spmv_row1<T, ACC, kRowPlain>;
     row_slices(A, lanes, 1, Y, [&](int m, const int *row_ptr, T *y) {
         const RowGrid g = row_grid(m, kBlock / lanes);
         k<<<g.grid, kBlock, 0, s>>>(m, g.chunk, row_ptr, A->row_col.p, val, X, y, accumulate);

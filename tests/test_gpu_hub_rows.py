@@ -73,9 +73,10 @@ def test_long_row_among_short_ones(pair, k, kind):
     assert np.array_equal(b[~uses], _product(alone, X[:N], Y[:m], k, kind, False)[~uses]) and not np.isfinite(b[uses]).any()
 
 
-@pytest.mark.parametrize("k,most", [(2, 1.4), (8, 2.0), (32, 2.6)])
+@pytest.mark.parametrize("k,most", [(1, 0.4), (2, 1.4), (8, 2.0), (32, 2.6)])
 def test_time_of_one_long_row(gpu, k, most):
-    """50,000 entries in one row, FP32, ms: 0.7, 0.8, 1.2 for k = 2, 8, 32; with four X rows in flight 1.6, 3.4, 4.1."""
+    """50,000 entries in one row, FP32, ms: 0.2, 0.7, 0.8, 1.2 for k = 1, 2, 8, 32; with two lanes for k = 1 and four X rows
+    in flight 0.63, 1.6, 3.4, 4.1."""
     m, n = 20_000, 100_000
     rng = np.random.default_rng(2)
     rows = np.r_[np.repeat(np.arange(m), 3), np.full(50_000, 777)]
