@@ -46,6 +46,7 @@ SIGNATURES = {
     "fl_device_count": (C.c_int, [i32p]),
     "fl_malloc": (C.c_int, [C.POINTER(vp), C.c_size_t]),
     "fl_free_device": (C.c_int, [vp]),
+    "fl_release_memory": (C.c_int, [C.POINTER(C.c_size_t)]),
     "fl_memcpy_h2d": (C.c_int, [vp, vp, C.c_size_t]),
     "fl_memcpy_d2h": (C.c_int, [vp, vp, C.c_size_t]),
     "fl_memcpy_d2d": (C.c_int, [vp, vp, C.c_size_t]),

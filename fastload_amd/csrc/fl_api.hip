@@ -360,6 +360,14 @@ int fl_malloc(void **dptr, size_t bytes) {
     FL_API_END
 }
 
+int fl_release_memory(size_t *bytes) {
+    FL_API_BEGIN
+    const size_t freed = dev_blocks_release();
+    if (bytes) *bytes = freed;
+    return FL_OK;
+    FL_API_END
+}
+
 int fl_free_device(void *dptr) {
     FL_API_BEGIN
     if (dptr) FL_HIP(hipFree(dptr));

@@ -118,7 +118,7 @@ struct DevBlock {
 };
 DevBlock dev_block_get(size_t bytes);  // throws HipError
 void dev_block_put(const DevBlock &b);
-void dev_blocks_release();  // frees every kept block
+size_t dev_blocks_release();  // frees every kept block, returns their bytes
 
 // RAII device buffer (a device block, put back on scope exit).
 template <typename T>

@@ -577,16 +577,19 @@ void settle_pending(bool keep) {
 }
 }  // namespace
 
-void dev_blocks_release() {
+size_t dev_blocks_release() {
     BlockStore &b = block_store();
     std::vector<void *> out;
+    size_t bytes = 0;
     {
         std::lock_guard<std::mutex> g(b.mu);
         for (auto &k : b.blocks) out.push_back(k.second.p);
+        bytes = (size_t)b.held;
         b.blocks.clear();
         b.held = 0;
     }
     for (void *p : out) (void)hipFree(p);
+    return bytes;
 }
 
 DevBlock dev_block_get(size_t bytes) {

@@ -84,6 +84,13 @@ def synchronize():
     check(lib.fl_synchronize(), "fl_synchronize")
 
 
+def release_memory() -> int:
+    """Frees the device memory that the library keeps for later objects; returns its bytes."""
+    n = C.c_size_t()
+    check(lib.fl_release_memory(C.byref(n)), "fl_release_memory")
+    return n.value
+
+
 class Stream:
     def __init__(self):
         p = C.c_void_p()

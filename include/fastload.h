@@ -150,6 +150,10 @@ int fl_slide_load(const char *path, slide_matrix *matrix, int *rowA, int *colA, 
 int fl_device_count(int *count);
 int fl_malloc(void **dptr, size_t bytes);
 int fl_free_device(void *dptr);
+/* Gives the device memory that the library keeps for later objects (of destroyed matrices, solvers and
+ * networks, and of finished preparations; at most 8 GiB per process) back to the system, for other allocators.
+ * Objects in use keep theirs. *bytes (may be NULL) receives how much it was. */
+int fl_release_memory(size_t *bytes);
 int fl_memcpy_h2d(void *dst, const void *src, size_t bytes);
 int fl_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int fl_memcpy_d2d(void *dst, const void *src, size_t bytes);
