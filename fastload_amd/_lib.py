@@ -72,6 +72,7 @@ SIGNATURES = {
     "fl_set_stream_policy": (C.c_int, [C.c_int]),
     "fl_spmv_assign_noalloc": (C.c_int, [vp, C.c_int, C.c_int, vp, vp, vp]),
     "fl_matrix_prepare_schedule": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, vp]),
+    "fl_band_rows": (C.c_int, [C.c_int, C.c_int, C.c_int]),
     "fl_matrix_prepare_hyb": (C.c_int, [vp, C.c_int, C.c_int, C.c_int, vp]),
     "fl_matrix_hyb_info": (C.c_int, [vp, i32p, C.POINTER(C.c_longlong)]),
     "fl_matrix_prepare_rows": (C.c_int, [vp, vp]),

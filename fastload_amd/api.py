@@ -303,12 +303,13 @@ class FastLoadMatrix:
         return m.value, e.value, i.value
 
     def prepare_schedule(self, kernel: int, batch_tiles: int = 256, band_rows: int = 16384, stream=None):
+        """A batched schedule. PB's bands have at most `band_rows` rows (band_rows() says how many)."""
         check(lib.fl_matrix_prepare_schedule(self.handle, kernel, batch_tiles, band_rows,
                                              stream.ptr if stream is not None else None), "fl_matrix_prepare_schedule")
 
     def prepare_hyb(self, heavy_cols: int | None = None, batch_tiles: int = 128, band_rows: int = 16384, stream=None):
         """The HYB schedule: the last `heavy_cols` sorted columns (default min(n, 32768)) from LDS,
-        the others through a PB sub-matrix of (batch_tiles, band_rows)."""
+        the others through a PB sub-matrix of (batch_tiles, at most band_rows)."""
         h = min(self.n, 32768) if heavy_cols is None else heavy_cols
         check(lib.fl_matrix_prepare_hyb(self.handle, h, batch_tiles, band_rows,
                                         stream.ptr if stream is not None else None), "fl_matrix_prepare_hyb")
@@ -364,6 +365,14 @@ class FastLoadMatrix:
             self.close()
         except Exception:
             pass
+
+
+def band_rows(m: int, batch_tiles: int = 256, most: int = 16384) -> int:
+    """Rows of a band of the PB schedule of a matrix with m rows, prepared with band_rows=most (fl_band_rows)."""
+    r = lib.fl_band_rows(m, batch_tiles, most)
+    if r < 0:
+        check(r, "fl_band_rows")
+    return r
 
 
 # -------------------------------------------------------------------- iterative solver

@@ -679,6 +679,12 @@ int fl_matrix_prepare_schedule(fl_matrix *A, int kernel, int batch_tiles, int ba
     FL_API_END
 }
 
+int fl_band_rows(int m, int batch_tiles, int band_rows) {
+    if (m < 0 || (batch_tiles != 64 && batch_tiles != 128 && batch_tiles != 256) || band_rows < 1024 || band_rows > 16384)
+        return invalid("fl_band_rows: m >= 0, batch_tiles of 64, 128 or 256 and band_rows in [1024, 16384] required");
+    return pb_band_rows(m, batch_tiles, band_rows);
+}
+
 int fl_spmv(fl_matrix *A, int kernel, int val_kind, const void *d_sortx, void *d_y, void *d_work, void *stream) {
     FL_API_BEGIN
     if (!A || (A->tilenum && (!d_sortx || !d_y))) return invalid("fl_spmv: NULL");

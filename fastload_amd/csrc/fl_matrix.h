@@ -230,6 +230,9 @@ inline bool stream_reads(long long bytes) {
     return p == FL_STREAM_AUTO ? bytes > kInfinityCacheBytes : p == FL_STREAM_ALWAYS;
 }
 
+// Rows of a PB band of a matrix of m rows, at most R.
+int pb_band_rows(int m, int bt, int R);
+
 // HYB schedule (fl_hyb.hip). Heavy x is staged in LDS: at most kHybMaxH32 FP32 or kHybMaxH64
 // FP64 columns.
 constexpr int kHybMaxH32 = 38912, kHybMaxH64 = 19456;

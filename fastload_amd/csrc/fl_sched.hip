@@ -685,7 +685,7 @@ static std::vector<int> pb_chunk_batches(const fl_matrix *A, int C, hipStream_t 
 // -> these): 1.5 M rows, Poisson(12) columns, FP32: 93 -> 77 us (92 bands -> 245; 82 us at 4,096 rows,
 // 88 at 2,048); 400 K rows: 39.5 -> 19.0 (25 -> 196 bands); 3 M rows in FP64: 174 -> 172. From 4.2 M
 // rows on the bands are as tall as asked for (4.2 M power-law rows: 154 us at 16K, 171 at 8K).
-static int pb_band_rows(int m, int bt, int R) {
+int pb_band_rows(int m, int bt, int R) {
     const int per = div_up(m, std::min(256, 2 * bt));
     return std::min(R, std::max(1024, (per + 1023) / 1024 * 1024));
 }

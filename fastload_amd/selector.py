@@ -14,7 +14,7 @@ Schedule space (tile width x reduction strategy x batch/band parameters):
   2 winr64       WIN on 64-tile batches of tiles grouped by row window (owned rows, no atomic)
   3-5 win{64,128,256}  batches of 64/128/256 tiles, rows compacted to LDS slots, one flush per
                  row of a batch (a store for rows no other batch touches, else one atomic)
-  6-10 pb*       propagation blocking, batch 128/256 tiles x band 4K/8K/16K rows, no atomics
+  6-10 pb*       propagation blocking, batch 128/256 tiles x bands of up to 4K/8K/16K rows, no atomics
   11 row         entries re-ordered by row (CSR), four lanes per row, no atomics (fl_spmm, k=1)
   12 hyb32k_pb128_r16k  the min(n, 32768) longest columns row by row with their x in LDS, the
                  rest PB 128 tiles x 16K rows on a sub-matrix
@@ -42,7 +42,7 @@ from ._lib import FastLoadError, check, lib
 from .api import (GEN_BANDED, GEN_BLOCKDIAG, GEN_STENCIL27, GEN_UNIFORM, GEN_ZIPF, GEN_ZIPF_DENSE, KERNEL_DROPIN,
                   KERNEL_FAST,
                   KERNEL_HYB,
-                  KERNEL_PB, KERNEL_WIN, KERNEL_WINR, VAL_F32, FastLoadMatrix, gen_matrix)
+                  KERNEL_PB, KERNEL_WIN, KERNEL_WINR, VAL_F32, FastLoadMatrix, band_rows, gen_matrix)
 from .device import DeviceArray, Event, synchronize
 
 N_FEATURES = 40
@@ -94,6 +94,14 @@ HYB_CLASS = next(c for c, sc in enumerate(SCHEDULES) if sc.kernel == KERNEL_HYB)
 # choose_refined also times the HYB class when the HYB_COLS longest columns hold at least
 # HYB_MIN_SHARE of the entries, whatever probability the network gives it
 HYB_MIN_SHARE = 0.35
+
+
+def effective(cls: int, m: int):
+    """What class `cls` runs on a matrix of m rows: classes of the same value are the same schedule there (PB's band
+    heights are upper limits: up to 1,048,576 rows its five classes are two)."""
+    s = SCHEDULES[cls]
+    band = band_rows(m, s.batch_tiles, s.band_rows) if s.kernel in (KERNEL_PB, KERNEL_HYB) else 0
+    return s.width, s.kernel, s.batch_tiles, band
 
 
 def heavy_share(n, dcolptr, cols: int = HYB_COLS) -> float:
@@ -345,8 +353,9 @@ class Selector:
         this matrix (`reps` steps each, after warm-up steps); the fastest is returned with the
         measured times. Candidates: the `top` best-ranked, or by default (top=None) those of
         tuning_candidates (probability >= TUNE_MIN_PROB, at most TUNE_MAX), plus the HYB class
-        when the HYB_COLS longest columns hold at least HYB_MIN_SHARE of the entries. One-time
-        cost: preparing and timing the candidates."""
+        when the HYB_COLS longest columns hold at least HYB_MIN_SHARE of the entries. Candidates that
+        are the same schedule on this matrix are timed once. One-time cost: preparing and timing the
+        candidates."""
         f = features(m, n, dcolptr, drowidx)
         if top is None:
             p = self.probs_features(f)
@@ -357,13 +366,16 @@ class Selector:
             cands = cands + [HYB_CLASS]
         if len(cands) == 1:
             return cands[0], {cands[0]: None}, f
-        mats, times = {}, {}
+        mats, times, timed = {}, {}, {}
         dx = DeviceArray.from_host(np.ones(n, np.float32))
         dy = DeviceArray(max(m, 1), np.float32)
         for c in cands:
-            run = ScheduledSpMV(m, n, dcolptr, drowidx, dval, c, mats)
-            run.set_x(dx)
-            times[c] = time_schedule(run.step, dy, reps_min=reps, reps_max=reps, rounds=1)
+            key = effective(c, m)
+            if key not in timed:
+                run = ScheduledSpMV(m, n, dcolptr, drowidx, dval, c, mats)
+                run.set_x(dx)
+                timed[key] = time_schedule(run.step, dy, reps_min=reps, reps_max=reps, rounds=1)
+            times[c] = timed[key]
         for M in mats.values():
             M.close()
         best = min(times, key=times.get)

@@ -308,10 +308,15 @@ int fl_spmv_assign_noalloc(fl_matrix *A, int kernel, int val_kind, const void *d
 
 /* Builds (once per parameter set) the preprocessing of a batched schedule on a 64-wide matrix:
  *   kernel FL_KERNEL_WIN / FL_KERNEL_WINR: batch_tiles in {64, 128, 256} (LDS <= batch_tiles*512 bytes);
- *   kernel FL_KERNEL_PB : batch_tiles as above, band_rows in [1024, 16384] (LDS = band_rows*8 bytes).
+ *   kernel FL_KERNEL_PB : batch_tiles as above, band_rows in [1024, 16384]: the most rows of a band (LDS
+ *     of 8 bytes each). The bands are as low as gives every compute unit one, so below 2 to 4 million rows they
+ *     have fewer rows than asked for, and different band_rows can mean the same schedule: fl_band_rows.
  * The PB schedule keeps a product buffer of nnz floats (doubles in FP64 mode) allocated on its
  * first use. */
 int fl_matrix_prepare_schedule(fl_matrix *A, int kernel, int batch_tiles, int band_rows, void *stream);
+/* The rows of a band that the PB schedule (and HYB's sub-matrix) of a matrix with m rows has when it is
+ * prepared with these parameters; FL_ERR_INVALID for parameters that are refused there. */
+int fl_band_rows(int m, int batch_tiles, int band_rows);
 /* Builds the FL_KERNEL_HYB schedule (no reference counterpart): the last heavy_cols sorted columns
  * in [0, min(n, 38912)] become the heavy part, the others a sub-matrix with the PB schedule of
  * batch_tiles and band_rows (as above). fl_matrix_prepare_schedule(A, FL_KERNEL_HYB, ...) uses
