@@ -94,10 +94,6 @@ __global__ void k_key_gather(const int *__restrict__ src, const int *__restrict_
     GRID_STRIDE(i, count) key[i] = (uint32_t)src[order[i]];
 }
 
-__global__ void k_key_copy(const int *__restrict__ src, uint32_t *__restrict__ key, int count, int div) {
-    GRID_STRIDE(i, count) key[i] = (uint32_t)(src[i] / div);
-}
-
 // Batch b runs on XCD b % 8 (workgroups are dealt to the 8 XCDs round-robin). Ordering a band's
 // runs by (b % 8, b / 8) puts the runs one XCD writes next to each other, so a cache line
 // shared by two neighbouring runs is usually completed in one L2 instead of two.
@@ -599,9 +595,7 @@ static void win_rows_sorted(fl_matrix *A, HostInts &h, hipStream_t s) {
     TmpBuf<uint32_t> key(nnz, s);
     TmpBuf<int> order(nnz, s), head(nnz, s), d((size_t)nnz + 1, s);
     // (row, g) order, then stable by batch -> (batch, row, g)
-    k_key_copy<<<sg(nnz), kBlock, 0, s>>>(A->sortrowidx.p, key.p, nnz, 1);
-    FL_LAUNCH_CHECK();
-    radix_sort_positions(key.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
+    radix_sort_positions((const uint32_t *)A->sortrowidx.p, key.p, order.p, nnz, bits_for((uint32_t)std::max(A->m - 1, 0)), s);
     k_key_gather<<<sg(nnz), kBlock, 0, s>>>(A->batch_of.p, order.p, key.p, nnz);
     FL_LAUNCH_CHECK();
     radix_sort_pairs(key.p, order.p, nnz, bits_for((uint32_t)std::max(nb - 1, 0)), s);
@@ -726,7 +720,7 @@ static void pb_place_table(fl_matrix *A, int R, const int *d_cb, int C, HostInts
     FL_LAUNCH_CHECK();
 }
 
-// The same by sorting the entries, for more bands than a workgroup counts in LDS.
+// The same by sorting the entries, for more bands than a workgroup counts in LDS and for tables much larger than the entries.
 static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInts &h, hipStream_t s) {
     const int nnz = A->nnz, nb = A->nbatches, nbands = A->nbands;
     TmpBuf<int> d_off(C, s);
@@ -748,10 +742,8 @@ static void pb_place_sorted(fl_matrix *A, int R, const int *d_cb, int C, HostInt
     FL_LAUNCH_CHECK();
     exclusive_scan_i32(head.p, runidx.p, nnz, s, h.out(0));
     const int nruns = h.wait()[0];
-    // The runs by (batch, band), and with their lengths the entries' staging slots. There are 20 to 60 times
-    // fewer runs than entries, and inside a run both orders are the same, so only the runs are sorted again.
-    // (Sorting the entries again was up to four passes over all of them and three gathers: the preparation of
-    // 18 M uniform entries 1,556 us, so 1,121; 9.6 M power-law entries 909 and 709; 1.8 M 289 and 289.)
+    // The runs by (batch, band), and with their lengths the entries' staging slots: inside a run both orders are the
+    // same, so only the runs are sorted again.
     pb_alloc_runs(A, nruns);
     TmpBuf<int> run_pos(nruns, s), by(nruns, s), start((size_t)nruns + 1, s), lstart_of(nruns, s);
     TmpBuf<uint32_t> run_key(nruns, s);
