@@ -1,5 +1,5 @@
-"""GPU test of the row kernels on matrices with a row much longer than the others: every k, both value kinds, rows that
-end at the edges of steps and groups next to one of 1,000 entries. The kernel is chosen by the whole matrix, so the same
+"""GPU test of the row kernels on matrices with a row much longer than the others: every k, both value kinds, X and Y at
+addresses for 16-byte lanes and narrower ones, rows that end at the edges of steps and groups next to one of 1,000 entries. The kernel is chosen by the whole matrix, so the same
 rows above rows of 600 entries, where the long one is none, have to give the same bits."""
 import time
 
@@ -25,10 +25,14 @@ def _matrix(m, n, rows, cols, vals):
     return M
 
 
-def _product(M, X, Y, k, kind, accumulate):
+def _product(M, X, Y, k, kind, accumulate, shift):
     dt = np.float64 if kind == fl.VAL_F64 else np.float32
-    dy = DeviceArray.from_host(Y.astype(dt).ravel())
-    M.spmm(DeviceArray.from_host(X.astype(dt).ravel()), dy, k, kind, accumulate=accumulate)
+
+    def put(a):  # `shift` elements from the start of an allocation
+        return DeviceArray.from_host(np.r_[np.zeros(shift, dt), a.astype(dt).ravel()]).view(shift, a.size)
+
+    dx, dy = put(X), put(Y)
+    M.spmm(dx, dy, k, kind, accumulate=accumulate)
     return dy.to_host().reshape(-1, k)
 
 
@@ -51,7 +55,8 @@ def pair(gpu):
 
 @pytest.mark.parametrize("kind", [fl.VAL_F64, fl.VAL_F32], ids=["f64", "f32"])
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 32, 64])
-def test_long_row_among_short_ones(pair, k, kind):
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_long_row_among_short_ones(pair, k, kind, shift):
     m, rows, cols, vals, alone, both = pair
     rng = np.random.default_rng(k)
     X = rng.standard_normal((2 * N, k)).astype(np.float32).astype(np.float64)
@@ -60,17 +65,17 @@ def test_long_row_among_short_ones(pair, k, kind):
     np.add.at(want, rows, vals[:, None] * X[cols])
     np.add.at(scale, rows, np.abs(vals[:, None] * X[cols]))
     for accumulate in (False, True):
-        a = _product(alone, X[:N], Y[:m], k, kind, accumulate)
+        a = _product(alone, X[:N], Y[:m], k, kind, accumulate, shift)
         more = Y[:m] if accumulate else 0.0
         assert np.all(np.abs(a - (want + more)) <= TOL[kind] * (scale + np.abs(more)))
-        assert np.array_equal(a, _product(both, X, Y, k, kind, accumulate)[:m])
+        assert np.array_equal(a, _product(both, X, Y, k, kind, accumulate, shift)[:m])
     # an X row of infinities reaches only the rows that use it
     Z = X.copy()
     Z[0] = np.inf
     uses = np.zeros(m, bool)
     uses[rows[cols == 0]] = True
-    b = _product(alone, Z[:N], Y[:m], k, kind, False)
-    assert np.array_equal(b[~uses], _product(alone, X[:N], Y[:m], k, kind, False)[~uses]) and not np.isfinite(b[uses]).any()
+    b = _product(alone, Z[:N], Y[:m], k, kind, False, shift)
+    assert np.array_equal(b[~uses], _product(alone, X[:N], Y[:m], k, kind, False, shift)[~uses]) and not np.isfinite(b[uses]).any()
 
 
 @pytest.mark.parametrize("k,most", [(1, 0.4), (2, 1.4), (8, 2.0), (32, 2.6)])
@@ -91,3 +96,14 @@ def test_time_of_one_long_row(gpu, k, most):
         fl.synchronize()
         best = min(best, (time.perf_counter() - t) / 10)
     assert best * 1e3 < most
+
+
+def test_long_row_from_a_file(pair, tmp_path):
+    """The row order read back: the same kernel, the same bits."""
+    m, rows, cols, vals, alone, _ = pair
+    alone.save(tmp_path / "hub.flmx")
+    loaded = fl.FastLoadMatrix.load(tmp_path / "hub.flmx")
+    for k in (1, 2, 8):
+        X, Y = np.random.default_rng(k).standard_normal((N, k)), np.zeros((m, k))
+        args = X, Y, k, fl.VAL_F64, False, 0
+        assert np.array_equal(_product(alone, *args), _product(loaded, *args))
