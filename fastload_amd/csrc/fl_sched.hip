@@ -674,7 +674,8 @@ static std::vector<int> pb_chunk_batches(const fl_matrix *A, int C, hipStream_t 
 }
 
 // Rows of a band: at most R, and few enough that phase 2, one workgroup per band, has one band for
-// each of the 256 compute units; but a batch (bt * 64 entries) then writes bt * 64 / bands products
+// each of the 256 compute units of a whole card (a constant, so that a layout does not depend on the device it is made
+// on); but a batch (bt * 64 entries) then writes bt * 64 / bands products
 // at a time, so there are no more bands than leave it 32. Measured (a product, 16K-row bands
 // -> these): 1.5 M rows, Poisson(12) columns, FP32: 93 -> 77 us (92 bands -> 245; 82 us at 4,096 rows,
 // 88 at 2,048); 400 K rows: 39.5 -> 19.0 (25 -> 196 bands); 3 M rows in FP64: 174 -> 172. From 4.2 M
