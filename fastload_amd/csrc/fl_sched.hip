@@ -1463,14 +1463,18 @@ static OrdTiles ord_tiles(const fl_matrix *A) {
 }
 
 template <typename V, typename X, typename Y, int MODE, int NT, bool ASSIGN, bool DOT>
-static auto win_kernel(int bt) {
-    // Tiles per group. FP64, 4 -> 8 (16): 80^3 27-point grid 33.8 -> 33.2 us (36.4), 127^3 150.2 -> 148.3 (160.0), a CG
-    // solve on 80^3 7,630 -> 7,510 (8,550); FP32 on 60^3 13.8 with 8, 14.7 with 16. In FP64 batches of 128 tiles keep 4,
-    // as 8 leave fewer of their 512-thread workgroups on a compute unit (WIN on 80^3: 64 tiles 33.3 with 4 and 8,
-    // 128 30.5 and 33.3, 256, where LDS decides that, 34.6 and 34.2).
-    constexpr int U = 8, U128 = sizeof(X) == 4 ? 8 : 4;
-    return (bt == 256) ? k_win<V, X, Y, MODE, U, 256, NT, ASSIGN, DOT>
-           : (bt == 128) ? k_win<V, X, Y, MODE, U128, 128, NT, ASSIGN, DOT> : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN, DOT>;
+static auto win_kernel(const fl_matrix *A) {
+    // Tiles per group: 8 where x has 4 bytes (60^3 grid 13.8 us, 14.7 with 16). In FP64 4, and 8 for batches of 64 tiles of
+    // one row window (WINR). FP64, 4 / 8 tiles, us: WINR with 64 tiles 90^3 40.5 / 39.6, 127^3 149.8 / 145.9 (16: 160), a CG
+    // solve on 80^3 7,629 / 7,523 (8,550); but the batches grouped by column 128^3 138 / 144 with 64 tiles and 129.5 / 137.5 with 256,
+    // 90^3 with 256 40.0 / 42.3; WINR with 256 tiles 128^3 135.7 / 137.2; WIN with 128 tiles 80^3 30.5 / 33.3, as 8 leave
+    // fewer of their 512-thread workgroups on a compute unit.
+    constexpr int U = sizeof(X) == 4 ? 8 : 4;
+    if constexpr (U != 8)
+        if (A->bt == 64 && A->ord_kind == 1) return k_win<V, X, Y, MODE, 8, 64, NT, ASSIGN, DOT>;
+    return A->bt == 256   ? k_win<V, X, Y, MODE, U, 256, NT, ASSIGN, DOT>
+           : A->bt == 128 ? k_win<V, X, Y, MODE, U, 128, NT, ASSIGN, DOT>
+                          : k_win<V, X, Y, MODE, U, 64, NT, ASSIGN, DOT>;
 }
 
 template <typename V, typename X, typename Y, int MODE>
@@ -1484,14 +1488,14 @@ static void launch_win(const fl_matrix *A, const V *val, const X *x, Y *y, bool 
     // + 64 spare slots, one per lane, for the lanes past a tile's end
     const size_t lds = ((size_t)std::max(A->win_maxslots, 1) + 64) * sizeof(double);
     const int nt = std::min(A->bt * 4, 512);
-    auto kern = (nt == 256) ? (assign ? win_kernel<V, X, Y, MODE, 256, true, false>(A->bt)
-                                      : win_kernel<V, X, Y, MODE, 256, false, false>(A->bt))
-                            : (assign ? win_kernel<V, X, Y, MODE, 512, true, false>(A->bt)
-                                      : win_kernel<V, X, Y, MODE, 512, false, false>(A->bt));
+    auto kern = (nt == 256) ? (assign ? win_kernel<V, X, Y, MODE, 256, true, false>(A)
+                                      : win_kernel<V, X, Y, MODE, 256, false, false>(A))
+                            : (assign ? win_kernel<V, X, Y, MODE, 512, true, false>(A)
+                                      : win_kernel<V, X, Y, MODE, 512, false, false>(A));
     if constexpr (mode_kind(MODE) == kPlain && std::is_same<X, V>::value) {  // FL_VAL_F64, FL_VAL_F32
         if (dot)
-            kern = (nt == 256) ? win_kernel<V, X, Y, MODE, 256, true, true>(A->bt)
-                               : win_kernel<V, X, Y, MODE, 512, true, true>(A->bt);
+            kern = (nt == 256) ? win_kernel<V, X, Y, MODE, 256, true, true>(A)
+                               : win_kernel<V, X, Y, MODE, 512, true, true>(A);
     }
     allow_lds(kern, lds);
     kern<<<A->nbatches, nt, lds, s>>>(ord_tiles(A), A->bt, slot, val, pf, std::max(A->win_maxslots, 1), x,
